@@ -220,3 +220,35 @@ def test_kv_decode_random_shapes(case):
     ref = orc.kv_decode_attention(q, kc, vc, ks, vs, table, np.asarray(lens, np.int32), bits, sm)
     nrel, mrel = _errs(y, ref)
     assert nrel <= 2e-3 and mrel <= 2e-3, (case, nrel, mrel)
+
+
+# Batches where the split by lengths takes its different ways: one long sequence among short and empty ones (many
+# chunks beside whole sequences), more live sequences than workgroups aimed at (`crowded`), evenly spread lengths whose
+# equal share gives too many chunks, a table wider than every sequence, exactly 64 sequences and 65 (the fixed plan),
+# 16-head groups (4 waves), and chunk sizes at the multiples of the wave count.
+RAGGED = [([5000] + [0, 3, 40, 17] * 3, 10, 2, 512),
+          ([9000] + list(range(1, 64)), 8, 8, 600),
+          ([256 * (i + 1) for i in range(16)], 40, 8, 512),
+          ([64 * (i + 1) for i in range(64)], 8, 2, 300),
+          ([900 - 13 * i for i in range(65)], 4, 1, 64),
+          ([3000, 1, 0, 2047, 2048, 2049], 32, 2, 400),
+          ([1024, 1025, 1040, 128, 129], 5, 1, 66),
+          ([0, 0, 0], 8, 8, 100)]
+
+
+@pytest.mark.parametrize("bits", [8, 4])
+@pytest.mark.parametrize("lens,Hq,Hkv,max_pages", RAGGED, ids=[f"B{len(c[0])}-q{c[1]}-kv{c[2]}" for c in RAGGED])
+def test_kv_decode_split_by_lengths(lens, Hq, Hkv, max_pages, bits):
+    """Ragged batches against the float64 closed form (the bar of this file: 2e-3), with empty sequences zero and
+    repeated calls bit-identical."""
+    q, kc, vc, ks, vs, table = _case(len(lens) + Hq + bits, lens, Hq, Hkv, bits, max_pages=max_pages)
+    sm = D ** -0.5
+    first = _run(q, kc, vc, ks, vs, table, lens, bits, sm)
+    y = first.cpu().numpy()
+    live = [b for b, L in enumerate(lens) if L > 0]
+    assert all((y[b] == 0).all() for b, L in enumerate(lens) if L == 0)
+    if live:
+        ref = orc.kv_decode_attention(q[live], kc, vc, ks, vs, table[live], np.asarray(lens, np.int32)[live], bits, sm)
+        nrel, mrel = _errs(y[live], ref)
+        assert nrel <= 2e-3 and mrel <= 2e-3, (nrel, mrel)
+    assert torch.equal(_run(q, kc, vc, ks, vs, table, lens, bits, sm), first)

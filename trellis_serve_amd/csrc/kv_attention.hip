@@ -8,7 +8,7 @@
 //   page_table int32 [B][max_pages]; seq_lens int32 [B]; q fp16 [B][Hq][D]; out fp16 [B][Hq][D]; D = 128.
 //   Query head h reads KV head h / (Hq / Hkv).
 //
-// kv_decode_kernel: grid (chunks of chunk_pages pages, Hkv, B), W = 8 (or 4) waves.  Wave w takes pages w, w+W, ...
+// kv_decode_kernel: grid (Hkv, chunks of pages over the batch), W = 8 (or 4) waves.  Wave w takes pages w, w+W, ...
 // of its workgroup's chunk, with the next page's codes in flight while it works on the current one, and keeps an
 // online softmax for the G = Hq/Hkv query heads (G <= 16; MFMA columns G..15 are idle).  Per 16-token page --
 // exactly one 16-wide MFMA block, so the page's two scales are wave-uniform:
@@ -210,18 +210,132 @@ struct KvState {
   }
 };
 
+// ---- split of a batch over the workgroups ----------------------------------------------------------------------------
+// The host knows the page table's width but not the lengths.  Chunks of a fixed share of the table leave most
+// workgroups idle on a ragged batch (or a table wider than its sequences): the longest sequence's chunks set the time.
+// So for up to 64 sequences every wave reads all lengths (one per lane) and derives the same plan: chunks of up to
+// `cp` pages, cp the batch's pages over the number of workgroups aimed at, so that a long sequence takes many chunks
+// and a short one a single chunk, which writes its output directly.  Measured against the fixed plan (a step of two
+// calls, 40 / 8 heads): 16 sequences of 256 .. 4096 tokens in an 8k table, 8 bits 71.4 -> 49.1 us; 7 sequences of
+// 4681 .. 32768 tokens, 4 bits 117-129 -> 76.6 us.  Deriving the plan costs 0.7-1.3 us per call (decode and merge), seen
+// where every sequence fills the table: 16 x 4k 8 bits 26.0 -> 27.3 us, one sequence of 32k 17.9 -> 18.9.
+struct KvSplit {
+  int by_length;            // 1: the split by the lengths, aiming at `target` chunks per kv head and with room for
+  int batch, max_tokens;    // `slots` partial states per (kv head, query head)
+  int target, slots;
+  float inv_target, inv_slots;
+  int chunk_pages, chunks;  // the fixed plan: `chunks` chunks of chunk_pages pages per sequence
+};
+
+__device__ __forceinline__ int wave_scan(int v) {  // inclusive prefix sum over the 64 lanes
+  v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xF, 0xF, true);   // row_shr:1, 2, 4, 8: inside each row of 16
+  v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xF, 0xF, true);
+  v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xF, 0xF, true);
+  v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xF, 0xF, true);
+  v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xA, 0xF, false);  // row_bcast:15 into rows 1 and 3
+  v += __builtin_amdgcn_update_dpp(0, v, 0x143, 0xC, 0xF, false);  // row_bcast:31 into rows 2 and 3
+  return v;
+}
+__device__ __forceinline__ int wave_total(int v) { return __builtin_amdgcn_readlane(wave_scan(v), 63); }
+
+// The plan of a batch of up to 64 sequences, one per lane: its length, pages, chunks, and the inclusive prefix sums of
+// the chunks (low half) and of the partial states, the chunks of split sequences (high half; both stay below 2^15).
+// Chunk counts come from an approximate reciprocal: one more chunk than needed only leaves the last one short or empty,
+// and the pages per chunk (kv_per) are exact in the count.
+struct KvBatch {
+  int len, pages, chunks, sums;
+};
+
+// Pages per chunk of a sequence of `pages` pages in `chunks` chunks, a multiple of `waves`
+__device__ __forceinline__ int kv_per(int pages, int chunks, int waves) {
+  return (int)(((unsigned)(pages + chunks - 1) / (unsigned)chunks + waves - 1) & -(unsigned)waves);
+}
+
+__device__ __forceinline__ KvBatch kv_batch(const KvSplit& s, const int* __restrict__ seq_lens, int waves) {
+  const int lane = threadIdx.x & 63;
+  asm volatile("" ::"s"(s.by_length), "s"(s.batch), "s"(s.max_tokens), "s"(s.target), "s"(s.slots), "s"(s.inv_target),
+               "s"(s.inv_slots), "s"(seq_lens));
+  KvBatch k;
+  k.len = max(min(seq_lens[min(lane, s.batch - 1)], s.max_tokens), 0);
+  k.len = lane < s.batch ? k.len : 0;
+  k.pages = (k.len + kPage - 1) / kPage;
+  const float np = (float)k.pages;
+  auto chunks_of = [&](int cp) { return (int)__builtin_ceilf(np * __builtin_amdgcn_rcpf((float)cp)); };
+  auto both = [](int c) { return c > 1 ? c * 0x10001 : c; };
+  auto up = [&](float pages) { return (int)(((unsigned)(int)pages + waves) & -(unsigned)waves); };  // above `pages`
+  // one sequence: every lane takes lane 0's value for the sum over the lanes
+  auto scan = [&](int v) { return s.batch == 1 ? __builtin_amdgcn_readfirstlane(v) : wave_scan(v); };
+  auto total_of = [&](int sums) { return __builtin_amdgcn_readlane(sums, 63); };
+  const float total = (float)total_of(scan(k.pages));
+  const int live = __builtin_popcountll(__builtin_amdgcn_ballot_w64(k.pages > 0));
+  // Chunks of an equal share of the batch, if that gives no more chunks than workgroups aimed at (one per CU: a CU
+  // with two takes twice as long) and the partial states fit.  Each sequence's last chunk is short, so a ragged batch
+  // needs longer ones: a share that leaves half or three quarters of a chunk per sequence is tried next, a whole one
+  // always does.  With more sequences than that the share stands, unless the partial states don't fit; chunks of
+  // three times the mean over the slots always fit (fewer than 2 n / cp + 1 chunks in a split sequence of n pages).
+  const bool crowded = 2 * live > s.target;
+  auto fits = [&](int sums) { return (sums >> 16) <= s.slots && (crowded || (sums & 0xFFFF) <= s.target); };
+  const int share = up(total * s.inv_target - 0.5f);
+  k.chunks = chunks_of(share);
+  k.sums = scan(both(k.chunks));
+  if (!fits(total_of(k.sums))) {
+    const float room = (float)max(min(s.target, s.slots) - live, 1);  // chunks left when each sequence wastes one
+    auto leaving = [&](float part) { return up(total * __builtin_amdgcn_rcpf(room + part * live)); };
+    const int half = crowded ? share + share / 2 : leaving(0.5f), most = crowded ? 2 * share : leaving(0.25f);
+    const int last = crowded ? up(fmaxf(3.f * total * s.inv_slots, 2.f * share)) : leaving(0.f);
+    const int b = wave_total(both(chunks_of(half))), c = wave_total(both(chunks_of(most)));
+    k.chunks = chunks_of(fits(b) ? half : fits(c) ? most : last);
+    k.sums = wave_scan(both(k.chunks));
+  }
+  return k;
+}
+
+// A workgroup's chunk: pages [p0, p1) of sequence b of length len; slot: its partial state, -1 when it is the whole
+// sequence; b = -1 past the last chunk.
+struct KvChunk {
+  int b, len, p0, p1, slot;
+};
+
+__device__ __forceinline__ KvChunk kv_chunk_at(const KvSplit& s, const int* __restrict__ seq_lens, int index,
+                                               int waves) {
+  if (!s.by_length) {
+    const int b = s.chunks == 1 ? index : index / s.chunks, i = index - b * s.chunks;
+    return KvChunk{b, min(seq_lens[b], s.max_tokens), i * s.chunk_pages, (i + 1) * s.chunk_pages,
+                   s.chunks > 1 ? index : -1};
+  }
+  const KvBatch k = kv_batch(s, seq_lens, waves);
+  if (index >= (__builtin_amdgcn_readlane(k.sums, 63) & 0xFFFF)) return KvChunk{-1, 0, 0, 0, -1};
+  const int at = __builtin_popcountll(__builtin_amdgcn_ballot_w64((k.sums & 0xFFFF) <= index));
+  const int pages = __builtin_amdgcn_readlane(k.pages, at), chunks = __builtin_amdgcn_readlane(k.chunks, at);
+  const int sums = __builtin_amdgcn_readlane(k.sums, at);
+  const int i = index - ((sums & 0xFFFF) - chunks);
+  const int per = chunks == 1 ? pages : kv_per(pages, chunks, waves);
+  return KvChunk{at, __builtin_amdgcn_readlane(k.len, at), i * per, (i + 1) * per,
+                 chunks > 1 ? (sums >> 16) - chunks + i : -1};
+}
+
+// The chunks of sequence b for the merge: their count, and the first one's partial state
+__device__ __forceinline__ int2 kv_chunks_at(const KvSplit& s, const int* __restrict__ seq_lens, int b, int waves) {
+  if (!s.by_length) return int2{s.chunks, b * s.chunks};
+  const KvBatch k = kv_batch(s, seq_lens, waves);
+  const int chunks = __builtin_amdgcn_readlane(k.chunks, b);
+  return int2{chunks, (__builtin_amdgcn_readlane(k.sums, b) >> 16) - chunks};
+}
+
 template <int BITS, int DEPTH, int WAVES>
 __global__ __launch_bounds__(WAVES * 64) void kv_decode_kernel(
     const _Float16* __restrict__ q, const uint8_t* kc, const uint8_t* vc, const uint16_t* ksc, const uint16_t* vsc,
     int num_pages,
     const int* __restrict__ page_table, int max_pages, const int* __restrict__ seq_lens, int Hq, int Hkv,
-    float qk_scale, int chunk_pages, float* __restrict__ part_o, float* __restrict__ part_ml,
+    float qk_scale, KvSplit split, float* __restrict__ part_o, float* __restrict__ part_ml,
     _Float16* __restrict__ out) {
   constexpr int ROW = KvRegs<BITS>::ROW;
   extern __shared__ float red[];  // [WAVES][G][D + 1] then [WAVES][G][2]
-  const int chunk = blockIdx.x, hk = blockIdx.y, b = blockIdx.z;
+  const int hk = blockIdx.x;
+  const KvChunk ch = kv_chunk_at(split, seq_lens, blockIdx.y, WAVES);
+  if (ch.b < 0) return;
+  const int b = ch.b, L = ch.len;
   const int G = Hq / Hkv;
-  const int L = min(seq_lens[b], max_pages * kPage);
   const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int l = threadIdx.x & 63;
   const int n = l & 15, g = l >> 4;
@@ -248,8 +362,8 @@ __global__ __launch_bounds__(WAVES * 64) void kv_decode_kernel(
   for (int db = 0; db < 8; db++) s.o[db] = float4_t{0.f, 0.f, 0.f, 0.f};
 
   // this wave's pages: logical pages p0 + w, p0 + w + WAVES, ... below min(chunk end, pages of the sequence)
-  const int p0 = chunk * chunk_pages;
-  const int p_end = min(p0 + chunk_pages, (L + kPage - 1) / kPage);
+  const int p0 = ch.p0;
+  const int p_end = min(ch.p1, (L + kPage - 1) / kPage);
   const int* ptab = page_table + (size_t)b * max_pages;
   const size_t blk_bytes = (size_t)kPage * ROW;
   int lp = p0 + w;
@@ -310,14 +424,14 @@ __global__ __launch_bounds__(WAVES * 64) void kv_decode_kernel(
 #pragma unroll
     for (int e = 0; e < 8; e++) acc[e] += src[e] * f;
   }
-  if (gridDim.x == 1) {  // one chunk per sequence: its state is the result (no merge launch)
+  if (ch.slot < 0) {  // the whole sequence: its state is the result
     half8_t h;
 #pragma unroll
     for (int e = 0; e < 8; e++) h[e] = (_Float16)(lsum > 0.f ? acc[e] / lsum : 0.f);
     *reinterpret_cast<half8_t*>(out + ((size_t)b * Hq + hk * G + tq) * kHeadDim + td) = h;
     return;
   }
-  const size_t slot = (((size_t)b * Hkv + hk) * gridDim.x + chunk) * G + tq;
+  const size_t slot = ((size_t)ch.slot * Hkv + hk) * G + tq;
   float4_t* po = reinterpret_cast<float4_t*>(part_o + slot * kHeadDim + td);
   po[0] = float4_t{acc[0], acc[1], acc[2], acc[3]};
   po[1] = float4_t{acc[4], acc[5], acc[6], acc[7]};
@@ -329,19 +443,23 @@ __global__ __launch_bounds__(WAVES * 64) void kv_decode_kernel(
 
 // out[b][h] = sum_c 2^(m_c - M) O_c / sum_c 2^(m_c - M) l_c.  One workgroup per query head; wave w folds chunks
 // w, w+4, ... into a running (M, L, O) (lane: dims 2l, 2l+1), then the 4 waves combine in LDS.  Fixed order.
+// A sequence of one chunk has its output already; an empty sequence gets zeros.
 __global__ __launch_bounds__(kMergeWaves * 64) void kv_merge_kernel(const float* __restrict__ part_o,
-                                                       const float* __restrict__ part_ml, int Hq, int Hkv, int chunks,
+                                                       const float* __restrict__ part_ml, int Hq, int Hkv,
+                                                       const int* __restrict__ seq_lens, KvSplit split, int waves,
                                                        _Float16* __restrict__ out) {
   __shared__ float sm_ml[kMergeWaves][2];
   __shared__ float sm_o[kMergeWaves][kHeadDim];
   const int h = blockIdx.x, b = blockIdx.y;
   const int G = Hq / Hkv, hk = h / G, q = h - hk * G;
   const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), l = threadIdx.x & 63;
-  const size_t base = ((size_t)b * Hkv + hk) * chunks;  // slot of chunk c: (base + c) * G + q
+  const int2 cs = kv_chunks_at(split, seq_lens, b, waves);
+  const int chunks = cs.x;
+  if (chunks == 1) return;
   float M = -INFINITY, L = 0.f, a0 = 0.f, a1 = 0.f;
 #pragma unroll 4
   for (int c = w; c < chunks; c += kMergeWaves) {
-    const size_t slot = (base + c) * G + q;
+    const size_t slot = ((size_t)(cs.y + c) * Hkv + hk) * G + q;
     const float mc = part_ml[slot * 2], lc = part_ml[slot * 2 + 1];
     const float2 oc = *reinterpret_cast<const float2*>(part_o + slot * kHeadDim + 2 * l);
     const float mn = fmaxf(M, mc);
@@ -375,7 +493,7 @@ __global__ __launch_bounds__(kMergeWaves * 64) void kv_merge_kernel(const float*
   out[((size_t)b * Hq + h) * kHeadDim + d] = (_Float16)(lsum > 0.f ? acc / lsum : 0.f);
 }
 
-// Workgroup shape and pages per workgroup.  8 waves per workgroup and chunks that fill the GPU about one workgroup
+// Workgroup shape, and the fixed plan's pages per workgroup (it sizes the workspace for the split by lengths too).  8 waves per workgroup and chunks that fill the GPU about one workgroup
 // per CU (256) deep; groups whose 8-wave LDS merge would pass 64 KB take 4 waves and about 1024 workgroups.  Fewer
 // chunks mean fewer partial states to write and merge: at 16 sequences x 8 kv heads, 2 chunks of 8 waves measured 3 %
 // faster (8-bit) than 8 chunks of 4 waves, and 4 chunks of 8 waves or 2 of 16 no faster than 2 of 8.  chunk_pages is
@@ -385,18 +503,21 @@ struct KvPlan {
 };
 // EXL3_KV_WAVES (4 or 8) and EXL3_KV_TARGET_WGS override the plan for measurements; read once per process, so the
 // workspace size and the launch always follow the same plan.
+static int kv_target(int waves) {
+  static const int env_target = [] {
+    const char* e = getenv("EXL3_KV_TARGET_WGS");
+    return e ? std::max(1, atoi(e)) : 0;
+  }();
+  return env_target ? env_target : waves == 8 ? 256 : 1024;
+}
 static KvPlan kv_plan(int batch, int num_kv_heads, int group, int max_pages) {
   static const int env_waves = [] {
     const char* e = getenv("EXL3_KV_WAVES");
     return e && atoi(e) == 4 ? 4 : kKvWaves;
   }();
-  static const int env_target = [] {
-    const char* e = getenv("EXL3_KV_TARGET_WGS");
-    return e ? std::max(1, atoi(e)) : 0;
-  }();
   int waves = env_waves;
   if ((size_t)waves * group * (kHeadDim + 1 + 2) * sizeof(float) > 65536) waves = 4;
-  const int target = env_target ? env_target : waves == 8 ? 256 : 1024;
+  const int target = kv_target(waves);
   const long pairs = (long)batch * num_kv_heads;
   const long chunks = std::max(1L, std::min((long)(max_pages + waves - 1) / waves, (target + pairs - 1) / pairs));
   int cp = (int)((max_pages + chunks - 1) / chunks);
@@ -443,7 +564,17 @@ extern "C" int exl3_kv_decode_attention(const void* q, const void* k_cache, cons
   const float qk_scale = sm_scale * 1.4426950408889634f;  // logits in base 2
   const size_t lds = (size_t)plan.waves * G * (kHeadDim + 1 + 2) * sizeof(float);
   hipStream_t st = as_stream(stream);
-  const dim3 grid(chunks, num_kv_heads, batch);
+  // The split by lengths, with the merge launch, unless one chunk per sequence needs no merge and either the table is
+  // short (8 pages per wave) or the pairs fill the GPU twice; batches past 64 sequences keep the fixed plan.
+  const bool by_length = batch <= 64 && max_pages > plan.waves &&
+                         !(chunks == 1 && (max_pages <= 8 * plan.waves || (long)batch * num_kv_heads >= 512));
+  const int target = (kv_target(plan.waves) + num_kv_heads - 1) / num_kv_heads, slots = batch * chunks;
+  const KvSplit split{by_length, batch, max_pages * kPage, target, slots, 1.0f / target, 1.0f / slots, plan.chunk_pages,
+                      chunks};
+  // by lengths: at most `slots` chunks of split sequences, and one for every other sequence.  The kv head is the fast
+  // index: workgroups past the last chunk then come last and take no CU from a chunk (with the chunk fast, 16 x 4k
+  // 26 -> 37 us), and the heads of a page, adjacent in memory, are read together.
+  const dim3 grid(num_kv_heads, by_length ? slots + batch : slots);
   auto qp = static_cast<const _Float16*>(q);
   auto kp = static_cast<const uint8_t*>(k_cache);
   auto vp = static_cast<const uint8_t*>(v_cache);
@@ -462,12 +593,12 @@ extern "C" int exl3_kv_decode_attention(const void* q, const void* k_cache, cons
       {{kv_decode_kernel<4, 2, 8>, kv_decode_kernel<4, 3, 8>, kv_decode_kernel<4, 4, 8>, kv_decode_kernel<4, 5, 8>},
        {kv_decode_kernel<8, 2, 8>, kv_decode_kernel<8, 3, 8>, kv_decode_kernel<8, 4, 8>, kv_decode_kernel<8, 5, 8>}}};
   table[plan.waves == 8][bits == 8][depth - 2]<<<grid, plan.waves * 64, lds, st>>>(
-      qp, kp, vp, ksp, vsp, num_pages, pt, max_pages, sl, num_q_heads, num_kv_heads, qk_scale, plan.chunk_pages,
+      qp, kp, vp, ksp, vsp, num_pages, pt, max_pages, sl, num_q_heads, num_kv_heads, qk_scale, split,
       part_o, part_ml, static_cast<_Float16*>(out));
   EXL3_CHECK_LAUNCH();
-  if (chunks > 1) {
+  if (by_length || chunks > 1) {
     kv_merge_kernel<<<dim3(num_q_heads, batch), kMergeWaves * 64, 0, st>>>(part_o, part_ml, num_q_heads,
-                                                                           num_kv_heads, chunks,
+                                                                           num_kv_heads, sl, split, plan.waves,
                                                                            static_cast<_Float16*>(out));
     EXL3_CHECK_LAUNCH();
   }
