@@ -59,6 +59,30 @@ def _run(case, prefill):
     mrel = ((y - ref).abs().max() / ref.abs().max()).item()
     assert nrel <= TOL and mrel <= TOL, (case, nrel, mrel)
 
+# The decode-GEMM's tiles of 64, 128, 192 and 256 rows at their edges: one row, a row below, at and past each height,
+# rows that leave a last tile of one row; whole tiles and shared runs of k-steps (a single k-step run included), shards
+# that end in a half tile, every width of k-step data.  (K, codebook, k, ns, rows, bf16)
+GEMM_EDGE_CASES = [(3, 1, 2048, (2176, 640), 1, False), (2, 0, 1280, (1024,), 63, False), (8, 2, 1280, (1024,), 64, True),
+                   (4, 1, 512, (384, 128), 65, False), (5, 2, 1024, (4096,), 128, False),
+                   (6, 0, 128, (128,), 129, False), (3, 1, 256, (17408, 17408), 192, False),
+                   (3, 0, 256, (17408, 17408), 193, True), (4, 2, 640, (8192, 1152), 255, False),
+                   (2, 1, 2048, (5120,), 257, False), (8, 0, 384, (896,), 385, False), (3, 1, 512, (16384,), 1025, False),
+                   (5, 1, 5120, (8192, 1024), 700, False)]
+# exl3_linear past 32 rows: large layers go to the decode-GEMM (from 4096 units of 128 x 128 weights), the last two
+# stay on the GEMV
+WIDE_LINEAR_CASES = [(3, 1, 8192, (8192,), 33, False), (4, 2, 5120, (6144, 6144, 1024), 48, True),
+                     (2, 0, 17408, (5120,), 64, False), (3, 1, 8192, (8064,), 64, False), (3, 1, 8192, (8192,), 32, False)]
+
+
+@pytest.mark.parametrize("case", GEMM_EDGE_CASES, ids=_ids(GEMM_EDGE_CASES))
+def test_gemm_tile_heights_at_their_edges(case):
+    _run(case, prefill=True)
+
+
+@pytest.mark.parametrize("case", WIDE_LINEAR_CASES, ids=_ids(WIDE_LINEAR_CASES))
+def test_linear_past_32_rows(case):
+    _run(case, prefill=False)
+
 
 @pytest.mark.parametrize("case", GEMV_CASES, ids=_ids(GEMV_CASES))
 def test_random_gemv_shapes(case):

@@ -42,6 +42,9 @@ size_t prefill_plain_workspace_bytes(int rows, int k, int n);
 int prefill_plain_gemm(const void* xh, int rows, int k, const void* trellis, int n, int K, int codebook, void* out,
                        void* workspace, size_t workspace_bytes, hipStream_t st);
 
+// Workspace bytes of the decode-GEMM for any fused linear of n_total columns (exl3_linear's large layers past 32 rows)
+size_t linear_gemm_workspace_bytes(int rows, int k, int n_total);
+
 // exl3_init_device's probe of the workgroup -> XCD assignment (exl3_linear.hip): enables split-K chains that stay
 // in one XCD's L2
 int xcd_probe(int device);

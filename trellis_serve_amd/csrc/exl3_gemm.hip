@@ -13,9 +13,18 @@
 //      (c, j) of a tile the 4 weights of column c at rows r(j, 0..3); tile row tr of the k-step supplies halves
 //      4tr..4tr+3 of the lane's 8-half B fragment.  A and B then agree on the k order of every MFMA.
 //
-// Tiling: workgroup 256 rows x 256 columns (two output rotation blocks; a shard of an odd number of 128-column blocks
-// ends in a half tile), 8 waves as 2 x 4, wave tile 128 x 64 (8 x 4 MFMA 16x16x32 tiles, 128 fp32 accumulators per
-// lane).  135 KB of LDS: one workgroup per CU, CUs tiles at once.
+// Tiling: workgroup 16 MI rows (64 to 256) x 256 columns (two output rotation blocks; a shard of an odd number of
+// 128-column blocks ends in a half tile), 8 waves.  Wave w owns 32 columns of every row: it decodes their weights into
+// registers, each once, and multiplies them (the MFMA's A operand) with the A fragments of all rows from LDS.  No
+// decoded weight goes through LDS and only the A pieces are shared between waves.  One workgroup per CU (two at 64
+// rows).  Against wave tiles of 128 x 64 with the decoded weights in LDS (two waves per weight, a barrier that the
+// step's first LDS reads wait behind): 5120 -> 16384 at 4096 rows, one k-step 1.05 -> 0.96 us, a tile's epilogue 22 ->
+// 6 us; 729-745 -> 641-676 us in all.
+//
+// What bounds it: issue.  Per k-step and wave of a 256-row tile 32 MFMAs (512 cycles) and ~90 VALU of decode (360),
+// two waves per SIMD; counted at 4096 rows: matrix core 54 % busy, VALU 37 %, 18 % both, at 2.0 GHz.  The two waves of
+// a SIMD take decode and multiply in opposite order (2-3 %); forced bursts, a deeper fragment window (8) and an explicit
+// MFMA / VALU interleave were slower.
 //
 // Work decomposition (1-D grid of work items, dispatched in order): tiles are numbered column block fastest, so
 // consecutive workgroups share their A rows in L2.  When the tile count is not a multiple of the machine's
@@ -25,20 +34,17 @@
 // run's first and last segments can cover part of a tile: such a segment stores its fp32 accumulators as a partial,
 // and the last of the tile's workgroups to arrive (a per-tile counter in the workspace's counter region) sums the
 // tile's partials in workgroup order (deterministic, independent of arrival order), then runs the same epilogue as a
-// whole tile and resets the counter.  When whole rounds would finish sooner (the partials cost about a quarter of a
-// tile-time), every tile is a whole-tile item.
+// whole tile and resets the counter.  When whole rounds would finish sooner, every tile is a whole-tile item.
 //
-// Pipeline: direct-to-LDS 16-byte buffer loads (no VGPR staging) into two 3-slot rings, one for A (per k-step each
-// wave loads 2 pieces, one m-block of 64 lanes x 16 B each: a lane's 16 bytes land exactly where its MFMA A fragment
-// lives) and one for the trellis bits (each wave loads its 4 tiles of the k-step).  A bundle of loads holds A of step
-// b and the bits of step b+1 and is issued two steps before its A is used, so every load has two steps of flight.
-// The compiler does not order LDS-DMA writes before LDS reads, so the waits are explicit (vmcnt), and one barrier per
-// k-step publishes the other waves' pieces and decoded weights.  Each k-step runs its 32 MFMAs per wave next to the
-// decode of the following k-step (32 tiles per workgroup, 4 per wave, into a double-buffered fp16 B fragment area),
-// so VALU decode work overlaps matrix work.
+// Pipeline: direct-to-LDS 16-byte buffer loads (no VGPR staging) into two 4-slot rings, one for A (a piece is a row
+// block of 64 lanes x 16 B: a lane's 16 bytes land exactly where its MFMA fragment lives) and one, private to each
+// wave, for the trellis bits.  The compiler does not order LDS-DMA writes before LDS reads, so the waits are explicit
+// (vmcnt); one barrier per k-step publishes the A pieces of the NEXT step, so that a wave's fragment reads run ahead
+// across the barrier.
 #include <stdlib.h>
 
 #include <algorithm>
+#include <type_traits>
 
 #include "exl3_api.hpp"
 #include "exl3_device.hpp"
@@ -47,20 +53,22 @@ namespace exl3 {
 
 typedef _Float16 half8_t __attribute__((ext_vector_type(8)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
-typedef float f32x2 __attribute__((ext_vector_type(2)));
 typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
 
-constexpr int kBM = 256, kBN = 256, kBK = 32;
+constexpr int kBN = 256, kBK = 32;
 constexpr int kGemmWaves = 8, kGemmThreads = kGemmWaves * 64;
-constexpr int kAStage = kBM * kBK * 2;            // 16 KB: [16 m-blocks][64 lanes][8 halves]
-constexpr int kBStage = kBN * kBK * 2;            // 16 KB: [16 n-blocks][64 lanes][8 halves]
-constexpr int kBitsStage = kGemmWaves * 64 * 16;  // 8 KB: per wave 64 lanes x 16 B (its 4 tiles of a k-step)
-constexpr int kRing = 3;                          // A and bits ring slots
-constexpr int kCStride = kBN + 8;                 // epilogue fp16 C tile row stride (halves)
-constexpr int kCoherentStore = 1 << 4;            // buffer cache policy sc1: device-scope coherent access
-constexpr int kPartialBytes = kBM * kBN * 4;      // one fp32 partial tile
-constexpr int kLoadRegion = kRing * (kAStage + kBitsStage) + 2 * kBStage;
-constexpr int kGemmLds = kLoadRegion > kBM * kCStride * 2 ? kLoadRegion : kBM * kCStride * 2;  // 135 KB: 1 per CU
+constexpr int kARing = 4, kBitsRing = 4;           // ring slots (powers of two)
+constexpr int kWindow = 4;                         // A fragments a wave holds ahead of their MFMAs
+constexpr int kBitsStage = kGemmWaves * 64 * 16;   // 8 KB: per wave 64 lanes x 16 B (its 4 tiles of a k-step)
+constexpr int kCStride = kBN + 8;                  // epilogue fp16 C tile row stride (halves)
+constexpr int kCoherentStore = 1 << 4;             // buffer cache policy sc1: device-scope coherent access
+constexpr int kPastEnd = 0x7FFFFFF0;               // a buffer offset past every partial
+// LDS of a tile of 16 MI rows: the rings, or the C tile of the epilogue
+__host__ __device__ constexpr int gemm_lds(int MI) {
+  const int rings = kARing * MI * 1024 + kBitsRing * kBitsStage, c = MI * 16 * kCStride * 2;
+  return rings > c ? rings : c;
+}
+constexpr size_t gemm_partial_bytes(int MI) { return (size_t)MI * 16 * kBN * 4; }  // one fp32 partial tile
 
 struct GemmShards {
   const uint32_t* trellis[EXL3_MAX_SHARDS];
@@ -265,20 +273,35 @@ __global__ __launch_bounds__(256) void had_in_frag_kernel(const void* __restrict
   }
 }
 
+// Output rotation of a 16-row x 128-column block of the fp16 C tile by MFMA: y^T = H C^T, H the +-1 Hadamard matrix
+// (exact in fp16; products and sums in fp32), * 1/sqrt(128) rounded to fp16, * svh (fp16 product).  A operand: rows of
+// H in the order n(t, i) = 32 (t / 2) + 8 (i / 4) + 4 (t & 1) + i % 4 for MFMA t = 0..7, so that a lane's 4 results of
+// MFMAs 2u and 2u + 1 are the 8 consecutive columns 32 u + 8 (l / 16) of row l % 16: one 16-byte store.  The sign of
+// H[n][k] at k = 32 kb + 8 (l / 16) + e splits into a part of the lane and e (had_frag), one of (t & 1, e) and one of
+// (t / 2, kb).
+__device__ __forceinline__ half8_t had_frag(int l) {
+  const int i = l & 15, j = l >> 4;
+  half8_t f;
+#pragma unroll
+  for (int e = 0; e < 8; e++)
+    f[e] = (__builtin_popcount(((i & 3) & (e & 3)) | ((((i >> 2) & j)) << 2)) & 1) ? (_Float16)-1.0f : (_Float16)1.0f;
+  return f;
+}
+
 // One segment of work: k-steps [kt0, kt1) of tile `tile`.  seg < 0: the whole tile, straight to the epilogue;
 // seg = 0 / 1: a stream-K segment at the start / end of workgroup `item`'s run, stored as that partial slot; the
 // last of the tile's workgroups to arrive sums every partial of the tile in workgroup order and runs the epilogue.
-// FEW (a launch of fewer than 256 rows, one row block): the MFMAs and A-fragment reads of 16-row blocks past M are
-// skipped (their accumulators stay zero and are never stored); every load, decode and barrier is unchanged.
-template <int K, int CB, bool Y_BF16, bool FEW>
+template <int K, int CB, int MI>
 __device__ __forceinline__ void gemm_segment(const GemmShards& sa, const GemmPlan& plan, int M, int k,
-                                             void* __restrict__ y, int n_total, int rotate_out, uint8_t* lds,
-                                             int item, int tile, int kt0, int kt1, int seg) {
+                                             void* __restrict__ y, int y_bf16, int n_total, int rotate_out,
+                                             uint8_t* lds, int item, int tile, int kt0, int kt1, int seg) {
   constexpr int CHUNKS = gemm_chunks<K>();
   static_assert(CHUNKS <= 64, "one gather per wave per k-step");
-  uint8_t* a_ring = lds;                             // [kRing][kAStage]
-  uint8_t* bits_ring = lds + kRing * kAStage;        // [kRing][8 waves][64 lanes][16 B]
-  uint8_t* b_lds = bits_ring + kRing * kBitsStage;   // [2][kBStage] decoded B fragments
+  constexpr int kRows = 16 * MI;
+  constexpr int kAStage = kRows * kBK * 2;
+  constexpr int PIECES = (MI + kGemmWaves - 1) / kGemmWaves;  // A pieces (16 rows) a wave loads per k-step
+  uint8_t* a_ring = lds;                          // [kARing][MI row blocks][64 lanes][8 halves]
+  uint8_t* bits_ring = lds + kARing * kAStage;    // [kBitsRing][8 waves][64 lanes][16 B]
 
   const int ct = tile % plan.nct, mblk = tile / plan.nct;
   int s = 0;
@@ -289,142 +312,159 @@ __device__ __forceinline__ void gemm_segment(const GemmShards& sa, const GemmPla
   const int tc0 = (ct - sa.ct0[s]) * 16;  // first tile column of this tile in the shard
   const int ntc = min(16, tn - tc0);      // tile columns present: 16, or 8 at the end of a shard of odd 128-blocks
   const int col0 = sa.col0[s] + tc0 * 16;  // first output column
-  const int row0 = mblk * kBM;
+  const int row0 = mblk * kRows;
 
   const int tid = threadIdx.x;
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int l = tid & 63;
-  const int wm = w >> 2, wn = w & 3;  // wave tile: rows 128 wm .., columns 64 wn ..
   const int c = l & 15, j = l >> 4;
-  const bool mfma_wave = 4 * wn < ntc;  // wave-uniform: its 64 columns exist
-  // 16-row blocks of the wave tile that hold rows below M (wave-uniform; all 8 unless FEW)
-  const int live_mi = FEW ? max(0, min(8, (M - row0 - wm * 128 + 15) / 16)) : 8;
+  const bool mfma_wave = 2 * w < ntc;  // wave-uniform: its 32 columns exist
 
-  // B: wave w loads and decodes tile row btr = w >> 2, tile columns btc .. btc+3 (btc = 4 (w & 3)) of every k-step;
-  // past the end of a half tile it re-reads the tile's first columns (in range, decoded into n-blocks nobody reads)
-  const int btr = w >> 2, btc = 4 * (w & 3);
+  // B: wave w loads and decodes its own two tile columns 2w, 2w + 1 (both tile rows of the k-step); past the end of a
+  // half tile it re-reads the tile's first columns (in range, never stored)
   const int tile_bytes = 32 * K;
   const int row_bytes = tn * tile_bytes;
   const __amdgpu_buffer_rsrc_t brsrc =
       __builtin_amdgcn_make_buffer_rsrc((void*)sa.trellis[s], (short)0, (k >> 4) * row_bytes, 0x00020000);
-  // STORED: the 4 tiles are adjacent in their tile row (+ tile row * row_bytes); BLOCKS: 8 tiles apart inside the
-  // unit of the column block (+ the unit of the 128-row block and the row inside it, per k-step)
+  // stage order [tile row][column][32K bytes].  STORED: the two columns are adjacent in their tile row; BLOCKS: the
+  // tiles of a column are adjacent, the columns 8 tiles apart inside the unit of the column block
   const bool blocks = sa.layout[s] == EXL3_LAYOUT_BLOCKS;
-  const int bj0 = tc0 + (btc < ntc ? btc : 0), bL = min(l, CHUNKS - 1);
-  const int bgoff = blocks ? ((bj0 >> 3) * (k >> 7) * 64 + ((bj0 & 7) + bL / (2 * K)) * 8) * tile_bytes +
-                                 (bL % (2 * K)) * 16
-                           : bj0 * tile_bytes + bL * 16;
+  const int bL = l < CHUNKS ? l : CHUNKS - 1, brow = bL / (4 * K), bcol = bL % (4 * K) / (2 * K), bpiece = bL % (2 * K);
+  const int bj = tc0 + (mfma_wave ? 2 * w : 0) + bcol;
+  const int bgoff = (blocks ? ((bj >> 3) * (k >> 7) * 64 + (bj & 7) * 8 + brow) * tile_bytes
+                            : brow * row_bytes + bj * tile_bytes) + bpiece * 16;
   const LaneGeo g = lane_geo<K>(c, j);
 
-  // A: wave w loads m-blocks 2w, 2w+1; lane l of a piece = row (l % 16) of the m-block, k-chunk l / 16.  Rows past
-  // M re-read row M-1 (finite, only feeds discarded C rows).
+  // A: lane l of a piece = row (l % 16) of the row block, k-chunk l / 16.  Rows past M re-read row M-1 (finite, only
+  // feeds discarded C rows).
   const uint16_t* xh = sa.xh[s];
   const __amdgpu_buffer_rsrc_t arsrc =
       __builtin_amdgcn_make_buffer_rsrc((void*)xh, (short)0, M * k * 2, 0x00020000);
-  int aoff[2];
+  int aoff[PIECES], apiece[PIECES];
 #pragma unroll
-  for (int q = 0; q < 2; q++) {
-    const int row = min(row0 + (2 * w + q) * 16 + c, M - 1);
-    aoff[q] = (row * 32 + j * 8) * 2;  // + k-step * M * 64 bytes
+  for (int q = 0; q < PIECES; q++) {
+    const int p = PIECES * w + q;
+    apiece[q] = p < MI ? p : p % MI;  // fewer pieces than waves: the others load one again (the same bytes)
+    const int row = row0 + apiece[q] * 16 + c;
+    aoff[q] = ((row < M ? row : M - 1) * 32 + j * 8) * 2;  // + k-step * M * 64 bytes
   }
 
-  // Loads come in bundles: bundle b = A of step b + trellis bits of step b+1 (3 loads per wave; past the end, steps
-  // clamp to the last one: in range, never used).  Step i of the item (k-step kt0 + i) reads A slot i % 3, decodes
-  // the bits of step i+1 from bits slot (i+1) % 3, and issues bundle i+2, so every load has two steps of flight.
+  // Loads come in bundles: bundle b = A of step b + trellis bits of step b + 1 (PIECES + 1 loads per wave; past the
+  // end, steps clamp to the last one: in range, never used), issued three steps ahead of the A's use and complete two
+  // steps later, one step before it: the barrier of step i publishes the A of step i + 1, so a wave reads its next
+  // fragments before the step's last MFMAs and no step starts with an LDS round trip.
   const int nk = kt1 - kt0;  // >= 1
   // (the k-step argument kt is clamped by the caller: no device-only calls inside these lambdas, whose host-side
   // instantiation would otherwise suppress the kernel's host stub)
   auto issue_a = [&](int i, int kt) {
-    uint8_t* st = a_ring + (i % kRing) * kAStage;
+    uint8_t* st = a_ring + (i & (kARing - 1)) * kAStage;
 #pragma unroll
-    for (int q = 0; q < 2; q++)
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(arsrc, (__attribute__((address_space(3))) void*)(st + (2 * w + q) * 1024),
+    for (int q = 0; q < PIECES; q++)
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(arsrc, (__attribute__((address_space(3))) void*)(st + apiece[q] * 1024),
                                                16, aoff[q], kt * M * kBK * 2, 0, 0);
   };
   auto issue_bits = [&](int i, int kt) {
-    uint8_t* st = bits_ring + (i % kRing) * kBitsStage + w * 1024;
-    const int tr = 2 * kt + btr;
+    uint8_t* st = bits_ring + (i & (kBitsRing - 1)) * kBitsStage + w * 1024;
+    const int tr = 2 * kt;
     __builtin_amdgcn_raw_ptr_buffer_load_lds(brsrc, (__attribute__((address_space(3))) void*)st, 16, bgoff,
                                              blocks ? ((tr >> 3) * 64 + (tr & 7)) * tile_bytes : tr * row_bytes, 0,
                                              0);
   };
-  // this wave's trellis words of step i (bits slot i % 3)
-  auto read_bits = [&](int i, uint32_t (&bw)[4][2]) {
-    const uint32_t* tw = reinterpret_cast<const uint32_t*>(bits_ring + (i % kRing) * kBitsStage + w * 1024);
+  // this wave's trellis words of step i: [column][tile row][word]
+  auto read_bits = [&](int i, uint32_t (&bw)[2][2][2]) {
+    const uint32_t* tw = reinterpret_cast<const uint32_t*>(bits_ring + (i & (kBitsRing - 1)) * kBitsStage + w * 1024);
 #pragma unroll
-    for (int t = 0; t < 4; t++) {
-      bw[t][0] = tw[t * 8 * K + g.dw0];
-      bw[t][1] = tw[t * 8 * K + g.dw1];
-    }
+    for (int tr = 0; tr < 2; tr++)
+#pragma unroll
+      for (int jj = 0; jj < 2; jj++) {
+        bw[jj][tr][0] = tw[(tr * 2 + jj) * 8 * K + g.dw0];
+        bw[jj][tr][1] = tw[(tr * 2 + jj) * 8 * K + g.dw1];
+      }
   };
-  // decoded weights of this wave's 4 tiles into decoded-B buffer i & 1: n-block btc + t, lane (c, j), halves
-  // 4 btr .. +3
-  auto write_b = [&](int i, const uint32_t (&bw)[4][2]) {
-    uint8_t* dst = b_lds + (i & 1) * kBStage;
-#pragma unroll
-    for (int t = 0; t < 4; t++) {
-      const half4_t v = decode_group<K, CB, false>(bw[t][0], bw[t][1], g);  // stored to LDS: no MFMA wait states
-      *reinterpret_cast<half4_t*>(dst + (((btc + t) * 64 + l) * 16) + btr * 8) = v;
-    }
+  auto frags = [&](int i) {
+    return reinterpret_cast<const half8_t*>(a_ring + (i & (kARing - 1)) * kAStage) + l;
   };
 
-  float4_t acc[8][4];
+  // weights as the A operand, activations as B: a lane's accumulator holds 4 consecutive columns of one row,
+  // acc[mi][jj][r] = C[16 mi + l % 16][32 w + 16 jj + 4 (l / 16) + r]
+  float4_t acc[MI][2];
 #pragma unroll
-  for (int mi = 0; mi < 8; mi++)
+  for (int mi = 0; mi < MI; mi++)
 #pragma unroll
-    for (int jj = 0; jj < 4; jj++) acc[mi][jj] = float4_t{0.f, 0.f, 0.f, 0.f};
+    for (int jj = 0; jj < 2; jj++) acc[mi][jj] = float4_t{0.f, 0.f, 0.f, 0.f};
 
+  auto last = [&](int i) { return kt0 + (i < nk ? i : nk - 1); };
   issue_bits(0, kt0);
-  issue_a(0, kt0);
-  issue_bits(1, kt0 + min(1, nk - 1));
-  issue_a(1, kt0 + min(1, nk - 1));
-  issue_bits(2, kt0 + min(2, nk - 1));
-  {
-    __builtin_amdgcn_s_waitcnt(waitcnt_vm(6));  // the bits of step 0 in (bundles 0 and 1 may be in flight)
-    lds_barrier();
-    uint32_t bw[4][2];
-    read_bits(0, bw);
-    write_b(0, bw);
+#pragma unroll
+  for (int i = 0; i < 3; i++) {
+    issue_a(i, last(i));
+    issue_bits(i + 1, last(i + 1));
   }
+  half8_t bcur[2], av[kWindow];
+  uint32_t bw[2][2][2];
+  __builtin_amdgcn_s_waitcnt(waitcnt_vm(2 * (PIECES + 1)));  // bundle 0 in (bundles 1 and 2 may be in flight)
+  lds_barrier();
+  read_bits(0, bw);
+#pragma unroll
+  for (int jj = 0; jj < 2; jj++)
+    bcur[jj] = decode_two_groups<K, CB>(bw[jj][0][0], bw[jj][0][1], bw[jj][1][0], bw[jj][1][1], g);
+  read_bits(1, bw);
+#pragma unroll
+  for (int q = 0; q < kWindow; q++) av[q] = frags(0)[q * 64];
 
-  for (int i = 0; i < nk; i++) {
-    // bundle i in (A of step i, bits of step i+1); bundle i+1 may still be in flight.  The barrier makes every wave's
-    // pieces and decoded weights of step i visible and retires every read of step i-1, freeing A slot (i-1) % 3,
-    // bits slot i % 3 and decoded-B buffer (i+1) & 1.
-    __builtin_amdgcn_s_waitcnt(waitcnt_vm(3));
-    lds_barrier();
-    issue_a(i + 2, kt0 + min(i + 2, nk - 1));
-    issue_bits(i + 3, kt0 + min(i + 3, nk - 1));
-    uint32_t bw[4][2];
-    read_bits(i + 1, bw);
-    if (mfma_wave) {
-      const half8_t* af = reinterpret_cast<const half8_t*>(a_ring + (i % kRing) * kAStage) + (wm * 8) * 64 + l;
-      const half8_t* bf = reinterpret_cast<const half8_t*>(b_lds + (i & 1) * kBStage) + (wn * 4) * 64 + l;
-      half8_t bv[4], av[8];
+  auto steps = [&](auto multiply_first) {
+    constexpr bool MULTIPLY_FIRST = decltype(multiply_first)::value;
+    for (int i = 0; i < nk; i++) {
+      // bundle i + 1 in; bundle i + 2 may still be in flight.  The barrier publishes the A of step i + 1 and retires
+      // every read of step i - 1 (consumed by MFMAs issued before it), freeing its slot.
+      __builtin_amdgcn_sched_barrier(0);
+      __builtin_amdgcn_s_waitcnt(waitcnt_vm(PIECES + 1));
+      asm volatile("s_barrier" ::: "memory");
+      __builtin_amdgcn_sched_barrier(0);
+      issue_a(i + 3, last(i + 3));
+      issue_bits(i + 4, last(i + 4));
+      uint32_t bn[2][2][2];
+      read_bits(i + 2, bn);
+      const half8_t *af = frags(i), *an = frags(i + 1);
+      half8_t bnext[2];
+      auto decode = [&]() {
 #pragma unroll
-      for (int jj = 0; jj < 4; jj++) bv[jj] = bf[jj * 64];
+        for (int jj = 0; jj < 2; jj++)
+          bnext[jj] = decode_two_groups<K, CB>(bw[jj][0][0], bw[jj][0][1], bw[jj][1][0], bw[jj][1][1], g);
+      };
+      auto multiply = [&]() {
 #pragma unroll
-      for (int mi = 0; mi < 8; mi++)
-        if (mi < live_mi) av[mi] = af[mi * 64];
+        for (int mi = 0; mi < MI; mi++) {
+          const half8_t a = av[mi % kWindow];
+          av[mi % kWindow] = mi + kWindow < MI ? af[(mi + kWindow) * 64] : an[(mi + kWindow - MI) * 64];
 #pragma unroll
-      for (int mi = 0; mi < 8; mi++)
-        if (mi < live_mi)
+          for (int jj = 0; jj < 2; jj++)
+            acc[mi][jj] = __builtin_amdgcn_mfma_f32_16x16x32_f16(bcur[jj], a, acc[mi][jj], 0, 0, 0);
+        }
+      };
+      // the two waves of a SIMD (w and w + 4) take the step's halves in opposite order
+      if constexpr (MULTIPLY_FIRST) {
+        multiply();
+        decode();
+      } else {
+        decode();
+        multiply();
+      }
 #pragma unroll
-          for (int jj = 0; jj < 4; jj++)
-            acc[mi][jj] = __builtin_amdgcn_mfma_f32_16x16x32_f16(av[mi], bv[jj], acc[mi][jj], 0, 0, 0);
+      for (int jj = 0; jj < 2; jj++) {
+        bcur[jj] = bnext[jj];
+#pragma unroll
+        for (int tr = 0; tr < 2; tr++) {
+          bw[jj][tr][0] = bn[jj][tr][0];
+          bw[jj][tr][1] = bn[jj][tr][1];
+        }
+      }
     }
-    // the next step's weights (at the last step: a stale but valid stage into a buffer nobody reads)
-    write_b(i + 1, bw);
-    // interleave: the fragment and trellis-word reads first, then one MFMA per two VALU ops of the decode, then its
-    // LDS writes
-    __builtin_amdgcn_sched_group_barrier(0x100, 20, 0);  // DS reads
-#pragma unroll
-    for (int q = 0; q < 32; q++) {
-      __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);  // MFMA
-      __builtin_amdgcn_sched_group_barrier(0x002, 2, 0);  // VALU
-    }
-    __builtin_amdgcn_sched_group_barrier(0x200, 4, 0);  // DS writes
-  }
+  };
+  if (MI >= 8 && (w & 4))
+    steps(std::integral_constant<bool, (MI >= 8)>{});
+  else
+    steps(std::false_type{});
   __builtin_amdgcn_s_waitcnt(waitcnt_vm(0));  // drain the trailing re-reads of every wave before LDS is reused
   __syncthreads();
 
@@ -433,20 +473,22 @@ __device__ __forceinline__ void gemm_segment(const GemmShards& sa, const GemmPla
   // workgroup order (deterministic, independent of arrival order)
   if (seg >= 0) {
     __shared__ int last_flag;
+    constexpr int kWaveBytes = MI * 2 * 64 * 16;  // a wave's share of a partial tile
     const __amdgpu_buffer_rsrc_t prsrc = __builtin_amdgcn_make_buffer_rsrc(
-        (void*)plan.partial, (short)0, plan.groups * 2 * kGemmWaves * 32 * 64 * 16, 0x00020000);
-    auto slot_off = [&](int g, int sl) { return (((g * 2 + sl) * kGemmWaves + w) * 32 * 64 + l) * 16; };
+        (void*)plan.partial, (short)0, plan.groups * 2 * kGemmWaves * kWaveBytes, 0x00020000);
+    auto slot_off = [&](int g, int sl) { return ((g * 2 + sl) * kGemmWaves + w) * kWaveBytes + l * 16; };
+    // only the 16-row blocks that hold output rows (rows >= M and columns past a half tile are never stored): the
+    // others' offsets lie past the buffer, where stores are dropped and loads give zeros without a request, so that
+    // no access is conditional and all are in flight together
+    const int live_rows = mfma_wave ? M - row0 : 0;  // wave-uniform
+    auto off = [&](int base, int mi, int jj) { return mi * 16 < live_rows ? base + (mi * 2 + jj) * 64 * 16 : kPastEnd; };
     const int mine = slot_off(item, seg);
-    // only the 16-row blocks that hold output rows (rows >= M and columns past a half tile are never stored), so a
-    // few-row prefill moves a fraction of the 256 KB per partial
-    const int live_rows = mfma_wave ? M - row0 - wm * 128 : 0;  // wave-uniform (mi * 16 < live_rows: mi < live_mi)
 #pragma unroll
-    for (int mi = 0; mi < 8; mi++)
-      if (mi * 16 < live_rows)
+    for (int mi = 0; mi < MI; mi++)
 #pragma unroll
-        for (int jj = 0; jj < 4; jj++)
-          __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, acc[mi][jj]), prsrc,
-                                               mine + (mi * 4 + jj) * 64 * 16, 0, kCoherentStore);
+      for (int jj = 0; jj < 2; jj++)
+        __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, acc[mi][jj]), prsrc, off(mine, mi, jj), 0,
+                                               kCoherentStore);
     __builtin_amdgcn_s_waitcnt(waitcnt_vm(0));  // this thread's partial stores are at the coherence point
     __syncthreads();
     const int64_t q0 = (int64_t)tile * plan.ksteps;
@@ -464,86 +506,91 @@ __device__ __forceinline__ void gemm_segment(const GemmShards& sa, const GemmPla
       g++;
     } else {
 #pragma unroll
-      for (int mi = 0; mi < 8; mi++)
+      for (int mi = 0; mi < MI; mi++)
 #pragma unroll
-        for (int jj = 0; jj < 4; jj++) acc[mi][jj] = float4_t{0.f, 0.f, 0.f, 0.f};
+        for (int jj = 0; jj < 2; jj++) acc[mi][jj] = float4_t{0.f, 0.f, 0.f, 0.f};
     }
     for (; g <= g_last; g++) {
       const int src = slot_off(g, sk_start(plan, g) >= q0 ? 0 : 1);  // the tile is g's first segment or its last
+      constexpr int kBatch = MI < 8 ? MI : 8;
 #pragma unroll
-      for (int mi = 0; mi < 8; mi++)
-        if (mi * 16 < live_rows)
+      for (int m0 = 0; m0 < MI; m0 += kBatch) {
+        u32x4 v[kBatch][2];
 #pragma unroll
-          for (int jj = 0; jj < 4; jj++)
-            acc[mi][jj] += __builtin_bit_cast(float4_t, __builtin_amdgcn_raw_buffer_load_b128(
-                                                          prsrc, src + (mi * 4 + jj) * 64 * 16, 0, kCoherentStore));
+        for (int q = 0; q < kBatch; q++)
+          if (m0 + q < MI)
+#pragma unroll
+            for (int jj = 0; jj < 2; jj++)
+              v[q][jj] = __builtin_amdgcn_raw_buffer_load_b128(prsrc, off(src, m0 + q, jj), 0, kCoherentStore);
+#pragma unroll
+        for (int q = 0; q < kBatch; q++)
+          if (m0 + q < MI)
+#pragma unroll
+            for (int jj = 0; jj < 2; jj++) acc[m0 + q][jj] += __builtin_bit_cast(float4_t, v[q][jj]);
+      }
     }
     if (tid == 0) __hip_atomic_store(&plan.counters[tile], 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   }
 
-  // ---- epilogue: the whole fp16 C tile (256 x 256, rounded once from fp32) goes to LDS, then each thread rotates
-  // one 128-column half-row in registers -- the 128-point butterfly of had128_x4 with the same pairings and order
-  // (h = 1, 2, 4, ..., 64; lower = a + b, upper = a - b, fp32), so results are identical -- scales by svh (fp16
-  // product) and stores it.  Per-row register butterflies have no cross-lane latency: a lane-parallel rotation chains
-  // five LDS permutes per row.
+  // ---- epilogue: the fp16 C tile (rounded once from fp32) goes to LDS, 4 columns of a row per 8-byte write; then each
+  // wave rotates its share of the (16-row, 128-column) blocks by MFMA and stores them (rotate_out), or stores the rows
+  // as they are.
   _Float16* cl = reinterpret_cast<_Float16*>(lds);
   if (mfma_wave) {
 #pragma unroll
-    for (int mi = 0; mi < 8; mi++)
+    for (int mi = 0; mi < MI; mi++)
 #pragma unroll
-      for (int jj = 0; jj < 4; jj++)
-#pragma unroll
-        for (int r = 0; r < 4; r++) {
-          const int m = wm * 128 + mi * 16 + 4 * j + r;
-          const int n = wn * 64 + jj * 16 + c;
-          cl[m * kCStride + n] = (_Float16)acc[mi][jj][r];
-        }
+      for (int jj = 0; jj < 2; jj++) {
+        const float4_t v = acc[mi][jj];
+        *reinterpret_cast<half4_t*>(cl + (mi * 16 + c) * kCStride + w * 32 + jj * 16 + 4 * j) =
+            half4_t{(_Float16)v.x, (_Float16)v.y, (_Float16)v.z, (_Float16)v.w};
+      }
   }
   __syncthreads();
-  const int er = tid & (kBM - 1), eh = tid / kBM;  // row and 128-column half of this thread
-  const int m = row0 + er;
-  if (m < M && 8 * eh < ntc) {
-    const half8_t* src = reinterpret_cast<const half8_t*>(cl + er * kCStride + eh * 128);
-    float v[128];
+  const half8_t f0 = had_frag(l);
+  half8_t f1 = f0;
 #pragma unroll
-    for (int q = 0; q < 16; q++) {
-      const half8_t h = src[q];
+  for (int e = 4; e < 8; e++) f1[e] = -f0[e];
+  for (int p = w; p < MI * 2; p += kGemmWaves) {
+    const int mi = p >> 1, h = p & 1;
+    const int m = row0 + mi * 16 + c;
+    if (8 * h >= ntc || row0 + mi * 16 >= M) continue;  // wave-uniform
+    const half8_t* src = reinterpret_cast<const half8_t*>(cl + (mi * 16 + c) * kCStride + h * 128 + 8 * j);
+    half8_t cf[4];
 #pragma unroll
-      for (int e = 0; e < 8; e++) v[8 * q + e] = (float)h[e];
-    }
-    const int col = col0 + eh * 128;
+    for (int kb = 0; kb < 4; kb++) cf[kb] = src[kb * 4];
+    const int col = col0 + h * 128 + 8 * j;
+    uint16_t* yr = static_cast<uint16_t*>(y) + (size_t)(m < M ? m : M - 1) * n_total + col;
     const half8_t* sv8 = reinterpret_cast<const half8_t*>(sa.svh[s] + (col - sa.col0[s]));
-    uint16_t* yr = static_cast<uint16_t*>(y) + (size_t)m * n_total + col;
-    if (rotate_out) {
 #pragma unroll
-      for (int hs = 1; hs < 128; hs <<= 1)
-#pragma unroll
-        for (int p = 0; p < 128; p++)
-          if (!(p & hs)) {
-            const float a = v[p], bb = v[p + hs];
-            v[p] = a + bb;
-            v[p + hs] = a - bb;
-          }
-    }
-#pragma unroll
-    for (int q = 0; q < 16; q++) {
+    for (int u = 0; u < 4; u++) {
       half8_t o;
       if (rotate_out) {
-        const half8_t sv = sv8[q];
+        const half8_t sv = sv8[u * 4];
 #pragma unroll
-        for (int e = 0; e < 8; e++) o[e] = had_scale_f16(v[8 * q + e]) * sv[e];
+        for (int v = 0; v < 2; v++) {
+          float4_t d = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+          for (int kb = 0; kb < 4; kb++) {
+            const half8_t hf = v ? f1 : f0;
+            d = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_popcount(u & kb) & 1 ? -hf : hf, cf[kb], d, 0, 0, 0);
+          }
+#pragma unroll
+          for (int r = 0; r < 4; r++) o[4 * v + r] = had_scale_f16(d[r]) * sv[4 * v + r];
+        }
       } else {
-#pragma unroll
-        for (int e = 0; e < 8; e++) o[e] = (_Float16)v[8 * q + e];
+        o = cf[u];
       }
-      if constexpr (Y_BF16) {
-        u32x4 ob;
+      if (m < M) {
+        if (y_bf16) {
+          u32x4 ob;
 #pragma unroll
-        for (int e = 0; e < 4; e++)
-          ob[e] = (uint32_t)f32_to_bf16((float)o[2 * e]) | ((uint32_t)f32_to_bf16((float)o[2 * e + 1]) << 16);
-        *reinterpret_cast<u32x4*>(yr + 8 * q) = ob;
-      } else {
-        *reinterpret_cast<half8_t*>(yr + 8 * q) = o;
+          for (int e = 0; e < 4; e++)
+            ob[e] = (uint32_t)f32_to_bf16((float)o[2 * e]) | ((uint32_t)f32_to_bf16((float)o[2 * e + 1]) << 16);
+          *reinterpret_cast<u32x4*>(yr + 32 * u) = ob;
+        } else {
+          *reinterpret_cast<half8_t*>(yr + 32 * u) = o;
+        }
       }
     }
   }
@@ -552,24 +599,28 @@ __device__ __forceinline__ void gemm_segment(const GemmShards& sa, const GemmPla
 
 // Grid: the stream-K workgroups first (each walks the segments of its run of k-steps), then one workgroup per
 // remaining whole tile.
-template <int K, int CB, bool Y_BF16, bool FEW>
-__global__ __launch_bounds__(kGemmThreads) void gemm_kernel(GemmShards sa, GemmPlan plan, int M, int k,
-                                                             void* __restrict__ y, int n_total, int rotate_out) {
+template <int K, int CB, int MI>
+__global__ __launch_bounds__(kGemmThreads, MI <= 4 ? 4 : 2) void gemm_kernel(GemmShards sa, GemmPlan plan, int M, int k,
+                                                             void* __restrict__ y, int y_bf16, int n_total,
+                                                             int rotate_out) {
   extern __shared__ __align__(16) uint8_t lds[];
   const int item = blockIdx.x;
+  int64_t q, b;  // global k-steps left
   if (item >= plan.groups) {
-    gemm_segment<K, CB, Y_BF16, FEW>(sa, plan, M, k, y, n_total, rotate_out, lds, item,
-                                plan.sk_tiles + (item - plan.groups), 0, plan.ksteps, -1);
-    return;
+    q = (int64_t)(plan.sk_tiles + (item - plan.groups)) * plan.ksteps;
+    b = q + plan.ksteps;
+  } else {
+    q = sk_start(plan, item);
+    b = sk_start(plan, item + 1);
   }
-  const int64_t a = sk_start(plan, item), b = sk_start(plan, item + 1);
-  for (int64_t q = a; q < b;) {
+  const int64_t a = q;
+  while (q < b) {
     const int t = (int)(q / plan.ksteps);
     const int64_t q0 = (int64_t)t * plan.ksteps;
     const int kt0 = (int)(q - q0), kt1 = (int)(b - q0 < plan.ksteps ? b - q0 : plan.ksteps);
     const bool whole = kt0 == 0 && kt1 == plan.ksteps;
-    gemm_segment<K, CB, Y_BF16, FEW>(sa, plan, M, k, y, n_total, rotate_out, lds, item, t, kt0, kt1,
-                                whole ? -1 : (q == a ? 0 : 1));
+    gemm_segment<K, CB, MI>(sa, plan, M, k, y, y_bf16, n_total, rotate_out, lds, item, t, kt0, kt1,
+                            whole ? -1 : (q == a ? 0 : 1));
     q = q0 + kt1;
   }
 }
@@ -604,7 +655,7 @@ static int gemm_slots() {
 }
 
 struct GemmLayout {
-  int nct, sk_tiles, groups, ksteps, tiles;
+  int mi, nct, sk_tiles, groups, ksteps, tiles;
   size_t xh_bytes, partial_off, total;
 };
 
@@ -616,32 +667,60 @@ static int gemm_col_tiles(const int* shard_n, int nshards) {  // tiles of 256 co
   return t;
 }
 
-// Whole tiles in rounds of the machine, except the last (partial) round plus one full round before it (when there
-// is one), which are shared out by runs of k-steps over one workgroup per slot (stream-K): every workgroup then
-// finishes after the same number of k-steps, 1 to 2 tiles' worth, and writes at most two partial tiles.  A run keeps
-// >= 8 k-steps so the pipeline start-up stays small against its work.  Whole rounds only, when they are sooner.
-static GemmLayout gemm_layout(int rows, int k, int nct, int nshards) {
+// The decomposition of `tiles` tiles of `ksteps` k-steps over the machine's slots: whole tiles in rounds, except the
+// last (partial) round plus one full round before it (when there is one), which are shared out by runs of k-steps over
+// one workgroup per slot (stream-K): every workgroup then finishes after the same number of k-steps, 1 to 2 tiles'
+// worth, and writes at most two partial tiles.  A run keeps >= 8 k-steps so the pipeline start-up stays small against
+// its work.  Whole rounds only, when they are sooner.  us: the estimated time, from the step time of the tile height
+// and what the partials cost it (store, the last arrival's reload of every partial at one CU's bandwidth), fitted at
+// 33-1500 rows of the four 27B layers (K = 3; within ~10 %).
+struct GemmShape {
+  int mi;          // 16-row blocks per tile
+  double step_us;  // one k-step of one workgroup per CU
+  double sk_us;    // stream-K: partials, and the tile's epilogue
+};
+constexpr GemmShape kGemmShapes[] = {{4, 0.42, 20}, {8, 0.62, 24}, {12, 0.78, 32}, {16, 0.95, 42}};
+constexpr double kEpilogueUs = 8;
+
+static double gemm_share(const GemmShape& shape, int slots, int tiles, int ksteps, int* sk_tiles, int* groups) {
+  const int rounds = tiles / slots, rem = tiles - rounds * slots;
+  const double tile_us = ksteps * shape.step_us + kEpilogueUs;
+  const double whole = (rounds + (rem > 0)) * tile_us;
+  *sk_tiles = *groups = 0;
+  if (rem == 0) return whole;
+  const int sk = rounds >= 1 ? rem + slots : rem;
+  const int g = (int)std::max<int64_t>(1, std::min<int64_t>(slots, (int64_t)sk * ksteps / 8));
+  const double shared = (tiles - sk) / slots * tile_us + (double)sk * ksteps / g * shape.step_us + shape.sk_us;
+  if (shared >= whole) return whole;
+  *sk_tiles = sk;
+  *groups = g;
+  return shared;
+}
+
+// The tile height with the least estimated time: few rows (or a remainder of few rows) waste less of a low tile and
+// write smaller partials, many rows share each decoded weight in a high one.  Measured against 256-row tiles alone (us,
+// K = 3): 80 rows gate/up 99 -> 74, down 82 -> 58; 256 rows q/k/v 88 -> 61, o 76 -> 48; 700 rows q/k/v 117 -> 95.
+static GemmLayout gemm_layout(int slots, int rows, int k, int nct, int nshards) {
   GemmLayout L{};
   L.nct = nct;
   L.ksteps = k / kBK;
-  L.tiles = ((rows + kBM - 1) / kBM) * nct;
-  const int slots = gemm_slots();
-  const int rounds = L.tiles / slots, rem = L.tiles - rounds * slots;
-  if (rem > 0) {
-    const int sk = rounds >= 1 ? rem + slots : rem;
-    // in tile-times: whole tiles only take rounds + 1; stream-K takes the whole rounds left plus sk / slots plus the
-    // partial tiles' store, reload and wait (measured ~0.25 of a tile-time at 5120 -> 17408: 512 rows 156 us against
-    // 183 us whole, 768 rows 211 against 199)
-    const double whole = rounds + 1, shared = (double)(L.tiles - sk) / slots + (double)sk / slots + 0.25;
-    if (shared < whole) {
+  double best = 0;
+  for (const GemmShape& shape : kGemmShapes) {
+    const int tiles = (rows + 16 * shape.mi - 1) / (16 * shape.mi) * nct;
+    int sk, groups;
+    const double us = gemm_share(shape, slots, tiles, L.ksteps, &sk, &groups);
+    if (L.mi == 0 || us < best) {
+      best = us;
+      L.mi = shape.mi;
+      L.tiles = tiles;
       L.sk_tiles = sk;
-      L.groups = (int)std::max<int64_t>(1, std::min<int64_t>(slots, (int64_t)sk * L.ksteps / 8));
+      L.groups = groups;
     }
   }
   // [counter region (fixed place and size)][rotated activations][partials: 2 per stream-K workgroup]
   L.xh_bytes = ((size_t)nshards * rows * k * 2 + 255) & ~(size_t)255;
   L.partial_off = kCounterBytes + L.xh_bytes;
-  L.total = L.partial_off + (size_t)L.groups * 2 * kPartialBytes;
+  L.total = L.partial_off + (size_t)L.groups * 2 * gemm_partial_bytes(L.mi);
   return L;
 }
 
@@ -654,9 +733,10 @@ extern "C" size_t exl3_prefill_workspace_bytes(int rows, int k, int n_total, int
     return 0;
   // the column-tile count depends on how n_total splits into shards (a shard of an odd number of 128-column blocks
   // ends in a half tile): take the largest need over every possible count
+  const int slots = gemm_slots();
   size_t need = 0;
   for (int nct = (n_total / 128 + 1) / 2; nct <= (n_total / 128 + nshards) / 2; nct++)
-    need = std::max(need, gemm_layout(rows, k, nct, nshards).total);
+    need = std::max(need, gemm_layout(slots, rows, k, nct, nshards).total);
   return need;
 }
 
@@ -669,7 +749,7 @@ static int launch_prefill(const void* x, bool x_bf16, int rows, int k, GemmShard
                           const int* shard_n, int K, int codebook, void* y, bool y_bf16, void* workspace,
                           size_t workspace_bytes, hipStream_t st, const char* what) {
   const int nshards = sa.count;
-  const GemmLayout L = gemm_layout(rows, k, gemm_col_tiles(shard_n, nshards), nshards);
+  const GemmLayout L = gemm_layout(gemm_slots(), rows, k, gemm_col_tiles(shard_n, nshards), nshards);
   EXL3_CHECK_ARG(workspace && workspace_bytes >= L.total, "%s: workspace %zu bytes, need %zu", what,
                  workspace_bytes, L.total);
   EXL3_CHECK_ARG(L.sk_tiles <= kMaxCounters, "%s: %d stream-K tiles exceed the counter region", what, L.sk_tiles);
@@ -703,18 +783,17 @@ static int launch_prefill(const void* x, bool x_bf16, int rows, int k, GemmShard
   EXL3_CHECK_LAUNCH();
   const dim3 grid((unsigned)(L.groups + L.tiles - L.sk_tiles));
   bool ok;
-#define EXL3_GEMM_LAUNCH(YB, FEW)                                                                              \
-  ok = EXL3_GEMM_DISPATCH(K, codebook, gemm_kernel<kK, kCB, YB, FEW><<<grid, kGemmThreads, kGemmLds, st>>>( \
-                                          sa, plan, rows, k, y, n_total, ROT ? 1 : 0))
-  const bool few = rows < kBM;  // one row block, mostly rows past M
-  if (y_bf16 && few)
-    EXL3_GEMM_LAUNCH(true, true);
-  else if (y_bf16)
-    EXL3_GEMM_LAUNCH(true, false);
-  else if (few)
-    EXL3_GEMM_LAUNCH(false, true);
+#define EXL3_GEMM_LAUNCH(MI_)                                                                                   \
+  ok = EXL3_GEMM_DISPATCH(K, codebook, gemm_kernel<kK, kCB, MI_><<<grid, kGemmThreads, gemm_lds(MI_), st>>>( \
+                                          sa, plan, rows, k, y, y_bf16 ? 1 : 0, n_total, ROT ? 1 : 0))
+  if (L.mi == 4)
+    EXL3_GEMM_LAUNCH(4);
+  else if (L.mi == 12)
+    EXL3_GEMM_LAUNCH(12);
+  else if (L.mi == 8)
+    EXL3_GEMM_LAUNCH(8);
   else
-    EXL3_GEMM_LAUNCH(false, false);
+    EXL3_GEMM_LAUNCH(16);
 #undef EXL3_GEMM_LAUNCH
   if (!ok) return set_error(EXL3_ERR_INVALID, "%s: unsupported K/codebook", what);
   EXL3_CHECK_LAUNCH();
@@ -764,9 +843,13 @@ extern "C" int exl3_linear_prefill(const void* x, int x_bf16, int rows, int k, c
 
 namespace exl3 {
 
+size_t linear_gemm_workspace_bytes(int rows, int k, int n_total) {
+  return exl3_prefill_workspace_bytes(rows, k, n_total, EXL3_MAX_SHARDS);
+}
+
 size_t prefill_plain_workspace_bytes(int rows, int k, int n) {
   const int nct = (n / 128 + 1) / 2;
-  return gemm_layout(rows, k, nct, 1).total;
+  return gemm_layout(gemm_slots(), rows, k, nct, 1).total;
 }
 
 // exl3_gemm_rotated from kPrefillRows rows: the rows as given (fp16, already in the rotated basis), no output

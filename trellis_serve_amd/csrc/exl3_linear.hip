@@ -640,6 +640,14 @@ static size_t gemv_workspace_bytes(int rows, int k, int n_total, int K, int laun
          gemv_pre_bytes(rows, k, n_total, rotate);
 }
 
+// Rows that exl3_linear hands to the decode-GEMM: past 32 rows of a large layer the GEMV would stream and decode the
+// weights twice (two launches of two row groups), where one 64- or 128-row GEMM tile reads them once (48 rows, us:
+// gate/up 81.5 -> 55, down 61 -> 53).  Below 4096 units of 128 x 128 weights (q/k/v 2560, o 1920) the GEMV's one
+// four-group launch is as fast (31-39 and 29-36 us at 33-64 rows against 35-39 and 30-40).
+static bool linear_takes_gemm(int rows, int k, int n_total) {
+  return rows > kGemvPairRows && rows <= kGemvQuadRows && (size_t)(n_total / 128) * (k / 128) >= 4096;
+}
+
 // ---- split-K chain inside one XCD ---------------------------------------------------------------------------
 // The launches' grids are x = column block (fastest), y = k-split, so the splits of a column block have linear
 // workgroup ids that agree mod the column-block count.  When workgroups whose ids agree mod 8 run on one XCD (the
@@ -959,6 +967,7 @@ extern "C" size_t exl3_linear_workspace_bytes(int rows, int k, int n_total, int 
   if (rows <= 0 || k <= 0 || n_total <= 0 || k % 128 || n_total % 128 || n_total / 128 > kMaxCounters ||
       !valid_bits(K))
     return 0;
+  if (linear_takes_gemm(rows, k, n_total)) return linear_gemm_workspace_bytes(rows, k, n_total);
   // exl3_linear's launches: up to 64 rows each (1, 2 or 4 row groups per decoded tile), then the remainder
   return gemv_workspace_bytes(rows, k, n_total, K, kGemvQuadRows, true);
 }
@@ -973,6 +982,13 @@ extern "C" int exl3_linear(const void* x, int x_bf16, int rows, int k, const exl
   int n_total = 0;
   if (int rc = build_shards(shards_host, nshards, k, K, &sa, &n_total)) return rc;
   if (rows == 0) return EXL3_OK;
+  if (linear_takes_gemm(rows, k, n_total)) {
+    const size_t need = linear_gemm_workspace_bytes(rows, k, n_total);
+    EXL3_CHECK_ARG(workspace && workspace_bytes >= need, "exl3_linear: workspace %zu bytes, need %zu", workspace_bytes,
+                   need);
+    return exl3_linear_prefill(x, x_bf16, rows, k, shards_host, nshards, K, codebook, y, y_bf16, workspace,
+                               workspace_bytes, stream);
+  }
   return launch_gemv(sa, x, true, x_bf16 != 0, rows, k, K, codebook, n_total, workspace, workspace_bytes, y,
                      y_bf16 != 0, as_stream(stream), kGemvQuadRows, "exl3_linear");
 }
