@@ -493,7 +493,8 @@ __global__ __launch_bounds__(kMergeWaves * 64) void kv_merge_kernel(const float*
   out[((size_t)b * Hq + h) * kHeadDim + d] = (_Float16)(lsum > 0.f ? acc / lsum : 0.f);
 }
 
-// Workgroup shape, and the fixed plan's pages per workgroup (it sizes the workspace for the split by lengths too).  8 waves per workgroup and chunks that fill the GPU about one workgroup
+// Workgroup shape, and the fixed plan's pages per workgroup (it sizes the workspace for the split by lengths too).
+// 8 waves per workgroup and chunks that fill the GPU about one workgroup
 // per CU (256) deep; groups whose 8-wave LDS merge would pass 64 KB take 4 waves and about 1024 workgroups.  Fewer
 // chunks mean fewer partial states to write and merge: at 16 sequences x 8 kv heads, 2 chunks of 8 waves measured 3 %
 // faster (8-bit) than 8 chunks of 4 waves, and 4 chunks of 8 waves or 2 of 16 no faster than 2 of 8.  chunk_pages is
@@ -565,8 +566,9 @@ extern "C" int exl3_kv_decode_attention(const void* q, const void* k_cache, cons
   const size_t lds = (size_t)plan.waves * G * (kHeadDim + 1 + 2) * sizeof(float);
   hipStream_t st = as_stream(stream);
   // The split by lengths, with the merge launch, unless one chunk per sequence needs no merge and either the table is
-  // short (8 pages per wave) or the pairs fill the GPU twice; batches past 64 sequences keep the fixed plan.
-  const bool by_length = batch <= 64 && max_pages > plan.waves &&
+  // short (8 pages per wave) or the pairs fill the GPU twice; batches past 64 sequences keep the fixed plan, and so do
+  // tables whose fixed chunks are one page per wave already (a 1.1 us longer start for nothing).
+  const bool by_length = batch <= 64 && plan.chunk_pages > plan.waves &&
                          !(chunks == 1 && (max_pages <= 8 * plan.waves || (long)batch * num_kv_heads >= 512));
   const int target = (kv_target(plan.waves) + num_kv_heads - 1) / num_kv_heads, slots = batch * chunks;
   const KvSplit split{by_length, batch, max_pages * kPage, target, slots, 1.0f / target, 1.0f / slots, plan.chunk_pages,
