@@ -360,3 +360,45 @@ def test_moe_full_shape_single_token_mixed_bitrates(coracle):
     y = ops.moe_forward(torch.from_numpy(x).cuda(), torch.from_numpy(ids).cuda(), torch.from_numpy(w).cuda(), st, cb)
     nrel, mrel = _errs(y.cpu().numpy(), orc.moe_forward(x, ids, w, ex, None, cb, w_cache=cache))
     assert nrel <= 2e-3 and mrel <= 2e-3, (nrel, mrel)
+
+
+# The expert decode-GEMMs (many slots per expert): slots per expert at the edges of the 16-row blocks and of the tiles of
+# 64 and 128 slots, experts without slots, ids outside [0, E), an odd number of 128-column blocks of H (a half tile of
+# down), every codebook and several bitrates.  (H, I, K gate/up, K down, codebook, slots per expert, bf16)
+MOE_GEMM_CASES = [(384, 128, 3, 3, 1, (1, 15, 16, 17, 63, 64, 0, 65, 70, 33), False),
+                  (256, 256, 2, 4, 0, (127, 128, 129, 200, 256, 257, 0), True),
+                  (640, 384, 5, 6, 2, (300, 1, 180, 90), False),
+                  (128, 128, 8, 8, 1, (400,), False),
+                  (512, 640, 4, 3, 2, (65, 66, 128, 130, 48, 100), True)]
+
+
+@pytest.mark.parametrize("case", MOE_GEMM_CASES, ids=[f"H{c[0]}-I{c[1]}-K{c[2]}-{c[3]}-cb{c[4]}" for c in MOE_GEMM_CASES])
+def test_moe_expert_gemms_at_tile_edges(case):
+    """Against the float64 exact layer (the bar of this file, 2e-3; bf16 outputs 6e-3: half an ulp of bf16 is 2^-9),
+    and repeated calls bit-identical although the slots' order inside an expert is not."""
+    from trellis_serve_amd import ops
+    H, I, K, K_down, cb, counts, bf16 = case
+    E = len(counts)
+    rng = np.random.default_rng(sum(counts) + H)
+    ex = _experts(rng, E, H, I, K, K_down)
+    flat = np.concatenate([np.full(n, e) for e, n in enumerate(counts)] + [np.array([-1, E, -1])])
+    top_k = 2
+    if flat.size % top_k:
+        flat = np.append(flat, -1)
+    ids = rng.permutation(flat).reshape(-1, top_k).astype(np.int32)
+    T = ids.shape[0]
+    x = (rng.standard_normal((T, H)) * 0.1).astype(np.float16)
+    xt = torch.from_numpy(x).cuda()
+    if bf16:
+        xt = xt.bfloat16()
+        x = xt.float().cpu().numpy().astype(np.float16)
+    w = rng.random((T, top_k)).astype(np.float32)
+    st = _stack(ex)
+    args = (torch.from_numpy(ids).cuda(), torch.from_numpy(w).cuda(), st, cb)
+    y = ops.moe_forward(xt, *args)
+    ref = orc.moe_forward(x, ids, w, ex, None, cb)
+    nrel, mrel = _errs(y.float().cpu().numpy(), ref)
+    tol = 6e-3 if bf16 else 2e-3
+    assert nrel <= tol and mrel <= tol, (case, nrel, mrel)
+    for _ in range(3):
+        assert torch.equal(ops.moe_forward(xt, *args), y)

@@ -154,3 +154,18 @@ def test_mixed_stage_chain_matches_exact_layer(coracle, layer):
         assert nrel <= 2e-3 and mrel <= 2e-3, (t, nrel, mrel)
     fused = ops.moe_forward_classes(x, ids, w, classes, E, CB).cpu().numpy().astype(np.float64)
     assert np.abs(y - fused).max() <= 2e-3 * np.abs(fused).max()
+
+
+def test_mixed_layer_through_the_expert_gemms(layer, coracle):
+    """320 tokens (20 slots per expert: the expert decode-GEMMs), two K classes: sampled tokens against the exact layer,
+    repeats bit-identical."""
+    rng, ex, classes = layer
+    x = (rng.standard_normal((320, H)) * 0.05).astype(np.float16)
+    ids, w = _routing(rng, 320)
+    y = _ops().moe_forward_classes(torch.from_numpy(x).cuda(), ids, w, classes, E, CB)
+    toks = [0, 101, 319]
+    exact = _exact(coracle, ex, {}, x, ids.cpu().numpy(), w.cpu().numpy(), toks)
+    ref = np.stack([exact[t] for t in toks])
+    nrel, mrel = _errs(y[toks].cpu().numpy(), ref)
+    assert nrel <= 2e-3 and mrel <= 2e-3, (nrel, mrel)
+    assert torch.equal(_ops().moe_forward_classes(torch.from_numpy(x).cuda(), ids, w, classes, E, CB), y)

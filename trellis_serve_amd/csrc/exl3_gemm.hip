@@ -44,30 +44,18 @@
 #include <stdlib.h>
 
 #include <algorithm>
-#include <type_traits>
 
 #include "exl3_api.hpp"
 #include "exl3_device.hpp"
+#include "exl3_tile.hpp"
 
 namespace exl3 {
 
 typedef _Float16 half8_t __attribute__((ext_vector_type(8)));
-typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
 
-constexpr int kBN = 256, kBK = 32;
-constexpr int kGemmWaves = 8, kGemmThreads = kGemmWaves * 64;
-constexpr int kARing = 4, kBitsRing = 4;           // ring slots (powers of two)
-constexpr int kWindow = 4;                         // A fragments a wave holds ahead of their MFMAs
-constexpr int kBitsStage = kGemmWaves * 64 * 16;   // 8 KB: per wave 64 lanes x 16 B (its 4 tiles of a k-step)
-constexpr int kCStride = kBN + 8;                  // epilogue fp16 C tile row stride (halves)
 constexpr int kCoherentStore = 1 << 4;             // buffer cache policy sc1: device-scope coherent access
 constexpr int kPastEnd = 0x7FFFFFF0;               // a buffer offset past every partial
-// LDS of a tile of 16 MI rows: the rings, or the C tile of the epilogue
-__host__ __device__ constexpr int gemm_lds(int MI) {
-  const int rings = kARing * MI * 1024 + kBitsRing * kBitsStage, c = MI * 16 * kCStride * 2;
-  return rings > c ? rings : c;
-}
 constexpr size_t gemm_partial_bytes(int MI) { return (size_t)MI * 16 * kBN * 4; }  // one fp32 partial tile
 
 struct GemmShards {
@@ -103,9 +91,6 @@ __host__ __device__ __forceinline__ int sk_owner(const GemmPlan& p, int64_t q) {
 
 // lds_barrier() (exl3_device.hpp) between k-steps: the direct-to-LDS writes are waited for explicitly (waitcnt_vm)
 // before each barrier.
-
-template <int K>
-__host__ __device__ constexpr int gemm_chunks() { return 4 * 32 * K / 16; }  // 16-byte pieces of a wave's 4 tiles
 
 // per-shard input scales of one prefill call (the rotation runs every shard in one launch)
 struct ShardSuh {
@@ -273,21 +258,6 @@ __global__ __launch_bounds__(256) void had_in_frag_kernel(const void* __restrict
   }
 }
 
-// Output rotation of a 16-row x 128-column block of the fp16 C tile by MFMA: y^T = H C^T, H the +-1 Hadamard matrix
-// (exact in fp16; products and sums in fp32), * 1/sqrt(128) rounded to fp16, * svh (fp16 product).  A operand: rows of
-// H in the order n(t, i) = 32 (t / 2) + 8 (i / 4) + 4 (t & 1) + i % 4 for MFMA t = 0..7, so that a lane's 4 results of
-// MFMAs 2u and 2u + 1 are the 8 consecutive columns 32 u + 8 (l / 16) of row l % 16: one 16-byte store.  The sign of
-// H[n][k] at k = 32 kb + 8 (l / 16) + e splits into a part of the lane and e (had_frag), one of (t & 1, e) and one of
-// (t / 2, kb).
-__device__ __forceinline__ half8_t had_frag(int l) {
-  const int i = l & 15, j = l >> 4;
-  half8_t f;
-#pragma unroll
-  for (int e = 0; e < 8; e++)
-    f[e] = (__builtin_popcount(((i & 3) & (e & 3)) | ((((i >> 2) & j)) << 2)) & 1) ? (_Float16)-1.0f : (_Float16)1.0f;
-  return f;
-}
-
 // One segment of work: k-steps [kt0, kt1) of tile `tile`.  seg < 0: the whole tile, straight to the epilogue;
 // seg = 0 / 1: a stream-K segment at the start / end of workgroup `item`'s run, stored as that partial slot; the
 // last of the tile's workgroups to arrive sums every partial of the tile in workgroup order and runs the epilogue.
@@ -295,13 +265,10 @@ template <int K, int CB, int MI>
 __device__ __forceinline__ void gemm_segment(const GemmShards& sa, const GemmPlan& plan, int M, int k,
                                              void* __restrict__ y, int y_bf16, int n_total, int rotate_out,
                                              uint8_t* lds, int item, int tile, int kt0, int kt1, int seg) {
-  constexpr int CHUNKS = gemm_chunks<K>();
-  static_assert(CHUNKS <= 64, "one gather per wave per k-step");
   constexpr int kRows = 16 * MI;
-  constexpr int kAStage = kRows * kBK * 2;
   constexpr int PIECES = (MI + kGemmWaves - 1) / kGemmWaves;  // A pieces (16 rows) a wave loads per k-step
-  uint8_t* a_ring = lds;                          // [kARing][MI row blocks][64 lanes][8 halves]
-  uint8_t* bits_ring = lds + kARing * kAStage;    // [kBitsRing][8 waves][64 lanes][16 B]
+  uint8_t* a_ring = lds;                            // [kARing][MI row blocks][64 lanes][8 halves]
+  uint8_t* bits_ring = lds + kARing * MI * 1024;    // [kBitsRing][8 waves][64 lanes][16 B]
 
   const int ct = tile % plan.nct, mblk = tile / plan.nct;
   int s = 0;
@@ -326,147 +293,39 @@ __device__ __forceinline__ void gemm_segment(const GemmShards& sa, const GemmPla
   const int row_bytes = tn * tile_bytes;
   const __amdgpu_buffer_rsrc_t brsrc =
       __builtin_amdgcn_make_buffer_rsrc((void*)sa.trellis[s], (short)0, (k >> 4) * row_bytes, 0x00020000);
-  // stage order [tile row][column][32K bytes].  STORED: the two columns are adjacent in their tile row; BLOCKS: the
-  // tiles of a column are adjacent, the columns 8 tiles apart inside the unit of the column block
+  // STORED: the two columns are adjacent in their tile row; BLOCKS: the tiles of a column are adjacent, the columns 8
+  // tiles apart inside the unit of the column block
   const bool blocks = sa.layout[s] == EXL3_LAYOUT_BLOCKS;
-  const int bL = l < CHUNKS ? l : CHUNKS - 1, brow = bL / (4 * K), bcol = bL % (4 * K) / (2 * K), bpiece = bL % (2 * K);
-  const int bj = tc0 + (mfma_wave ? 2 * w : 0) + bcol;
-  const int bgoff = (blocks ? ((bj >> 3) * (k >> 7) * 64 + (bj & 7) * 8 + brow) * tile_bytes
-                            : brow * row_bytes + bj * tile_bytes) + bpiece * 16;
-  const LaneGeo g = lane_geo<K>(c, j);
+  const BitsLane bl = bits_lane<K>(l);
+  const int bj = tc0 + (mfma_wave ? 2 * w : 0) + bl.col;
+  const int bgoff = (blocks ? ((bj >> 3) * (k >> 7) * 64 + (bj & 7) * 8 + bl.row) * tile_bytes
+                            : bl.row * row_bytes + bj * tile_bytes) + bl.piece * 16;
 
   // A: lane l of a piece = row (l % 16) of the row block, k-chunk l / 16.  Rows past M re-read row M-1 (finite, only
   // feeds discarded C rows).
-  const uint16_t* xh = sa.xh[s];
-  const __amdgpu_buffer_rsrc_t arsrc =
-      __builtin_amdgcn_make_buffer_rsrc((void*)xh, (short)0, M * k * 2, 0x00020000);
-  int aoff[PIECES], apiece[PIECES];
+  ActLoads<PIECES> act;
+  act.rsrc = __builtin_amdgcn_make_buffer_rsrc((void*)sa.xh[s], (short)0, M * k * 2, 0x00020000);
+  act.step = M * kBK * 2;
+  act.stage = MI * 1024;
 #pragma unroll
   for (int q = 0; q < PIECES; q++) {
-    const int p = PIECES * w + q;
-    apiece[q] = p < MI ? p : p % MI;  // fewer pieces than waves: the others load one again (the same bytes)
-    const int row = row0 + apiece[q] * 16 + c;
-    aoff[q] = ((row < M ? row : M - 1) * 32 + j * 8) * 2;  // + k-step * M * 64 bytes
+    const int p = PIECES * w + q, piece = p < MI ? p : p % MI;  // fewer pieces than waves: some are loaded twice
+    const int row = row0 + piece * 16 + c;
+    act.src[q] = ((row < M ? row : M - 1) * 32 + j * 8) * 2;
+    act.dst[q] = piece * 1024;
   }
 
-  // Loads come in bundles: bundle b = A of step b + trellis bits of step b + 1 (PIECES + 1 loads per wave; past the
-  // end, steps clamp to the last one: in range, never used), issued three steps ahead of the A's use and complete two
-  // steps later, one step before it: the barrier of step i publishes the A of step i + 1, so a wave reads its next
-  // fragments before the step's last MFMAs and no step starts with an LDS round trip.
   const int nk = kt1 - kt0;  // >= 1
-  // (the k-step argument kt is clamped by the caller: no device-only calls inside these lambdas, whose host-side
-  // instantiation would otherwise suppress the kernel's host stub)
-  auto issue_a = [&](int i, int kt) {
-    uint8_t* st = a_ring + (i & (kARing - 1)) * kAStage;
-#pragma unroll
-    for (int q = 0; q < PIECES; q++)
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(arsrc, (__attribute__((address_space(3))) void*)(st + apiece[q] * 1024),
-                                               16, aoff[q], kt * M * kBK * 2, 0, 0);
-  };
-  auto issue_bits = [&](int i, int kt) {
-    uint8_t* st = bits_ring + (i & (kBitsRing - 1)) * kBitsStage + w * 1024;
-    const int tr = 2 * kt;
-    __builtin_amdgcn_raw_ptr_buffer_load_lds(brsrc, (__attribute__((address_space(3))) void*)st, 16, bgoff,
-                                             blocks ? ((tr >> 3) * 64 + (tr & 7)) * tile_bytes : tr * row_bytes, 0,
-                                             0);
-  };
-  // this wave's trellis words of step i: [column][tile row][word]
-  auto read_bits = [&](int i, uint32_t (&bw)[2][2][2]) {
-    const uint32_t* tw = reinterpret_cast<const uint32_t*>(bits_ring + (i & (kBitsRing - 1)) * kBitsStage + w * 1024);
-#pragma unroll
-    for (int tr = 0; tr < 2; tr++)
-#pragma unroll
-      for (int jj = 0; jj < 2; jj++) {
-        bw[jj][tr][0] = tw[(tr * 2 + jj) * 8 * K + g.dw0];
-        bw[jj][tr][1] = tw[(tr * 2 + jj) * 8 * K + g.dw1];
-      }
-  };
-  auto frags = [&](int i) {
-    return reinterpret_cast<const half8_t*>(a_ring + (i & (kARing - 1)) * kAStage) + l;
-  };
-
-  // weights as the A operand, activations as B: a lane's accumulator holds 4 consecutive columns of one row,
-  // acc[mi][jj][r] = C[16 mi + l % 16][32 w + 16 jj + 4 (l / 16) + r]
   float4_t acc[MI][2];
 #pragma unroll
   for (int mi = 0; mi < MI; mi++)
 #pragma unroll
     for (int jj = 0; jj < 2; jj++) acc[mi][jj] = float4_t{0.f, 0.f, 0.f, 0.f};
 
-  auto last = [&](int i) { return kt0 + (i < nk ? i : nk - 1); };
-  issue_bits(0, kt0);
-#pragma unroll
-  for (int i = 0; i < 3; i++) {
-    issue_a(i, last(i));
-    issue_bits(i + 1, last(i + 1));
-  }
-  half8_t bcur[2], av[kWindow];
-  uint32_t bw[2][2][2];
-  __builtin_amdgcn_s_waitcnt(waitcnt_vm(2 * (PIECES + 1)));  // bundle 0 in (bundles 1 and 2 may be in flight)
-  lds_barrier();
-  read_bits(0, bw);
-#pragma unroll
-  for (int jj = 0; jj < 2; jj++)
-    bcur[jj] = decode_two_groups<K, CB>(bw[jj][0][0], bw[jj][0][1], bw[jj][1][0], bw[jj][1][1], g);
-  read_bits(1, bw);
-#pragma unroll
-  for (int q = 0; q < kWindow; q++) av[q] = frags(0)[q * 64];
-
-  auto steps = [&](auto multiply_first) {
-    constexpr bool MULTIPLY_FIRST = decltype(multiply_first)::value;
-    for (int i = 0; i < nk; i++) {
-      // bundle i + 1 in; bundle i + 2 may still be in flight.  The barrier publishes the A of step i + 1 and retires
-      // every read of step i - 1 (consumed by MFMAs issued before it), freeing its slot.
-      __builtin_amdgcn_sched_barrier(0);
-      __builtin_amdgcn_s_waitcnt(waitcnt_vm(PIECES + 1));
-      asm volatile("s_barrier" ::: "memory");
-      __builtin_amdgcn_sched_barrier(0);
-      issue_a(i + 3, last(i + 3));
-      issue_bits(i + 4, last(i + 4));
-      uint32_t bn[2][2][2];
-      read_bits(i + 2, bn);
-      const half8_t *af = frags(i), *an = frags(i + 1);
-      half8_t bnext[2];
-      auto decode = [&]() {
-#pragma unroll
-        for (int jj = 0; jj < 2; jj++)
-          bnext[jj] = decode_two_groups<K, CB>(bw[jj][0][0], bw[jj][0][1], bw[jj][1][0], bw[jj][1][1], g);
-      };
-      auto multiply = [&]() {
-#pragma unroll
-        for (int mi = 0; mi < MI; mi++) {
-          const half8_t a = av[mi % kWindow];
-          av[mi % kWindow] = mi + kWindow < MI ? af[(mi + kWindow) * 64] : an[(mi + kWindow - MI) * 64];
-#pragma unroll
-          for (int jj = 0; jj < 2; jj++)
-            acc[mi][jj] = __builtin_amdgcn_mfma_f32_16x16x32_f16(bcur[jj], a, acc[mi][jj], 0, 0, 0);
-        }
-      };
-      // the two waves of a SIMD (w and w + 4) take the step's halves in opposite order
-      if constexpr (MULTIPLY_FIRST) {
-        multiply();
-        decode();
-      } else {
-        decode();
-        multiply();
-      }
-#pragma unroll
-      for (int jj = 0; jj < 2; jj++) {
-        bcur[jj] = bnext[jj];
-#pragma unroll
-        for (int tr = 0; tr < 2; tr++) {
-          bw[jj][tr][0] = bn[jj][tr][0];
-          bw[jj][tr][1] = bn[jj][tr][1];
-        }
-      }
-    }
-  };
-  if (MI >= 8 && (w & 4))
-    steps(std::integral_constant<bool, (MI >= 8)>{});
-  else
-    steps(std::false_type{});
-  __builtin_amdgcn_s_waitcnt(waitcnt_vm(0));  // drain the trailing re-reads of every wave before LDS is reused
-  __syncthreads();
+  tile_multiply<K, CB, MI, PIECES>(
+      a_ring, act, 0, bits_ring + w * 1024, brsrc, bgoff,
+      [&](int kt) { return blocks ? ((kt >> 2) * 64 + (kt & 3) * 2) * tile_bytes : 2 * kt * row_bytes; }, kt0, nk,
+      (w & 4) != 0, l, acc);
 
   // ---- stream-K segment: store the partial (16-byte stores with device-scope coherence: the reader may sit on
   // another XCD, whose L2 is not this one's); the tile's last workgroup to arrive sums all of the tile's partials in
@@ -536,21 +395,9 @@ __device__ __forceinline__ void gemm_segment(const GemmShards& sa, const GemmPla
   // wave rotates its share of the (16-row, 128-column) blocks by MFMA and stores them (rotate_out), or stores the rows
   // as they are.
   _Float16* cl = reinterpret_cast<_Float16*>(lds);
-  if (mfma_wave) {
-#pragma unroll
-    for (int mi = 0; mi < MI; mi++)
-#pragma unroll
-      for (int jj = 0; jj < 2; jj++) {
-        const float4_t v = acc[mi][jj];
-        *reinterpret_cast<half4_t*>(cl + (mi * 16 + c) * kCStride + w * 32 + jj * 16 + 4 * j) =
-            half4_t{(_Float16)v.x, (_Float16)v.y, (_Float16)v.z, (_Float16)v.w};
-      }
-  }
+  if (mfma_wave) tile_to_lds<MI>(cl, acc, w, l);
   __syncthreads();
-  const half8_t f0 = had_frag(l);
-  half8_t f1 = f0;
-#pragma unroll
-  for (int e = 4; e < 8; e++) f1[e] = -f0[e];
+  const HadFrags had = had_frags_rows(l);
   for (int p = w; p < MI * 2; p += kGemmWaves) {
     const int mi = p >> 1, h = p & 1;
     const int m = row0 + mi * 16 + c;
@@ -564,22 +411,12 @@ __device__ __forceinline__ void gemm_segment(const GemmShards& sa, const GemmPla
     const half8_t* sv8 = reinterpret_cast<const half8_t*>(sa.svh[s] + (col - sa.col0[s]));
 #pragma unroll
     for (int u = 0; u < 4; u++) {
-      half8_t o;
+      half8_t o = cf[u];
       if (rotate_out) {
+        o = had_pair(had, cf, u);
         const half8_t sv = sv8[u * 4];
 #pragma unroll
-        for (int v = 0; v < 2; v++) {
-          float4_t d = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-          for (int kb = 0; kb < 4; kb++) {
-            const half8_t hf = v ? f1 : f0;
-            d = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_popcount(u & kb) & 1 ? -hf : hf, cf[kb], d, 0, 0, 0);
-          }
-#pragma unroll
-          for (int r = 0; r < 4; r++) o[4 * v + r] = had_scale_f16(d[r]) * sv[4 * v + r];
-        }
-      } else {
-        o = cf[u];
+        for (int e = 0; e < 8; e++) o[e] = o[e] * sv[e];
       }
       if (m < M) {
         if (y_bf16) {
@@ -784,7 +621,7 @@ static int launch_prefill(const void* x, bool x_bf16, int rows, int k, GemmShard
   const dim3 grid((unsigned)(L.groups + L.tiles - L.sk_tiles));
   bool ok;
 #define EXL3_GEMM_LAUNCH(MI_)                                                                                   \
-  ok = EXL3_GEMM_DISPATCH(K, codebook, gemm_kernel<kK, kCB, MI_><<<grid, kGemmThreads, gemm_lds(MI_), st>>>( \
+  ok = EXL3_GEMM_DISPATCH(K, codebook, gemm_kernel<kK, kCB, MI_><<<grid, kGemmThreads, tile_lds(MI_, MI_), st>>>( \
                                           sa, plan, rows, k, y, y_bf16 ? 1 : 0, n_total, ROT ? 1 : 0))
   if (L.mi == 4)
     EXL3_GEMM_LAUNCH(4);

@@ -34,6 +34,7 @@
 
 #include "exl3_api.hpp"
 #include "exl3_device.hpp"
+#include "exl3_moe_gemm.hpp"
 #include "exl3_stream.hpp"
 
 namespace exl3 {
@@ -598,16 +599,47 @@ struct MoePlan {
   bool slot_mode;  // a single token: grid rows = its slots, no routing or prep launches
   int groups;      // P: 16-slot groups per pass over an expert's weights (1, 2 or 4)
   int nt;          // tile rows per chunk
+  int tile_rows;   // > 0: the expert decode-GEMMs (exl3_moe_gemm.hip) in tiles of 64 or 128 slots instead of the GEMVs
   MoePhase gu, dn;
-  size_t off_counts, off_nactive, off_active, off_lists, off_gu, off_dn, off_cnt_gu, off_cnt_dn, off_pre_in,
+  size_t off_sorted, off_totals, off_tiles, off_counts, off_nactive, off_active, off_lists, off_gu, off_dn, off_cnt_gu, off_cnt_dn, off_pre_in,
       off_pre_dn, off_partial, total;
 };
 
 static size_t align256(size_t v) { return (v + 255) & ~(size_t)255; }
 
+// Whether a call takes the expert decode-GEMMs (exl3_moe_gemm.hip), and their tile height in slots; 0: the expert GEMVs.
+// The lower of two estimates (us), fitted at 8-128 experts, hidden 1024-4096, inter 512-1536 and 2-128 slots per expert:
+//   GEMVs: the experts' weights once per 16-64 slots (per 4.72 M weights, 128 experts at 2048 / 768 measured 111 us at 4
+//   slots per expert, 165 at 10, 230 at 16, 458 at 32, 1247 at 128), at least 2.4 us per slot of an expert (few experts);
+//   GEMMs: a tile per expert and column block, so at least one tile's k-steps per phase (the same layer 135-140 us up to
+//   10 slots per expert, 176 at 16, 189 at 32, 409 at 128; 8 experts at 4096 / 1536 about 103 us up to 64).
+// Tiles of 128 slots from 128 per expert (16 experts at 250: 70.8 us against 79.5 with tiles of 64; at 62: 58 against 50).
+static int moe_tile_rows(int slots, int E, int H, int I) {
+  const int active = std::min(E, slots);
+  const double mean = (double)slots / active, units = active * (3.0 * H * I / 4718592);
+  const double gemv = 22 + std::max(units * (0.5 + 0.06 * mean), 2.4 * mean);
+  const int rows = mean >= 128 ? 128 : 64;
+  const double tiles = active * std::ceil(mean / rows);
+  auto phase = [&](int ksteps, int ncb) { return ksteps * 0.48 * std::max(1.0, tiles * ncb / 256); };
+  const double gemm = 19 + phase(H / 32, I / 128) + phase(I / 32, (H + 255) / 256);
+  return gemm < gemv ? rows : 0;
+}
+
 static MoePlan moe_plan(int tokens, int top_k, int E, int H, int I, int K_gu, int K_dn) {
   MoePlan p{};
   const int slots = tokens * top_k;
+  p.tile_rows = moe_tile_rows(slots, E, H, I);
+  if (p.tile_rows > 0) {
+    size_t o = kCounterBytes;  // unused here, but every workspace starts with it
+    p.off_sorted = o; o = align256(o + (size_t)slots * sizeof(int2));
+    p.off_totals = o; o = align256(o + 8);
+    p.off_tiles = o; o = align256(o + (size_t)moe_gemm_max_tiles(slots, E, p.tile_rows) * sizeof(MoeTile));
+    p.off_dn = o; o = align256(o + (size_t)slots * H * 2);
+    p.off_pre_in = o; o = align256(o + (size_t)2 * slots * H * 2);
+    p.off_pre_dn = o; o = align256(o + (size_t)slots * I * 2);
+    p.total = o;
+    return p;
+  }
   p.slot_mode = tokens == 1 && slots <= E;
   const int rows = p.slot_mode ? slots : std::max(1, std::min(E, slots));
   p.nt = 16;  // 32 measured slower with 256 tokens, equal with 16
@@ -694,6 +726,14 @@ static bool moe_shape_ok(int tokens, int top_k, int E, int H, int I) {
   return tokens > 0 && top_k > 0 && E > 0 && H > 0 && I > 0 && (int64_t)E * (2 * I + H) / 128 <= kMaxCounters;
 }
 
+static void launch_combine(const uint16_t* dn, const void* topk_ids, const void* topk_weights, int tokens, int top_k,
+                           int num_experts, int hidden, void* y, int y_bf16, hipStream_t st) {
+  const dim3 grid((unsigned)(((size_t)tokens * (hidden / 128) + 7) / 8));
+  auto combine = y_bf16 ? moe_combine_kernel<true> : moe_combine_kernel<false>;
+  combine<<<grid, 256, 0, st>>>(dn, static_cast<const int*>(topk_ids), static_cast<const float*>(topk_weights), tokens,
+                                top_k, num_experts, hidden, y);
+}
+
 static int moe_forward_impl(const char* what, const void* x, int x_bf16, int tokens, int hidden, const void* topk_ids,
                             const void* topk_weights, int top_k, int num_experts, int inter, const MoeClass* cls,
                             int ncls, int codebook, void* y, int y_bf16, void* workspace, size_t workspace_bytes,
@@ -728,6 +768,43 @@ static int moe_forward_impl(const char* what, const void* x, int x_bf16, int tok
   EXL3_CHECK_ARG(workspace && workspace_bytes >= p.total, "%s: workspace %zu bytes, need %zu", what, workspace_bytes,
                  p.total);
   uint8_t* ws = static_cast<uint8_t*>(workspace);
+  if (p.tile_rows > 0) {
+    MoeGemmArgs g{};
+    g.E = num_experts;
+    g.H = hidden;
+    g.I = inter;
+    g.top_k = top_k;
+    g.slots = slots;
+    g.tile_rows = p.tile_rows;
+    g.topk_ids = static_cast<const int*>(topk_ids);
+    g.sorted = reinterpret_cast<int2*>(ws + p.off_sorted);
+    g.totals = reinterpret_cast<int*>(ws + p.off_totals);
+    g.tiles = reinterpret_cast<MoeTile*>(ws + p.off_tiles);
+    g.pre_in = reinterpret_cast<uint16_t*>(ws + p.off_pre_in);
+    g.pre_dn = reinterpret_cast<uint16_t*>(ws + p.off_pre_dn);
+    g.dn = reinterpret_cast<uint16_t*>(ws + p.off_dn);
+    if (int rc = moe_gemm_route(g, st)) return rc;
+    for (int c = 0; c < ncls; c++) {
+      const exl3_moe_weights* w = cls[c].w;
+      g.tr[0] = static_cast<const uint32_t*>(w->gate_trellis);
+      g.tr[1] = static_cast<const uint32_t*>(w->up_trellis);
+      g.tr[2] = static_cast<const uint32_t*>(w->down_trellis);
+      g.suh[0] = static_cast<const uint16_t*>(w->gate_suh);
+      g.suh[1] = static_cast<const uint16_t*>(w->up_suh);
+      g.suh[2] = static_cast<const uint16_t*>(w->down_suh);
+      g.svh[0] = static_cast<const uint16_t*>(w->gate_svh);
+      g.svh[1] = static_cast<const uint16_t*>(w->up_svh);
+      g.svh[2] = static_cast<const uint16_t*>(w->down_svh);
+      g.emap = cls[c].emap;
+      g.E_local = cls[c].E_local;
+      if (int rc = moe_gemm_inputs(g, x, x_bf16 != 0, st)) return rc;
+      if (int rc = moe_gemm_gate_up(g, cls[c].K_gu, codebook, st)) return rc;
+      if (int rc = moe_gemm_down(g, cls[c].K_dn, codebook, st)) return rc;
+    }
+    launch_combine(g.dn, topk_ids, topk_weights, tokens, top_k, num_experts, hidden, y, y_bf16, st);
+    EXL3_CHECK_LAUNCH();
+    return EXL3_OK;
+  }
   MoeArgs a{};
   a.E = num_experts;
   a.H = hidden;
@@ -801,15 +878,7 @@ static int moe_forward_impl(const char* what, const void* x, int x_bf16, int tok
     if (!ok) return set_error(EXL3_ERR_INVALID, "%s: unsupported K/codebook", what);
     EXL3_CHECK_LAUNCH();
   }
-  const dim3 cgrid((unsigned)(((size_t)tokens * (hidden / 128) + 7) / 8));
-  if (y_bf16)
-    moe_combine_kernel<true><<<cgrid, 256, 0, st>>>(dn, static_cast<const int*>(topk_ids),
-                                                    static_cast<const float*>(topk_weights), tokens, top_k,
-                                                    num_experts, hidden, y);
-  else
-    moe_combine_kernel<false><<<cgrid, 256, 0, st>>>(dn, static_cast<const int*>(topk_ids),
-                                                     static_cast<const float*>(topk_weights), tokens, top_k,
-                                                     num_experts, hidden, y);
+  launch_combine(dn, topk_ids, topk_weights, tokens, top_k, num_experts, hidden, y, y_bf16, st);
   EXL3_CHECK_LAUNCH();
   return EXL3_OK;
 }
@@ -868,14 +937,8 @@ extern "C" int exl3_moe_combine(const void* yd, const float* topk_weights, const
                  num_experts);
   EXL3_CHECK_ARG((int64_t)tokens * top_k * hidden <= INT32_MAX, "exl3_moe_combine: too many rows");
   if (tokens == 0) return EXL3_OK;
-  const dim3 grid((unsigned)(((size_t)tokens * (hidden / 128) + 7) / 8));
-  hipStream_t st = as_stream(stream);
-  if (y_bf16)
-    moe_combine_kernel<true><<<grid, 256, 0, st>>>(static_cast<const uint16_t*>(yd), topk_ids, topk_weights, tokens,
-                                                   top_k, num_experts, hidden, y);
-  else
-    moe_combine_kernel<false><<<grid, 256, 0, st>>>(static_cast<const uint16_t*>(yd), topk_ids, topk_weights, tokens,
-                                                    top_k, num_experts, hidden, y);
+  launch_combine(static_cast<const uint16_t*>(yd), topk_ids, topk_weights, tokens, top_k, num_experts, hidden, y, y_bf16,
+                 as_stream(stream));
   EXL3_CHECK_LAUNCH();
   return EXL3_OK;
 }
