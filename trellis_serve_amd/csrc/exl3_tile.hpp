@@ -103,7 +103,7 @@ __device__ __forceinline__ void tile_multiply(uint8_t* a_ring, const ActLoads<PI
     issue_a(i, last(i));
     issue_bits(i + 1, last(i + 1));
   }
-  half8_t bcur[2], av[kWindow];
+  half8_t bcur[2], bnext[2], av[kWindow];
   uint32_t bw[2][2][2];
   __builtin_amdgcn_s_waitcnt(waitcnt_vm(2 * (PIECES + 1)));  // bundle 0 in (bundles 1 and 2 may be in flight)
   lds_barrier();
@@ -115,54 +115,50 @@ __device__ __forceinline__ void tile_multiply(uint8_t* a_ring, const ActLoads<PI
 #pragma unroll
   for (int q = 0; q < kWindow; q++) av[q] = frags(0)[q * 64];
 
-  auto steps = [&](auto multiply_first) {
-    constexpr bool MULTIPLY_FIRST = decltype(multiply_first)::value;
-    for (int i = 0; i < nk; i++) {
-      // bundle i + 1 in; bundle i + 2 may still be in flight.  The barrier publishes the A of step i + 1 and retires
-      // every read of step i - 1 (consumed by MFMAs issued before it), freeing its slot.
-      __builtin_amdgcn_sched_barrier(0);
-      __builtin_amdgcn_s_waitcnt(waitcnt_vm(PIECES + 1));
-      asm volatile("s_barrier" ::: "memory");
-      __builtin_amdgcn_sched_barrier(0);
-      issue_a(i + 3, last(i + 3));
-      issue_bits(i + 4, last(i + 4));
-      uint32_t bn[2][2][2];
-      read_bits(i + 2, bn);
-      const half8_t *af = frags(i), *an = frags(i + 1);
-      half8_t bnext[2];
-      auto decode = [&]() {
+  // step i: the weights `cur` of the step, `next` those of step i + 1, decoded here from the words in bw, which then
+  // take step i + 2's
+  auto step = [&](auto multiply_first, int i, const half8_t (&cur)[2], half8_t (&next)[2]) {
+    // bundle i + 1 in; bundle i + 2 may still be in flight.  The barrier publishes the A of step i + 1 and retires
+    // every read of step i - 1 (consumed by MFMAs issued before it), freeing its slot.
+    __builtin_amdgcn_sched_barrier(0);
+    __builtin_amdgcn_s_waitcnt(waitcnt_vm(PIECES + 1));
+    asm volatile("s_barrier" ::: "memory");
+    __builtin_amdgcn_sched_barrier(0);
+    issue_a(i + 3, last(i + 3));
+    issue_bits(i + 4, last(i + 4));
+    const half8_t *af = frags(i), *an = frags(i + 1);
+    auto decode = [&]() {
+#pragma unroll
+      for (int jj = 0; jj < 2; jj++)
+        next[jj] = decode_two_groups<K, CB>(bw[jj][0][0], bw[jj][0][1], bw[jj][1][0], bw[jj][1][1], g);
+      read_bits(i + 2, bw);
+    };
+    auto multiply = [&]() {
+#pragma unroll
+      for (int mi = 0; mi < MI; mi++) {
+        const half8_t a = av[mi % kWindow];
+        av[mi % kWindow] = mi + kWindow < MI ? af[(mi + kWindow) * 64] : an[(mi + kWindow - MI) * 64];
 #pragma unroll
         for (int jj = 0; jj < 2; jj++)
-          bnext[jj] = decode_two_groups<K, CB>(bw[jj][0][0], bw[jj][0][1], bw[jj][1][0], bw[jj][1][1], g);
-      };
-      auto multiply = [&]() {
-#pragma unroll
-        for (int mi = 0; mi < MI; mi++) {
-          const half8_t a = av[mi % kWindow];
-          av[mi % kWindow] = mi + kWindow < MI ? af[(mi + kWindow) * 64] : an[(mi + kWindow - MI) * 64];
-#pragma unroll
-          for (int jj = 0; jj < 2; jj++)
-            acc[mi][jj] = __builtin_amdgcn_mfma_f32_16x16x32_f16(bcur[jj], a, acc[mi][jj], 0, 0, 0);
-        }
-      };
-      // the two waves of a SIMD (w and w + 4) take the step's halves in opposite order
-      if constexpr (MULTIPLY_FIRST) {
-        multiply();
-        decode();
-      } else {
-        decode();
-        multiply();
+          acc[mi][jj] = __builtin_amdgcn_mfma_f32_16x16x32_f16(cur[jj], a, acc[mi][jj], 0, 0, 0);
       }
-#pragma unroll
-      for (int jj = 0; jj < 2; jj++) {
-        bcur[jj] = bnext[jj];
-#pragma unroll
-        for (int tr = 0; tr < 2; tr++) {
-          bw[jj][tr][0] = bn[jj][tr][0];
-          bw[jj][tr][1] = bn[jj][tr][1];
-        }
-      }
+    };
+    // the two waves of a SIMD (w and w + 4) take the step's halves in opposite order
+    if constexpr (decltype(multiply_first)::value) {
+      multiply();
+      decode();
+    } else {
+      decode();
+      multiply();
     }
+  };
+  auto steps = [&](auto multiply_first) {  // in pairs, so that the weights change registers without copies
+    int i = 0;
+    for (; i + 2 <= nk; i += 2) {
+      step(multiply_first, i, bcur, bnext);
+      step(multiply_first, i + 1, bnext, bcur);
+    }
+    if (i < nk) step(multiply_first, i, bcur, bnext);
   };
   if (MI >= 8 && multiply_first)
     steps(std::integral_constant<bool, (MI >= 8)>{});
