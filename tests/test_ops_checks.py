@@ -59,3 +59,32 @@ def test_ops_reject_bad_out_and_routing_before_launching():
         ops.moe_forward(xm, ids[:2], w[:2], experts, 1)                  # fewer routing rows than tokens
     with pytest.raises(ValueError):
         ops.moe_forward(xm, ids, w, experts, 1, out=torch.empty((3, H), dtype=torch.float32, device="cuda"))
+
+
+@pytest.mark.gpu
+def test_linear_takes_every_form_of_its_rows():
+    """The rows of x as one 2-D tensor, as a strided view, with more and with fewer dimensions, in fp32 and empty, give
+    the same results in x's shape and dtype; tensors off the GPU are refused before anything is launched."""
+    from trellis_serve_amd.runtime import ops as runtime_ops
+    trs, suhs, svhs = _group(256, [128, 256])
+    g = torch.Generator().manual_seed(4)
+    for fn, rows in ((ops.linear, 6), (ops.linear_prefill, 6), (runtime_ops.linear, 6), (runtime_ops.linear, 90)):
+        x = torch.randn((rows, 256), generator=g).half().cuda()
+        y = fn(x, trs, suhs, svhs, 1)
+        assert y.shape == (rows, 384) and y.dtype == torch.float16
+        wide = torch.zeros((rows, 512), dtype=torch.float16, device="cuda")
+        wide[:, :256] = x
+        assert torch.equal(fn(wide[:, :256], trs, suhs, svhs, 1), y)
+        assert torch.equal(fn(x.view(2, rows // 2, 256), trs, suhs, svhs, 1), y.view(2, rows // 2, 384))
+        one = fn(x[0], trs, suhs, svhs, 1)
+        assert one.shape == (384,) and torch.equal(one, fn(x[:1], trs, suhs, svhs, 1)[0])
+        assert fn(x[:0], trs, suhs, svhs, 1).shape == (0, 384)
+        if fn is runtime_ops.linear:
+            y32 = fn(x.float().view(1, rows, 256), trs, suhs, svhs, 1)
+            assert y32.dtype == torch.float32 and torch.equal(y32, y.float().view(1, rows, 384))
+        else:
+            with pytest.raises(ValueError):
+                fn(x.cpu(), trs, suhs, svhs, 1)
+    with pytest.raises(ValueError):
+        ops.had_in_group(torch.ones((1, 256), dtype=torch.float16), torch.ones(256, dtype=torch.float16, device="cuda"),
+                         torch.empty((1, 256), dtype=torch.float16, device="cuda"))

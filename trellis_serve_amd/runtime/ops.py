@@ -25,14 +25,11 @@ _lib = torch.library.Library("exl3_mi355x", "FRAGMENT")  # must stay alive at mo
 
 def _linear(x: torch.Tensor, trellis: list[torch.Tensor], suh: list[torch.Tensor], svh: list[torch.Tensor],
             codebook: int) -> torch.Tensor:
-    rows = x.reshape(-1, x.shape[-1])
-    n_total = sum(t.shape[1] * 16 for t in trellis)
-    if rows.dtype not in (torch.float16, torch.bfloat16):   # an fp32 caller: explicit cast, as the reference does
-        y = _linear(rows.to(torch.float16), trellis, suh, svh, codebook)
-        return y.to(x.dtype).view(*x.shape[:-1], n_total)
-    fn = _kernels.linear_prefill if rows.shape[0] >= PREFILL_ROWS else _kernels.linear
-    y = fn(rows.contiguous(), trellis, suh, svh, codebook)
-    return y.view(*x.shape[:-1], n_total)
+    if x.dtype not in (torch.float16, torch.bfloat16):   # an fp32 caller: explicit cast, as the reference does
+        return _linear(x.to(torch.float16), trellis, suh, svh, codebook).to(x.dtype)
+    rows = x.shape[0] if x.dim() == 2 else x.reshape(-1, x.shape[-1]).shape[0]
+    fn = _kernels.linear_prefill if rows >= PREFILL_ROWS else _kernels.linear
+    return fn(x, trellis, suh, svh, codebook)   # [..., sum n_s]
 
 
 def _linear_fake(x, trellis, suh, svh, codebook):
