@@ -8,7 +8,7 @@
 //   A: xh in "fragment order", k-step major: the rotated activations with k permuted inside every 32-wide block so
 //      that the 8 halves one MFMA lane needs are contiguous, and the blocks of one k-step stored together:
 //      xh_f[b][m][8q + 4tr + e] = xh[m][32b + 16tr + r(q, e)], r(q, e) = 2q + (e & 1) + 8(e >> 1) (written by
-//      had_in_frag_kernel).  One k-step of 256 rows is one contiguous 16 KB run: the GEMM's loads use whole lines.
+//      rotate_rows_kernel).  One k-step of 256 rows is one contiguous 16 KB run: the GEMM's loads use whole lines.
 //   B: the trellis.  A k-step covers 32 rows = 2 tile rows.  The lane-geometry decode of exl3_device.hpp gives lane
 //      (c, j) of a tile the 4 weights of column c at rows r(j, 0..3); tile row tr of the k-step supplies halves
 //      4tr..4tr+3 of the lane's 8-half B fragment.  A and B then agree on the k order of every MFMA.
@@ -51,8 +51,6 @@
 
 namespace exl3 {
 
-typedef _Float16 half8_t __attribute__((ext_vector_type(8)));
-typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
 
 constexpr int kCoherentStore = 1 << 4;             // buffer cache policy sc1: device-scope coherent access
 constexpr int kPastEnd = 0x7FFFFFF0;               // a buffer offset past every partial
@@ -102,159 +100,47 @@ __device__ __forceinline__ const uint16_t* unit_suh(const ShardSuh& su_all, int 
   return s == 0 ? su_all.suh[0] : s == 1 ? su_all.suh[1] : s == 2 ? su_all.suh[2] : su_all.suh[3];
 }
 
-// The 8 values of a 16-lane unit's lane (positions 8t .. 8t+7) as 4 fp16 pairs: fp16(Had(fp16(x) * suh)) (ROT), or
-// x as given (fp16 rows)
+// The activations of every shard in fragment order, k-step major (see the header comment): xh_f[s][kt][row][32].  One
+// wave per (16 rows, 128-block): it loads the block once as MFMA fragments and, per shard, multiplies by suh (fp16
+// product), rotates by MFMA and stores whole fragments, 1 KB per k-step.  The butterfly on 16 lanes per row that this
+// replaces took 130 VALU instructions and 8-byte stores per row and block: 4096 rows, 2 shards of k = 5120 49 us against
+// 28 (126 MB; at a large copy's rate 25).  ROT = false: the fp16 rows as given, only put in fragment order (the
+// rotation-free GEMM of exl3_gemm_rotated).  gridDim.z: shards over workgroups (few rows), else all in one wave.
 template <bool X_BF16, bool ROT>
-__device__ __forceinline__ void frag16_values(u32x4_t xv, u32x4_t sv, uint32_t d[4]) {
+__global__ __launch_bounds__(256) void rotate_rows_kernel(const uint16_t* __restrict__ x, int rows, int k,
+                                                          ShardSuh su_all, int shards, uint16_t* __restrict__ xh) {
+  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), l = threadIdx.x & 63, c = l & 15, j = l >> 4;
+  const int row0 = (blockIdx.x * 4 + w) * 16, b = blockIdx.y;
+  if (row0 >= rows) return;  // wave-uniform
+  const int row = row0 + c, from = row < rows ? row : rows - 1;
+  uint16_t* dst = xh + ((size_t)(b * 4) * rows + row) * 32 + 8 * j;
   if constexpr (!ROT) {
+    // slot 8 j + 4 tr + e of a 32-block holds position 16 tr + 2 j + (e & 1) + 8 (e >> 1)
+    const uint16_t* xr = x + (size_t)from * k + b * 128 + 2 * j;
+    u32x4 v[4];
 #pragma unroll
-    for (int q = 0; q < 4; q++) d[q] = xv[q];
-    return;
-  }
-  const half8_t sc = __builtin_bit_cast(half8_t, sv);
-  float f[8];
+    for (int u = 0; u < 4; u++)
 #pragma unroll
-  for (int i = 0; i < 8; i++) {
-    const uint32_t w = xv[i >> 1];
-    const uint16_t raw = (uint16_t)((i & 1) ? w >> 16 : w & 0xFFFF);
-    const _Float16 v = X_BF16 ? (_Float16)bf16_to_f32(raw) : __builtin_bit_cast(_Float16, raw);
-    f[i] = (float)(_Float16)(v * sc[i]);
-  }
+      for (int q = 0; q < 4; q++) v[u][q] = *reinterpret_cast<const uint32_t*>(xr + 32 * u + 8 * q);
 #pragma unroll
-  for (int h = 1; h < 8; h <<= 1)
-#pragma unroll
-    for (int i = 0; i < 8; i++)
-      if (!(i & h)) {
-        const float a = f[i], bb = f[i + h];
-        f[i] = a + bb;
-        f[i + h] = a - bb;
-      }
-  had_stage<1>(f[0], f[1], f[2], f[3]);
-  had_stage<1>(f[4], f[5], f[6], f[7]);
-  had_stage<2>(f[0], f[1], f[2], f[3]);
-  had_stage<2>(f[4], f[5], f[6], f[7]);
-  had_stage<4>(f[0], f[1], f[2], f[3]);
-  had_stage<4>(f[4], f[5], f[6], f[7]);
-  had_stage<8>(f[0], f[1], f[2], f[3]);
-  had_stage<8>(f[4], f[5], f[6], f[7]);
-#pragma unroll
-  for (int q = 0; q < 4; q++)
-    d[q] = __builtin_bit_cast(uint32_t, half2_t{had_scale_f16(f[2 * q]), had_scale_f16(f[2 * q + 1])});
-}
-
-// The same rotation with 16 lanes per 128-value (row, block) unit: lane t holds positions 8t .. 8t+7, read with one
-// 16-byte load of x and one of suh (x and every suh 16-byte aligned; the host checks).  The butterfly runs the stages
-// of had128_x4 in the same order on the same pairs -- h = 1, 2, 4 inside the lane (h = 4 was the lane-xor-1 stage
-// of the 4-per-lane form: lower = a + b, upper = a - b, the same sums), then lane xor 1, 2, 4, 8 for h = 8 .. 64 --
-// so the rotated values are bit-identical.  Fragment order: lane t (a = t & 3) holds, per q = 0..3, the slot pair
-// (q, tr = a >> 1, e = 2 (a & 1) + 0/1); lanes a and a ^ 1 swap two dwords (DPP) so that each stores two 8-byte
-// slot groups (q, tr) whole.  A 16-lane group takes U consecutive units with all loads issued first.
-// ROT = false: the fp16 rows are taken as given (no sign vector, no butterfly, no rounding) and only put in fragment
-// order (the rotation-free GEMM of exl3_gemm_rotated).
-template <bool X_BF16, int U, bool ROT = true>
-__global__ __launch_bounds__(256) void had_in_frag16_kernel(const void* __restrict__ x, int rows, int k,
-                                                            ShardSuh su_all, int shards, uint16_t* __restrict__ xh) {
-  const int kb = k >> 7;
-  const int units = shards * rows * kb;
-  const int u0 = (blockIdx.x * 16 + (threadIdx.x >> 4)) * U;
-  if (u0 >= units) return;  // the whole 16-lane row: the DPP stages below stay inside rows of 16 lanes
-  const int t = threadIdx.x & 15;
-  u32x4_t xv[U], sv[U];
-#pragma unroll
-  for (int j = 0; j < U; j++) {
-    const int u = min(u0 + j, units - 1);  // past the end: a repeat of the last unit, not stored
-    const int s = u / (rows * kb), rem = u - s * rows * kb, r = rem / kb, b = rem - r * kb;
-    const int kk = b * 128 + 8 * t;
-    xv[j] = *reinterpret_cast<const u32x4_t*>(static_cast<const uint16_t*>(x) + (size_t)r * k + kk);
-    sv[j] = ROT ? *reinterpret_cast<const u32x4_t*>(unit_suh(su_all, s) + kk) : u32x4_t{0u, 0u, 0u, 0u};
-  }
-#pragma unroll
-  for (int j = 0; j < U; j++) {
-    const int u = u0 + j;
-    if (u >= units) break;
-    const int s = u / (rows * kb), rem = u - s * rows * kb, r = rem / kb, b = rem - r * kb;
-    uint32_t d[4];  // d[q] = fp16 pair (positions 2q, 2q+1 of the lane)
-    frag16_values<X_BF16, ROT>(xv[j], sv[j], d);
-    const bool low = (t & 1) == 0;
-    // lane a (even) stores q = 0, 2 as [own, partner's]; lane a + 1 stores q = 1, 3 as [partner's, own]
-    const uint32_t g0 = (uint32_t)__builtin_amdgcn_mov_dpp((int)(low ? d[1] : d[0]), 0xB1, 0xF, 0xF, false);
-    const uint32_t g1 = (uint32_t)__builtin_amdgcn_mov_dpp((int)(low ? d[3] : d[2]), 0xB1, 0xF, 0xF, false);
-    const uint2_t o0 = low ? uint2_t{d[0], g0} : uint2_t{g0, d[1]};
-    const uint2_t o1 = low ? uint2_t{d[2], g1} : uint2_t{g1, d[3]};
-    const int a = t & 3, blk32 = t >> 2, tr = a >> 1, q0 = low ? 0 : 1;
-    uint16_t* dst = xh + (size_t)s * rows * k + ((size_t)(b * 4 + blk32) * rows + r) * 32 + tr * 4;
-    *reinterpret_cast<uint2_t*>(dst + q0 * 8) = o0;
-    *reinterpret_cast<uint2_t*>(dst + (q0 + 2) * 8) = o1;
-  }
-}
-
-// The 4 values of a 32-lane unit's lane (positions 4t .. 4t+3) as 2 fp16 pairs: fp16(Had(fp16(x) * suh)) (ROT), or
-// x as given (fp16 rows)
-template <bool X_BF16, bool ROT>
-__device__ __forceinline__ void frag_values(uint2_t xv, uint2_t sv, uint32_t& lo_w, uint32_t& hi_w) {
-  if constexpr (!ROT) {
-    lo_w = xv.x;
-    hi_w = xv.y;
-    return;
-  }
-  _Float16 v[4];
-  if constexpr (X_BF16) {
-    v[0] = (_Float16)bf16_to_f32((uint16_t)(xv.x & 0xFFFF));
-    v[1] = (_Float16)bf16_to_f32((uint16_t)(xv.x >> 16));
-    v[2] = (_Float16)bf16_to_f32((uint16_t)(xv.y & 0xFFFF));
-    v[3] = (_Float16)bf16_to_f32((uint16_t)(xv.y >> 16));
+    for (int u = 0; u < 4; u++)
+      if (row < rows) *reinterpret_cast<u32x4*>(dst + (size_t)u * rows * 32) = v[u];
   } else {
-    const half4_t raw = __builtin_bit_cast(half4_t, xv);
-    v[0] = raw.x; v[1] = raw.y; v[2] = raw.z; v[3] = raw.w;
-  }
-  const half4_t sc = __builtin_bit_cast(half4_t, sv);
-  float f0 = (float)(_Float16)(v[0] * sc.x), f1 = (float)(_Float16)(v[1] * sc.y);
-  float f2 = (float)(_Float16)(v[2] * sc.z), f3 = (float)(_Float16)(v[3] * sc.w);
-  had128_x4(f0, f1, f2, f3);
-  lo_w = __builtin_bit_cast(uint32_t, half2_t{had_scale_f16(f0), had_scale_f16(f1)});
-  hi_w = __builtin_bit_cast(uint32_t, half2_t{had_scale_f16(f2), had_scale_f16(f3)});
-}
-
-// rotated activations in fragment order: xh_f[s*rows + r][k] for shard s (see the header comment).  A half-wave
-// takes U consecutive 128-value (row, block) units, issues all their loads first (one round of load latency per
-// half-wave instead of one per unit), then rotates and stores each; lane t holds positions 4t .. 4t+3 of a block.
-// U = 4 from 2^17 units (measured at 8192 rows: 60 -> 52 us; equal at 2048 rows, slower at 512 rows).
-template <bool X_BF16, int U, bool ROT = true>
-__global__ __launch_bounds__(256) void had_in_frag_kernel(const void* __restrict__ x, int rows, int k, ShardSuh su_all,
-                                                          int shards, uint16_t* __restrict__ xh) {
-  const int kb = k >> 7;
-  const int units = shards * rows * kb;
-  const int u0 = (blockIdx.x * 8 + (threadIdx.x >> 5)) * U;
-  if (u0 >= units) return;
-  const int t = threadIdx.x & 31;
-  uint2_t xv[U], sv[U];
+    half8_t xv[4];
+    load_row_frags<X_BF16>(x + (size_t)from * k + b * 128 + 8 * j, xv);
+    const HadFrags had = had_frags_act(l);
+    const int s0 = gridDim.z > 1 ? blockIdx.z : 0, s1 = gridDim.z > 1 ? s0 + 1 : shards;
+    for (int s = s0; s < s1; s++) {
+      const uint16_t* suh = unit_suh(su_all, s) + b * 128 + 8 * j;
+      half8_t in[4];
 #pragma unroll
-  for (int j = 0; j < U; j++) {
-    const int u = min(u0 + j, units - 1);  // past the end: a repeat of the last unit, not stored
-    const int s = u / (rows * kb), rem = u - s * rows * kb, r = rem / kb, b = rem - r * kb;
-    const int kk = b * 128 + 4 * t;
-    xv[j] = *reinterpret_cast<const uint2_t*>(static_cast<const uint16_t*>(x) + (size_t)r * k + kk);
-    sv[j] = ROT ? *reinterpret_cast<const uint2_t*>(unit_suh(su_all, s) + kk) : uint2_t{0u, 0u};
-  }
+      for (int kb = 0; kb < 4; kb++) in[kb] = times8(xv[kb], suh + 32 * kb);
 #pragma unroll
-  for (int j = 0; j < U; j++) {
-    const int u = u0 + j;
-    if (u >= units) break;
-    const int s = u / (rows * kb), rem = u - s * rows * kb, r = rem / kb, b = rem - r * kb;
-    uint32_t lo_w, hi_w;  // fp16 pairs: positions 4t, 4t+1 and 4t+2, 4t+3
-    frag_values<X_BF16, ROT>(xv[j], sv[j], lo_w, hi_w);
-    // k-step major: the 32 halves of row r in k-step kt (one MFMA k-block) at [kt][r][32], so that one k-step of a
-    // row block is one contiguous run and every 16-row A piece of the GEMM reads whole cache lines.  Inside a
-    // 32-block, slot (q, tr, e) holds position 16 tr + 2q + (e & 1) + 8 (e >> 1).  With a = t & 3, lane t's positions
-    // are 16 tr + 4a + i: lanes a < 2 hold e = 0, 1 of q = 2a (i < 2) and of q = 2a + 1 (i >= 2), lanes a + 2 the
-    // e = 2, 3 of the same q.  The pair (a, a + 2) swaps one dword (a DPP quad permute) and each lane stores its q's
-    // 4 slots as one 8-byte word.
-    const bool low = (t & 2) == 0;
-    const uint32_t got = (uint32_t)__builtin_amdgcn_mov_dpp((int)(low ? hi_w : lo_w), 0x4E, 0xF, 0xF, false);
-    const uint2_t out = low ? uint2_t{lo_w, got} : uint2_t{got, hi_w};
-    const int blk32 = t >> 3, tr = (t >> 2) & 1, q = 2 * (t & 1) + (low ? 0 : 1);
-    uint16_t* dst = xh + (size_t)s * rows * k;
-    *reinterpret_cast<uint2_t*>(dst + ((size_t)(b * 4 + blk32) * rows + r) * 32 + q * 8 + tr * 4) = out;
+      for (int u = 0; u < 4; u++) {
+        const half8_t o = had_pair(had, in, u);
+        if (row < rows) *reinterpret_cast<half8_t*>(dst + (size_t)s * rows * k + (size_t)u * rows * 32) = o;
+      }
+    }
   }
 }
 
@@ -598,25 +484,12 @@ static int launch_prefill(const void* x, bool x_bf16, int rows, int k, GemmShard
   int n_total = 0;
   for (int s = 0; s < nshards; s++) n_total += shard_n[s];
   // the input pass: every shard in one launch
-  const size_t hunits = (size_t)nshards * rows * (k / 128);
-  bool aligned16 = ((uintptr_t)x & 15) == 0;
-  if constexpr (ROT)
-    for (int s = 0; s < nshards; s++) aligned16 = aligned16 && ((uintptr_t)su.suh[s] & 15) == 0;
-  if (aligned16) {
-    const int hu = hunits >= (1u << 17) ? 4 : hunits >= (1u << 15) ? 2 : 1;
-    const dim3 hgrid((unsigned)((hunits + 16 * hu - 1) / (16 * hu)));
-    auto frag = x_bf16 ? (hu == 4 ? had_in_frag16_kernel<true, 4, ROT> : hu == 2 ? had_in_frag16_kernel<true, 2, ROT>
-                                                                                 : had_in_frag16_kernel<true, 1, ROT>)
-                       : (hu == 4 ? had_in_frag16_kernel<false, 4, ROT> : hu == 2 ? had_in_frag16_kernel<false, 2, ROT>
-                                                                                  : had_in_frag16_kernel<false, 1, ROT>);
-    frag<<<hgrid, 256, 0, st>>>(x, rows, k, su, nshards, xh);
-  } else {
-    const int hu = hunits >= (1u << 17) ? 4 : 1;
-    const dim3 hgrid((unsigned)((hunits + 8 * hu - 1) / (8 * hu)));
-    auto frag = x_bf16 ? (hu == 4 ? had_in_frag_kernel<true, 4, ROT> : had_in_frag_kernel<true, 1, ROT>)
-                       : (hu == 4 ? had_in_frag_kernel<false, 4, ROT> : had_in_frag_kernel<false, 1, ROT>);
-    frag<<<hgrid, 256, 0, st>>>(x, rows, k, su, nshards, xh);
-  }
+  const dim3 hgrid((unsigned)((rows + 63) / 64), (unsigned)(k / 128), ROT && rows < 1024 ? (unsigned)nshards : 1u);
+  const uint16_t* xr = static_cast<const uint16_t*>(x);
+  if (x_bf16)
+    rotate_rows_kernel<true, ROT><<<hgrid, 256, 0, st>>>(xr, rows, k, su, nshards, xh);
+  else
+    rotate_rows_kernel<false, ROT><<<hgrid, 256, 0, st>>>(xr, rows, k, su, nshards, xh);
   EXL3_CHECK_LAUNCH();
   const dim3 grid((unsigned)(L.groups + L.tiles - L.sk_tiles));
   bool ok;

@@ -80,86 +80,31 @@ __global__ __launch_bounds__(kSortThreads) void moe_sort_kernel(MoeGemmArgs a) {
   }
 }
 
-typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
-
-// 8 fp16 (or raw 16-bit) values by two 8-byte loads: the tensors need no more alignment
-__device__ __forceinline__ u32x4 load8(const uint16_t* p) {
-  const u32x2 a = *reinterpret_cast<const u32x2*>(p), b = *reinterpret_cast<const u32x2*>(p + 4);
-  return u32x4{a.x, a.y, b.x, b.y};
-}
-
-// fp16(Had(fp16(x) * suh)) of a 128-block on 16 lanes, lane t holding positions 8t .. 8t+7, as fp16 pairs: the stages and
-// pairings of had128_x4 (h = 1, 2, 4 in the lane, then lane xor 1, 2, 4, 8)
-template <bool X_BF16>
-__device__ __forceinline__ void rotate16(u32x4 xv, u32x4 sv, uint32_t (&d)[4]) {
-  const half8_t sc = __builtin_bit_cast(half8_t, sv);
-  float f[8];
-#pragma unroll
-  for (int i = 0; i < 8; i++) {
-    const uint16_t raw = (uint16_t)((i & 1) ? xv[i >> 1] >> 16 : xv[i >> 1] & 0xFFFF);
-    const _Float16 v = X_BF16 ? (_Float16)bf16_to_f32(raw) : __builtin_bit_cast(_Float16, raw);
-    f[i] = (float)(_Float16)(v * sc[i]);
-  }
-#pragma unroll
-  for (int h = 1; h < 8; h <<= 1)
-#pragma unroll
-    for (int i = 0; i < 8; i++)
-      if (!(i & h)) {
-        const float p = f[i], q = f[i + h];
-        f[i] = p + q;
-        f[i + h] = p - q;
-      }
-  had_stage<1>(f[0], f[1], f[2], f[3]);
-  had_stage<1>(f[4], f[5], f[6], f[7]);
-  had_stage<2>(f[0], f[1], f[2], f[3]);
-  had_stage<2>(f[4], f[5], f[6], f[7]);
-  had_stage<4>(f[0], f[1], f[2], f[3]);
-  had_stage<4>(f[4], f[5], f[6], f[7]);
-  had_stage<8>(f[0], f[1], f[2], f[3]);
-  had_stage<8>(f[4], f[5], f[6], f[7]);
-#pragma unroll
-  for (int q = 0; q < 4; q++)
-    d[q] = __builtin_bit_cast(uint32_t, half2_t{had_scale_f16(f[2 * q]), had_scale_f16(f[2 * q + 1])});
-}
-
-// The rotated gate and up inputs of every routed slot of the class by sorted position, in fragment order.  16 lanes per
-// (position, two 128-blocks), both projections from one load of x, all loads first; the 4 positions of a wave are
-// adjacent, so each k-step's 64 bytes of them form one 256-byte run.
-constexpr int kInBlocks = 2;
+// The rotated gate and up inputs of every routed slot of the class by sorted position, in fragment order: one wave per
+// (16 positions, 128-block), both projections from one load of x (2048 tokens: 51 us with the butterfly on 16 lanes per
+// row, 39 so; 134 MB written).
 template <bool X_BF16>
 __global__ __launch_bounds__(256) void moe_gemm_in_kernel(MoeGemmArgs a, const uint16_t* __restrict__ x) {
-  const int pos = blockIdx.x * 16 + (threadIdx.x >> 4), b0 = blockIdx.y * kInBlocks, t = threadIdx.x & 15;
-  if (pos >= a.totals[0]) return;  // whole 16-lane rows: the lane stages stay inside them
-  const int2 at = a.sorted[pos];
-  const int el = moe_row(a, at.y);
-  if (el < 0) return;
-  const int blocks = a.H >> 7;
-  u32x4 xv[kInBlocks], sv[kInBlocks][2];
+  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), l = threadIdx.x & 63, c = l & 15, j = l >> 4;
+  const int pos0 = (blockIdx.x * 4 + w) * 16, b = blockIdx.y, total = a.totals[0];
+  if (pos0 >= total) return;  // wave-uniform
+  const int pos = pos0 + c;
+  const int2 at = a.sorted[pos < total ? pos : total - 1];
+  const int el = moe_row(a, at.y);  // -1: another class's row, read as expert 0's and not stored
+  const size_t kk = b * 128 + 8 * j, e0 = (size_t)(el < 0 ? 0 : el) * a.H;
+  half8_t xv[4];
+  load_row_frags<X_BF16>(x + (size_t)(at.x / a.top_k) * a.H + kk, xv);
+  const HadFrags had = had_frags_act(l);
 #pragma unroll
-  for (int i = 0; i < kInBlocks; i++) {
-    const int kk = (b0 + i < blocks ? b0 + i : b0) * 128 + 8 * t;  // past the last block: b0 again, not stored
-    xv[i] = load8(x + (size_t)(at.x / a.top_k) * a.H + kk);
-    sv[i][0] = load8(a.suh[0] + (size_t)el * a.H + kk);
-    sv[i][1] = load8(a.suh[1] + (size_t)el * a.H + kk);
-  }
+  for (int s = 0; s < 2; s++) {
+    half8_t in[4];
 #pragma unroll
-  for (int i = 0; i < kInBlocks; i++) {
-    if (b0 + i >= blocks) break;
+    for (int kb = 0; kb < 4; kb++) in[kb] = times8(xv[kb], a.suh[s] + e0 + kk + 32 * kb);
+    uint16_t* dst = a.pre_in + ((size_t)(s * (a.H >> 5) + b * 4) * a.slots + pos) * 32 + 8 * j;
 #pragma unroll
-    for (int s = 0; s < 2; s++) {
-      uint32_t d[4];
-      rotate16<X_BF16>(xv[i], sv[i][s], d);
-      // fragment order: in the 32-block of lanes t / 4, lane a = t % 4 holds, per q = 0..3, the slot pair (q, tr = a / 2,
-      // e = 2 (a & 1) + 0/1); lanes a and a ^ 1 swap two pairs so that each stores whole 8-byte groups (q, tr)
-      const bool low = (t & 1) == 0;
-      const uint32_t g0 = (uint32_t)__builtin_amdgcn_mov_dpp((int)(low ? d[1] : d[0]), 0xB1, 0xF, 0xF, false);
-      const uint32_t g1 = (uint32_t)__builtin_amdgcn_mov_dpp((int)(low ? d[3] : d[2]), 0xB1, 0xF, 0xF, false);
-      const u32x2 o0 = low ? u32x2{d[0], g0} : u32x2{g0, d[1]};
-      const u32x2 o1 = low ? u32x2{d[2], g1} : u32x2{g1, d[3]};
-      const int tr = (t & 3) >> 1, q0 = low ? 0 : 1;
-      uint16_t* dst = a.pre_in + ((size_t)(s * (a.H >> 5) + (b0 + i) * 4 + (t >> 2)) * a.slots + pos) * 32 + tr * 4;
-      *reinterpret_cast<u32x2*>(dst + q0 * 8) = o0;
-      *reinterpret_cast<u32x2*>(dst + (q0 + 2) * 8) = o1;
+    for (int u = 0; u < 4; u++) {
+      const half8_t o = had_pair(had, in, u);
+      if (pos < total && el >= 0) *reinterpret_cast<half8_t*>(dst + (size_t)u * a.slots * 32) = o;
     }
   }
 }
@@ -206,13 +151,6 @@ __device__ __forceinline__ void moe_multiply(const MoeGemmArgs& a, const uint16_
   tile_multiply<K, CB, MI, PIECES>(
       lds, act, part * MI * 1024, lds + kARing * AP * 1024 + w * 1024, brsrc, bgoff,
       [&](int kt) { return 2 * kt * row_bytes; }, 0, steps, (w & 4) != 0, l, acc);
-}
-
-__device__ __forceinline__ half8_t times8(half8_t v, const uint16_t* p) {
-  const half8_t s = __builtin_bit_cast(half8_t, load8(p));
-#pragma unroll
-  for (int e = 0; e < 8; e++) v[e] = (_Float16)(v[e] * s[e]);
-  return v;
 }
 
 // 128 columns of gate (waves 0-3) and the same of up (waves 4-7), then per 16-row block in one wave: both output
@@ -324,7 +262,7 @@ int moe_gemm_route(const MoeGemmArgs& a, hipStream_t st) {
 }
 
 int moe_gemm_inputs(const MoeGemmArgs& a, const void* x, bool x_bf16, hipStream_t st) {
-  const dim3 grid((unsigned)((a.slots + 15) / 16), (unsigned)((a.H / 128 + kInBlocks - 1) / kInBlocks));
+  const dim3 grid((unsigned)((a.slots + 63) / 64), (unsigned)(a.H / 128));
   if (x_bf16)
     moe_gemm_in_kernel<true><<<grid, 256, 0, st>>>(a, static_cast<const uint16_t*>(x));
   else

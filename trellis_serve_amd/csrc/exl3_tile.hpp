@@ -14,6 +14,38 @@ namespace exl3 {
 
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
+typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+
+// 8 fp16 (or raw 16-bit) values by two 8-byte loads: the tensors need no more alignment
+__device__ __forceinline__ u32x4 load8(const uint16_t* p) {
+  const u32x2 a = *reinterpret_cast<const u32x2*>(p), b = *reinterpret_cast<const u32x2*>(p + 4);
+  return u32x4{a.x, a.y, b.x, b.y};
+}
+
+__device__ __forceinline__ half8_t times8(half8_t v, const uint16_t* p) {
+  const half8_t s = __builtin_bit_cast(half8_t, load8(p));
+#pragma unroll
+  for (int e = 0; e < 8; e++) v[e] = (_Float16)(v[e] * s[e]);
+  return v;
+}
+
+// A row's 128 values as MFMA fragments: v[kb] = values 32 kb ..+7 from p (the lane's 8 l / 16 included), bf16 rounded to
+// fp16
+template <bool X_BF16>
+__device__ __forceinline__ void load_row_frags(const uint16_t* p, half8_t (&v)[4]) {
+  u32x4 raw[4];
+#pragma unroll
+  for (int kb = 0; kb < 4; kb++) raw[kb] = load8(p + 32 * kb);
+#pragma unroll
+  for (int kb = 0; kb < 4; kb++) {
+    v[kb] = __builtin_bit_cast(half8_t, raw[kb]);
+    if constexpr (X_BF16)
+#pragma unroll
+      for (int e = 0; e < 8; e++)
+        v[kb][e] = (_Float16)bf16_to_f32((uint16_t)((e & 1) ? raw[kb][e >> 1] >> 16 : raw[kb][e >> 1] & 0xFFFF));
+  }
+}
+
 constexpr int kBN = 256, kBK = 32;
 constexpr int kGemmWaves = 8, kGemmThreads = kGemmWaves * 64;
 constexpr int kARing = 4, kBitsRing = 4;           // ring slots (powers of two)
