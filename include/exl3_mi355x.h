@@ -67,9 +67,9 @@ typedef struct exl3_shard {
 int exl3_abi_version(void);
 const char* exl3_last_error(void);
 /* Checks that `device` is a gfx950, then probes (one small launch, synchronous) that workgroups whose ids agree mod 8
- * run on one XCD; once a probe has passed, decode-GEMV launches whose column-block count is a multiple of 8 keep their
- * split-K partials and counters in that XCD's L2 (otherwise, and before any call here, they use device-coherent
- * accesses; results are the same bits either way).  Call it before capturing graphs.  Replaces init_device
+ * run on one XCD; once a probe has passed, decode-GEMV launches whose column-block count is a multiple of 8 keep
+ * their split-K partials and counters in that XCD's L2 (otherwise, and before any call here, they use device-
+ * coherent accesses; results are the same bits either way).  Call it before capturing graphs.  Replaces init_device
  * (cuda/csrc/exl3_marlin.cu:537). */
 int exl3_init_device(int device);
 /* 1 when split-K chains may stay in one XCD's L2 (a probe of exl3_init_device passed and EXL3_GEMV_XCD_LOCAL is not
@@ -103,17 +103,20 @@ int exl3_had_out_into(const void* y, int rows, int n, const void* svh, void* out
 
 /* ---- fused decode-GEMV / GEMM (subsystems 2, 3) --------------------------------------------------------------- */
 /* Workspace bytes exl3_linear needs for `rows` rows of a group with input width k and `n_total` output columns
- * (n_total / 128 at most EXL3_WORKSPACE_COUNTER_BYTES / 4); 0 means none.  Deterministic in its arguments.  The
- * workspace holds the split counters (EXL3_WORKSPACE_COUNTER_BYTES, zero before the first use) and fp32 split
- * partials; calls that share a workspace must be ordered on one stream.  exl3_linear checks the workspace against the
- * split plans of its own launches and returns EXL3_ERR_INVALID, launching nothing, when it is short. */
+ * (n_total / 128 at most EXL3_WORKSPACE_COUNTER_BYTES / 4); 0 means none.  Deterministic in its arguments (and, for
+ * 33-64 rows of a large layer, the current device's CU count).  The workspace holds the split counters
+ * (EXL3_WORKSPACE_COUNTER_BYTES, zero before the first use), fp32 split partials and rotated rows; calls that share
+ * a workspace must be ordered on one stream.  exl3_linear checks the workspace against the split plans of its own
+ * launches and returns EXL3_ERR_INVALID, launching nothing, when it is short. */
 size_t exl3_linear_workspace_bytes(int rows, int k, int n_total, int K);
 
 /* y[rows, sum n_s] = concat_s( Had128(Had128(x * suh_s) @ W_s) * svh_s ) with fp32 accumulation; fp16 output of
  * the GEMM, output transform as exl3_had_out_into.  x fp16|bf16 [rows, k]; y fp16|bf16 [rows, sum n_s].
  * All shards share K and codebook.  One launch serves up to 64 rows (each decoded tile feeds 1, 2 or 4 16-row MFMA
- * groups); more rows take more launches.  Replaces exl3_linear_marlin_out / exl3_linear_marlin_multi_out
- * (cuda/csrc/exl3_marlin.cu:489-527) behind torch.ops.sglang_exl3.linear (cuda/src/sglang_exl3/runtime/ops.py:133). */
+ * groups); 33-64 rows of a layer of at least 4096 units of 128 x 128 weights run as exl3_linear_prefill does (one
+ * decode for all rows); more rows take more launches.
+ * Replaces exl3_linear_marlin_out / exl3_linear_marlin_multi_out (cuda/csrc/exl3_marlin.cu:489-527) behind
+ * torch.ops.sglang_exl3.linear (cuda/src/sglang_exl3/runtime/ops.py:133). */
 int exl3_linear(const void* x, int x_bf16, int rows, int k, const exl3_shard* shards_host, int nshards, int K,
                 int codebook, void* y, int y_bf16, void* workspace, size_t workspace_bytes, void* stream);
 
@@ -121,10 +124,11 @@ int exl3_linear(const void* x, int x_bf16, int rows, int k, const exl3_shard* sh
  * those of the prefill decode-GEMM); 0 for bad shapes.  Same counter-region contract as exl3_linear_workspace_bytes. */
 size_t exl3_gemm_rotated_workspace_bytes(int rows, int k, int n, int K);
 /* out fp16 [rows, n] = xh @ W_inner in the rotated basis (no Hadamards, no sign vectors); fp32 accumulation, one
- * rounding to fp16; xh fp16 [rows, k].  Identity rows of xh read W_inner out exactly.  The rows run through the kernel
- * that serves the same row count in a linear: below 65 rows the decode-GEMV (one 16-row group per launch, two decoded
- * tiles per MFMA), from 65 rows the prefill decode-GEMM.  Replaces exl3_gemm_marlin (cuda/csrc/exl3_marlin.cu:411-423),
- * the one-hot test entry of cuda/src/sglang_exl3/parity/marlin_parity.py:149-159. */
+ * rounding to fp16; xh fp16 [rows, k].  Identity rows of xh read W_inner out exactly.  The rows run through the
+ * kernel that serves the same row count in a linear: below 65 rows the decode-GEMV (one 16-row group per launch, two
+ * decoded tiles per MFMA), from 65 rows the prefill decode-GEMM.  Replaces exl3_gemm_marlin
+ * (cuda/csrc/exl3_marlin.cu:411-423), the one-hot test entry of
+ * cuda/src/sglang_exl3/parity/marlin_parity.py:149-159. */
 int exl3_gemm_rotated(const void* xh, int rows, int k, const void* trellis, int n, int K, int codebook, void* out,
                       void* workspace, size_t workspace_bytes, void* stream);
 
@@ -147,14 +151,14 @@ int exl3_linear_noalloc(const void* x, int x_bf16, int rows, int k, const exl3_s
 /* ---- prefill decode-GEMM (subsystem 3) ------------------------------------------------------------------------ */
 /* Workspace bytes of exl3_linear_prefill for `rows` rows of a group with input width k, n_total output columns and
  * nshards shards: EXL3_WORKSPACE_COUNTER_BYTES of split counters (zero before the first use; every call leaves them
- * zero), the per-shard rotated activations (fp16 [nshards][rows][k]), then fp32 partials of the k-split tail tiles.
+ * zero), the per-shard rotated activations (fp16 [nshards][rows][k]), then fp32 partials of the shared tiles.
  * Depends on the current device's CU count. */
 size_t exl3_prefill_workspace_bytes(int rows, int k, int n_total, int nshards);
 /* Same contract as exl3_linear for many rows: the input rotation of every shard goes to the workspace, then one
- * fused decode-GEMM launch (weights decoded into LDS, fp16 MFMA, fp32 accumulation, output rotation in the epilogue)
- * writes y.  Tiles that do not fill a whole round of the machine are split along k and summed in a fixed order, so
- * results do not depend on scheduling.  Replaces the reference's prefill branch -- rotation, ExLlamaV3 reconstruct, cuBLAS, rotation
- * (cuda/src/sglang_exl3/runtime/ops.py:36-59, 87-95). */
+ * fused decode-GEMM launch (weights decoded into registers, fp16 MFMA, fp32 accumulation, output rotation in the
+ * epilogue) writes y.  Tiles that do not fill a whole round of the machine are split along k and summed in a fixed
+ * order, so results do not depend on scheduling.  Replaces the reference's prefill branch -- rotation, ExLlamaV3
+ * reconstruct, cuBLAS, rotation (cuda/src/sglang_exl3/runtime/ops.py:36-59, 87-95). */
 int exl3_linear_prefill(const void* x, int x_bf16, int rows, int k, const exl3_shard* shards_host, int nshards, int K,
                         int codebook, void* y, int y_bf16, void* workspace, size_t workspace_bytes, void* stream);
 
@@ -186,7 +190,8 @@ size_t exl3_moe_workspace_bytes(int tokens, int top_k, int num_experts, int hidd
  * topk_ids int32 [T, top_k] (top_k <= 64), topk_weights fp32 [T, top_k], y fp16|bf16 [T, H].  Replaces the five
  * launches of cuda/src/sglang_exl3/kernels/marlin_moe.py:272-294 (moe_had_in, moe_gemm, moe_glu_had_in, moe_gemm,
  * moe_combine; cuda/csrc/exl3_marlin_moe.cu:376-499) and the align step (exl3_marlin_moe.cu:532-594) with four
- * launches (three for a single token).  Calls that share a workspace must not overlap. */
+ * launches (three for a single token, five with many slots per expert: the decode-GEMMs over slots sorted by
+ * expert).  Calls that share a workspace must not overlap. */
 int exl3_moe_forward(const void* x, int x_bf16, int tokens, int hidden, const void* topk_ids, const void* topk_weights,
                      int top_k, int num_experts, int inter, const exl3_moe_weights* weights_host, int K_gate_up,
                      int K_down, int codebook, void* y, int y_bf16, void* workspace, size_t workspace_bytes,
@@ -218,8 +223,8 @@ int exl3_moe_forward_classes(const void* x, int x_bf16, int tokens, int hidden, 
 
 /* ---- MoE per-launch stages (the reference's moe_align_decode, moe_had_in, moe_gemm, moe_glu_had_in, moe_combine:
  * cuda/csrc/exl3_marlin_moe.cu:376-618; run order cuda/src/sglang_exl3/kernels/marlin_moe.py:272-294).  The same
- * arithmetic as exl3_moe_forward, one launch per stage, for callers that drive the stages themselves.  Weights are the
- * stored trellis stacks ([E][k/16][n/16][16K] per projection), not a repacked stack. */
+ * arithmetic as exl3_moe_forward, one launch per stage, for callers that drive the stages themselves.  Weights are
+ * the stored trellis stacks ([E][k/16][n/16][16K] per projection), not a repacked stack. */
 
 /* Routing in the layout of vLLM's moe_align_block_size for one block size (1..64): the slots of every expert (ids
  * outside [0, num_experts), or mapped to -1 by expert_map, dropped) in ascending expert order, each expert's run
@@ -284,12 +289,13 @@ int exl3_moe_combine(const void* yd, const float* topk_weights, const int* topk_
 /* Workspace bytes of exl3_kv_decode_attention (fp32 partial (m, l, O) per chunk of pages).  No zero-fill needed.
  * Not monotone in batch (a smaller batch can take more chunks per sequence); never larger for fewer pages. */
 size_t exl3_kv_decode_workspace_bytes(int batch, int num_q_heads, int num_kv_heads, int max_pages);
-/* out[b][h] = softmax(sm_scale * q[b][h] . K_b^T) V_b over the first seq_lens[b] tokens of sequence b, whose pages are
- * page_table[b][0 .. ceil(seq_lens[b] / 16)); query head h reads KV head h / (Hq / Hkv) (Hq / Hkv <= 16).
- * q fp16 [B][Hq][128], page_table int32 [B][max_pages], seq_lens int32 [B], out fp16 [B][Hq][128].  A sequence of
- * length 0 gives zeros; page ids outside [0, num_pages) are clamped (never read outside the cache).  head_dim must be
- * 128 and page_size 16.  Two launches (split-KV over page chunks, then the log-sum-exp merge), one when a single chunk
- * covers every sequence; deterministic. */
+/* out[b][h] = softmax(sm_scale * q[b][h] . K_b^T) V_b over the first seq_lens[b] tokens of sequence b, whose pages
+ * are page_table[b][0 .. ceil(seq_lens[b] / 16)); query head h reads KV head h / (Hq / Hkv) (Hq / Hkv <= 16). q fp16
+ * [B][Hq][128], page_table int32 [B][max_pages], seq_lens int32 [B], out fp16 [B][Hq][128].  A sequence of length 0
+ * gives zeros; page ids outside [0, num_pages) are clamped (never read outside the cache).  head_dim must be 128 and
+ * page_size 16.  Two launches (split-KV over page chunks, then the log-sum-exp merge), one where the table's width
+ * already says that a single chunk covers every sequence; deterministic.  Up to 64 sequences are split by their
+ * lengths, so a sequence's rounding can depend on the other lengths of its batch. */
 int exl3_kv_decode_attention(const void* q, const void* k_cache, const void* v_cache, const void* k_scale,
                              const void* v_scale, int num_pages, const void* page_table, int max_pages,
                              const void* seq_lens, int batch, int num_q_heads, int num_kv_heads, int head_dim,

@@ -19,12 +19,12 @@
 // decoded weight goes through LDS and only the A pieces are shared between waves.  One workgroup per CU (two at 64
 // rows).  Against wave tiles of 128 x 64 with the decoded weights in LDS (two waves per weight, a barrier that the
 // step's first LDS reads wait behind): 5120 -> 16384 at 4096 rows, one k-step 1.05 -> 0.96 us, a tile's epilogue 22 ->
-// 6 us; 729-745 -> 641-676 us in all.
+// 6 us; 729-745 -> 641-676 us in all (636 with the k-steps in pairs).
 //
-// What bounds it: issue.  Per k-step and wave of a 256-row tile 32 MFMAs (512 cycles) and ~90 VALU of decode (360),
-// two waves per SIMD; counted at 4096 rows: matrix core 54 % busy, VALU 37 %, 18 % both, at 2.0 GHz.  The two waves of
-// a SIMD take decode and multiply in opposite order (2-3 %); forced bursts, a deeper fragment window (8) and an explicit
-// MFMA / VALU interleave were slower.
+// What bounds it: issue.  Per k-step and wave of a 256-row tile 32 MFMAs (512 cycles) and 71 VALU of decode (284),
+// two waves per SIMD.  With 88 VALU (one k-step at a time) the counters at 4096 rows read: matrix core 54 % busy, VALU
+// 37 %, 18 % both, at 2.0 GHz.  The two waves of a SIMD take decode and multiply in opposite order (2-3 %); forced
+// bursts, a deeper fragment window (8) and an explicit MFMA / VALU interleave were slower.
 //
 // Work decomposition (1-D grid of work items, dispatched in order): tiles are numbered column block fastest, so
 // consecutive workgroups share their A rows in L2.  When the tile count is not a multiple of the machine's

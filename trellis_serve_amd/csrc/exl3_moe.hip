@@ -8,10 +8,11 @@
 //   y[t] = sum_j w[t, j] * d[slot] in fp32, slot order, one rounding; slots whose expert id is outside [0, E) are
 //          skipped (exl3_marlin_moe.cu:274)
 //
-// Launches (the reference uses five plus an align launch):
+// Launches (the reference uses five plus an align launch), by the number of slots:
 //   single token (slot mode): moe_gemv_kernel<PHASE 0> -> moe_gemv_kernel<PHASE 1> -> moe_combine_kernel; grid row =
 //                      slot, its expert read from topk_ids; the gate/up reducers write fp16 g|u rows and the down
 //                      workgroups compute the GLU and the input rotations in their prologues.
+//   many slots per expert (moe_tile_rows): the sorted decode-GEMMs of exl3_moe_gemm.hip, then moe_combine_kernel.
 //   several tokens: moe_route_prep_kernel -> moe_gemv_kernel<PHASE 0> -> moe_gemv_kernel<PHASE 1> ->
 //                      moe_combine_kernel; grid row = active expert.
 //   moe_route_prep_kernel  the rotated gate/up inputs fp16(Had(x[token] * suh)) per (slot, shard), written once

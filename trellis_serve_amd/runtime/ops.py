@@ -5,10 +5,9 @@ row-count dispatch, dtype handling and output allocation live inside the op so a
 Dispatch (the reference's `_linear`, runtime/ops.py:62-126, with MI355X switch points):
   rows < PREFILL_ROWS  -> fused decode-GEMV (exl3_linear, up to 64 rows per launch)
   rows >= PREFILL_ROWS -> fused decode-GEMM (exl3_linear_prefill)
-PREFILL_ROWS comes from measured crossovers on the 27B shapes: the GEMV streams the weights once per 32 or 64 rows
-(two or four 16-row MFMA groups per decoded tile), the fused GEMM once for up to 256 rows.  At 64 rows the layer set
-is faster on the GEMV (q/k/v 39.3 vs 49.6 us, o 37.4 vs 51.6, gate/up 104.3 vs 96.5, down 74.3 vs 74.6), at 96 rows
-on the GEMM (382 vs 308 us).
+PREFILL_ROWS is the row count from which the fused GEMM is faster on every 27B shape: it decodes the weights once for up
+to 256 rows.  Below it exl3_linear itself gives 33-64 rows of a large layer to the GEMM (48 rows: gate/up 81.5 -> 55 us,
+down 61 -> 53) and keeps the narrow ones on the GEMV (q/k/v 33.5 us at 48 rows against 36, o 30 against 30-38).
 """
 from __future__ import annotations
 
