@@ -103,8 +103,8 @@ int exl3_had_out_into(const void* y, int rows, int n, const void* svh, void* out
 
 /* ---- fused decode-GEMV / GEMM (subsystems 2, 3) --------------------------------------------------------------- */
 /* Workspace bytes exl3_linear needs for `rows` rows of a group with input width k and `n_total` output columns
- * (n_total / 128 at most EXL3_WORKSPACE_COUNTER_BYTES / 4); 0 means none.  Deterministic in its arguments (and, for
- * 33-64 rows of a large layer, the current device's CU count).  The workspace holds the split counters
+ * (n_total / 128 at most EXL3_WORKSPACE_COUNTER_BYTES / 4); 0 means none.  Deterministic in its arguments (and, past
+ * 32 rows of a large layer, the current device's CU count).  The workspace holds the split counters
  * (EXL3_WORKSPACE_COUNTER_BYTES, zero before the first use), fp32 split partials and rotated rows; calls that share
  * a workspace must be ordered on one stream.  exl3_linear checks the workspace against the split plans of its own
  * launches and returns EXL3_ERR_INVALID, launching nothing, when it is short. */
@@ -125,8 +125,8 @@ int exl3_linear(const void* x, int x_bf16, int rows, int k, const exl3_shard* sh
 size_t exl3_gemm_rotated_workspace_bytes(int rows, int k, int n, int K);
 /* out fp16 [rows, n] = xh @ W_inner in the rotated basis (no Hadamards, no sign vectors); fp32 accumulation, one
  * rounding to fp16; xh fp16 [rows, k].  Identity rows of xh read W_inner out exactly.  The rows run through the
- * kernel that serves the same row count in a linear: below 65 rows the decode-GEMV (one 16-row group per launch, two
- * decoded tiles per MFMA), from 65 rows the prefill decode-GEMM.  Replaces exl3_gemm_marlin
+ * kernels of a linear: below 65 rows the decode-GEMV (one 16-row group per launch, two decoded tiles per MFMA; a
+ * linear's 33-64 rows of a large layer take the GEMM), from 65 rows the prefill decode-GEMM.  Replaces exl3_gemm_marlin
  * (cuda/csrc/exl3_marlin.cu:411-423), the one-hot test entry of
  * cuda/src/sglang_exl3/parity/marlin_parity.py:149-159. */
 int exl3_gemm_rotated(const void* xh, int rows, int k, const void* trellis, int n, int K, int codebook, void* out,

@@ -136,6 +136,15 @@ def test_reported_workspace_sizes_cover_every_launch_plan(lib):
                         _lib.EXL3_ERR_INVALID, (K, k, n, rows)
 
 
+@pytest.mark.parametrize("k,n,K", [(5120, 34816, 3), (17408, 5120, 3), (8192, 8192, 4), (5120, 13312, 8)])
+def test_linear_workspace_of_the_most_rows_serves_fewer(lib, k, n, K):
+    """Layers whose 33-64 rows take the decode-GEMM: a buffer sized for 33, 64, 65 or 200 rows still serves every smaller
+    row count past 16 (one row group's launches split k by their own rule)."""
+    need = [lib.exl3_linear_workspace_bytes(r, k, n, K) for r in range(201)]
+    for most in (33, 64, 65, 200):
+        assert need[most] >= max(need[17:most + 1]), most
+
+
 def test_kv_workspace_reserved_for_the_largest_batch_covers_every_smaller_call(lib):
     """A smaller batch can split each sequence into more page chunks, so the KV workspace is not monotone in the
     batch: the reservation takes the maximum over batch sizes 1..max_batch at the reserved page count, and that must

@@ -643,9 +643,11 @@ static size_t gemv_workspace_bytes(int rows, int k, int n_total, int K, int laun
 // Rows that exl3_linear hands to the decode-GEMM: past 32 rows of a large layer the GEMV would stream and decode the
 // weights twice (two launches of two row groups), where one 64- or 128-row GEMM tile reads them once (48 rows, us:
 // gate/up 81.5 -> 55, down 61 -> 53).  Below 4096 units of 128 x 128 weights (q/k/v 2560, o 1920) the GEMV's one
-// four-group launch is as fast (31-39 and 29-36 us at 33-64 rows against 35-39 and 30-40).
+// four-group launch is as fast (31-39 and 29-36 us at 33-64 rows against 35-39 and 30-40).  Rows whose rotated copy
+// passes the GEMM's 2 GiB buffer range (k of 2^24 at 64 rows) stay with the GEMV, which has no such limit.
 static bool linear_takes_gemm(int rows, int k, int n_total) {
-  return rows > kGemvPairRows && rows <= kGemvQuadRows && (size_t)(n_total / 128) * (k / 128) >= 4096;
+  return rows > kGemvPairRows && rows <= kGemvQuadRows && (size_t)(n_total / 128) * (k / 128) >= 4096 &&
+         (int64_t)rows * k * 2 <= INT32_MAX;
 }
 
 // ---- split-K chain inside one XCD ---------------------------------------------------------------------------
@@ -967,9 +969,11 @@ extern "C" size_t exl3_linear_workspace_bytes(int rows, int k, int n_total, int 
   if (rows <= 0 || k <= 0 || n_total <= 0 || k % 128 || n_total % 128 || n_total / 128 > kMaxCounters ||
       !valid_bits(K))
     return 0;
-  if (linear_takes_gemm(rows, k, n_total)) return linear_gemm_workspace_bytes(rows, k, n_total);
-  // exl3_linear's launches: up to 64 rows each (1, 2 or 4 row groups per decoded tile), then the remainder
-  return gemv_workspace_bytes(rows, k, n_total, K, kGemvQuadRows, true);
+  // exl3_linear's launches: up to 64 rows each (1, 2 or 4 row groups per decoded tile), then the remainder; and past 32
+  // rows the decode-GEMM's of up to 64, so that one buffer sized for a caller's most rows serves fewer rows too
+  const size_t gemv = gemv_workspace_bytes(rows, k, n_total, K, kGemvQuadRows, true);
+  const int most = std::min(rows, kGemvQuadRows);
+  return linear_takes_gemm(most, k, n_total) ? std::max(gemv, linear_gemm_workspace_bytes(most, k, n_total)) : gemv;
 }
 
 extern "C" int exl3_linear(const void* x, int x_bf16, int rows, int k, const exl3_shard* shards_host, int nshards,
