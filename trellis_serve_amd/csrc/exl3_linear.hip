@@ -986,13 +986,14 @@ extern "C" int exl3_linear(const void* x, int x_bf16, int rows, int k, const exl
   int n_total = 0;
   if (int rc = build_shards(shards_host, nshards, k, K, &sa, &n_total)) return rc;
   if (rows == 0) return EXL3_OK;
-  if (linear_takes_gemm(rows, k, n_total)) {
-    const size_t need = linear_gemm_workspace_bytes(rows, k, n_total);
+  if (rows > kGemvPairRows) {  // the reported size also covers fewer rows: held to it here, before either path
+    const size_t need = exl3_linear_workspace_bytes(rows, k, n_total, K);
     EXL3_CHECK_ARG(workspace && workspace_bytes >= need, "exl3_linear: workspace %zu bytes, need %zu", workspace_bytes,
                    need);
+  }
+  if (linear_takes_gemm(rows, k, n_total))
     return exl3_linear_prefill(x, x_bf16, rows, k, shards_host, nshards, K, codebook, y, y_bf16, workspace,
                                workspace_bytes, stream);
-  }
   return launch_gemv(sa, x, true, x_bf16 != 0, rows, k, K, codebook, n_total, workspace, workspace_bytes, y,
                      y_bf16 != 0, as_stream(stream), kGemvQuadRows, "exl3_linear");
 }
