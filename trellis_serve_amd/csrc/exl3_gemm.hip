@@ -2,7 +2,7 @@
 //
 // Reference semantics: the reference's prefill is decode-to-HBM + cuBLAS between its rotation launches
 // (cuda/src/sglang_exl3/runtime/ops.py:36-59); the fused Marlin path serves < 256 rows
-// (exl3_marlin_template.h).  Here the weights are decoded into LDS inside the GEMM and never reach HBM.
+// (exl3_marlin_template.h).  Here the weights are decoded into registers inside the GEMM and never reach HBM.
 //
 // Operands
 //   A: xh in "fragment order", k-step major: the rotated activations with k permuted inside every 32-wide block so
@@ -364,7 +364,7 @@ __global__ __launch_bounds__(kGemmThreads, MI <= 4 ? 4 : 2) void gemm_kernel(Gem
 
 
 
-// Concurrent workgroups of the device (one per CU: 135 KB of LDS), per device, queried once.
+// Workgroups that run at once, counted as one per CU (a 256-row tile takes 135 KB of LDS), per device, queried once.
 static int gemm_slots() {
   static int slots[64] = {0};
   int dev = 0;

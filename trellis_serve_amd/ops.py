@@ -290,8 +290,8 @@ def had_out_into(y: torch.Tensor, svh: torch.Tensor, out: torch.Tensor, col0: in
 def gemm_rotated(xh: torch.Tensor, trellis: torch.Tensor, codebook: int,
                  out: torch.Tensor | None = None) -> torch.Tensor:
     """xh @ W_inner in the rotated basis, fp32 accumulation, fp16 out; identity rows read W_inner out exactly
-    (kernels/marlin.py:153-159).  Below 65 rows the decode-GEMV serves the rows, from 65 rows the prefill decode-GEMM,
-    as in a linear."""
+    (kernels/marlin.py:153-159).  Below 65 rows the decode-GEMV serves the rows, from 65 rows the prefill
+    decode-GEMM."""
     k, n, K = _check_trellis(trellis)
     xh = _half(xh, "xh")
     if xh.dim() != 2 or xh.shape[1] != k:
