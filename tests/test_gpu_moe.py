@@ -369,7 +369,10 @@ MOE_GEMM_CASES = [(384, 128, 3, 3, 1, (1, 15, 16, 17, 63, 64, 0, 65, 70, 33), Fa
                   (256, 256, 2, 4, 0, (127, 128, 129, 200, 256, 257, 0), True),
                   (640, 384, 5, 6, 2, (300, 1, 180, 90), False),
                   (128, 128, 8, 8, 1, (400,), False),
-                  (512, 640, 4, 3, 2, (65, 66, 128, 130, 48, 100), True)]
+                  (512, 640, 4, 3, 2, (65, 66, 128, 130, 48, 100), True),
+                  (384, 256, 3, 4, 1, (32, 31, 33, 1, 16, 17, 64, 2, 0, 30), False),
+                  # more workgroups than CUs, 0 to 34 slots per expert: the 32-row code beside the 64-row one
+                  (256, 128, 3, 4, 1, tuple(7 * e % 35 for e in range(300)), False)]
 
 
 @pytest.mark.parametrize("case", MOE_GEMM_CASES, ids=[f"H{c[0]}-I{c[1]}-K{c[2]}-{c[3]}-cb{c[4]}" for c in MOE_GEMM_CASES])

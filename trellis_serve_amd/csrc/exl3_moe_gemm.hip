@@ -233,23 +233,32 @@ __device__ __forceinline__ void moe_down_tile(const MoeGemmArgs& a, const MoeTil
   }
 }
 
-// A tile of at most 64 slots takes the 64-row code also where tiles go up to 128.  64-row kernels are held to 128 VGPRs:
-// two workgroups per CU.
+// A tile of at most 64 slots takes the 64-row code also where tiles go up to 128, and one of at most 32 the 32-row code
+// where there are more workgroups than CUs, which then share issue slots (128 experts, top-8, 256 tokens: 161.6 -> 145.1
+// us; 2048 tokens 407 -> 404).  With at most one workgroup per CU a step's latency sets the time, and less work per step
+// only hides less of it (16 experts, 61 tokens, two layers: 142.5 us at 64 rows, 144.5 at 32).  64-row kernels are held
+// to 128 VGPRs: two workgroups per CU.
 template <int K, int CB, int PHASE, int MI>
 __global__ __launch_bounds__(kGemmThreads, MI == 4 ? 4 : 2) void moe_gemm_kernel(MoeGemmArgs a) {
   extern __shared__ __align__(16) uint8_t lds[];
-  const MoeWork wk = moe_work(blockIdx.x, PHASE ? (a.H + 255) / 256 : a.I / 128);
-  if (wk.tile >= a.totals[1]) return;
+  const int ncb = PHASE ? (a.H + 255) / 256 : a.I / 128, tiles = a.totals[1];
+  const MoeWork wk = moe_work(blockIdx.x, ncb);
+  if (wk.tile >= tiles) return;
   const MoeTile tile = a.tiles[wk.tile];
   const int el = moe_row(a, tile.expert);
   if (el < 0 || tile.rows <= 0) return;
+  const bool low = tile.rows <= 32 && tiles * ncb > 256;  // workgroup-uniform
   if constexpr (PHASE == 0) {
-    if (MI == 4 || tile.rows <= 64)
+    if (low)
+      moe_gate_up_tile<K, CB, 2>(a, tile, el, wk.cb, lds);
+    else if (MI == 4 || tile.rows <= 64)
       moe_gate_up_tile<K, CB, 4>(a, tile, el, wk.cb, lds);
     else
       moe_gate_up_tile<K, CB, MI>(a, tile, el, wk.cb, lds);
   } else {
-    if (MI == 4 || tile.rows <= 64)
+    if (low)
+      moe_down_tile<K, CB, 2>(a, tile, el, wk.cb, lds);
+    else if (MI == 4 || tile.rows <= 64)
       moe_down_tile<K, CB, 4>(a, tile, el, wk.cb, lds);
     else
       moe_down_tile<K, CB, MI>(a, tile, el, wk.cb, lds);

@@ -49,7 +49,7 @@ __device__ __forceinline__ void load_row_frags(const uint16_t* p, half8_t (&v)[4
 constexpr int kBN = 256, kBK = 32;
 constexpr int kGemmWaves = 8, kGemmThreads = kGemmWaves * 64;
 constexpr int kARing = 4, kBitsRing = 4;           // ring slots (powers of two)
-constexpr int kWindow = 4;                         // A fragments a wave holds ahead of their MFMAs
+constexpr int kWindow = 4;                         // A fragments a wave holds ahead of their MFMAs (at most MI)
 constexpr int kBitsStage = kGemmWaves * 64 * 16;   // 8 KB: per wave 64 lanes x 16 B (its 4 tiles of a k-step)
 constexpr int kCStride = kBN + 8;                  // epilogue fp16 C tile row stride (halves)
 // LDS of a tile of 16 MI rows whose k-step stages hold `pieces` 1 KB activation pieces: the rings, or the C tile
@@ -100,6 +100,7 @@ __device__ __forceinline__ void tile_multiply(uint8_t* a_ring, const ActLoads<PI
                                               uint8_t* bits_ring, __amdgpu_buffer_rsrc_t brsrc, int bgoff,
                                               BitsOffset boff, int kt0, int nk, bool multiply_first, int l,
                                               float4_t (&acc)[MI][2]) {
+  constexpr int WINDOW = MI < kWindow ? MI : kWindow;
   const LaneGeo g = lane_geo<K>(l & 15, l >> 4);
   auto issue_a = [&](int i, int kt) {
     uint8_t* st = a_ring + (i & (kARing - 1)) * act.stage;
@@ -135,7 +136,7 @@ __device__ __forceinline__ void tile_multiply(uint8_t* a_ring, const ActLoads<PI
     issue_a(i, last(i));
     issue_bits(i + 1, last(i + 1));
   }
-  half8_t bcur[2], bnext[2], av[kWindow];
+  half8_t bcur[2], bnext[2], av[WINDOW];
   uint32_t bw[2][2][2];
   __builtin_amdgcn_s_waitcnt(waitcnt_vm(2 * (PIECES + 1)));  // bundle 0 in (bundles 1 and 2 may be in flight)
   lds_barrier();
@@ -145,7 +146,7 @@ __device__ __forceinline__ void tile_multiply(uint8_t* a_ring, const ActLoads<PI
     bcur[jj] = decode_two_groups<K, CB>(bw[jj][0][0], bw[jj][0][1], bw[jj][1][0], bw[jj][1][1], g);
   read_bits(1, bw);
 #pragma unroll
-  for (int q = 0; q < kWindow; q++) av[q] = frags(0)[q * 64];
+  for (int q = 0; q < WINDOW; q++) av[q] = frags(0)[q * 64];
 
   // step i: the weights `cur` of the step, `next` those of step i + 1, decoded here from the words in bw, which then
   // take step i + 2's
@@ -168,8 +169,8 @@ __device__ __forceinline__ void tile_multiply(uint8_t* a_ring, const ActLoads<PI
     auto multiply = [&]() {
 #pragma unroll
       for (int mi = 0; mi < MI; mi++) {
-        const half8_t a = av[mi % kWindow];
-        av[mi % kWindow] = mi + kWindow < MI ? af[(mi + kWindow) * 64] : an[(mi + kWindow - MI) * 64];
+        const half8_t a = av[mi % WINDOW];
+        av[mi % WINDOW] = mi + WINDOW < MI ? af[(mi + WINDOW) * 64] : an[(mi + WINDOW - MI) * 64];
 #pragma unroll
         for (int jj = 0; jj < 2; jj++)
           acc[mi][jj] = __builtin_amdgcn_mfma_f32_16x16x32_f16(cur[jj], a, acc[mi][jj], 0, 0, 0);
