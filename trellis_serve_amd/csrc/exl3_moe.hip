@@ -613,7 +613,7 @@ static size_t align256(size_t v) { return (v + 255) & ~(size_t)255; }
 //   GEMVs: the experts' weights once per 16-64 slots (per 4.72 M weights, 128 experts at 2048 / 768 measured 111 us at 4
 //   slots per expert, 165 at 10, 230 at 16, 458 at 32, 1247 at 128), at least 2.4 us per slot of an expert (few experts);
 //   GEMMs: a tile per expert and column block, so at least one tile's k-steps per phase (the same layer 135-140 us up to
-//   10 slots per expert, 176 at 16, 189 at 32, 409 at 128; 8 experts at 4096 / 1536 about 103 us up to 64).
+//   10 slots per expert, 141-145 at 16, 189 at 32, 395-404 at 128; 8 experts at 4096 / 1536 about 103 us up to 64).
 // Tiles of 128 slots from 128 per expert (16 experts at 250: 70.8 us against 79.5 with tiles of 64; at 62: 58 against 50).
 static int moe_tile_rows(int slots, int E, int H, int I) {
   const int active = std::min(E, slots);
