@@ -9,6 +9,7 @@ import numpy as np
 import pytest
 import torch
 
+import kv_plan
 from oracle import exl3_oracle as orc
 
 pytestmark = pytest.mark.gpu
@@ -223,24 +224,38 @@ def test_kv_decode_random_shapes(case):
 
 
 # Batches where the split by lengths takes its different ways: one long sequence among short and empty ones (many
-# chunks beside whole sequences), more live sequences than workgroups aimed at (`crowded`), evenly spread lengths whose
-# equal share gives too many chunks, a table wider than every sequence, exactly 64 sequences and 65 (the fixed plan),
-# 16-head groups (4 waves), and chunk sizes at the multiples of the wave count.
-RAGGED = [([5000] + [0, 3, 40, 17] * 3, 10, 2, 512),
-          ([9000] + list(range(1, 64)), 8, 8, 600),
-          ([256 * (i + 1) for i in range(16)], 40, 8, 512),
-          ([64 * (i + 1) for i in range(64)], 8, 2, 300),
-          ([900 - 13 * i for i in range(65)], 4, 1, 64),
-          ([3000, 1, 0, 2047, 2048, 2049], 32, 2, 400),
-          ([1024, 1025, 1040, 128, 129], 5, 1, 66),
-          ([0, 0, 0], 8, 8, 100)]
+# chunks beside whole sequences), evenly spread lengths whose equal share gives too many chunks, a table wider than every
+# sequence, 63 and 64 sequences and 65 (the plan of the table), 16-head groups (4 waves), chunk sizes at the multiples of
+# the wave count, full tables (the plan of the table), and more live sequences than half the chunks aimed at, with one
+# chunk per sequence in the table's plan (as many partial states as sequences) and with two.
+RAGGED = [([5000] + [0, 3, 40, 17] * 3, 10, 2, 512, "share"),
+          ([9000] + list(range(1, 64)), 8, 8, 600, "fixed"),
+          ([9000] + list(range(1, 63)), 8, 8, 600, "share"),
+          ([256 * (i + 1) for i in range(16)], 40, 8, 512, "half"),
+          ([64 * (i + 1) for i in range(64)], 8, 2, 300, "half"),
+          ([900 - 13 * i for i in range(65)], 4, 1, 64, "fixed"),
+          ([3000, 1, 0, 2047, 2048, 2049], 32, 2, 400, "share"),
+          ([1024, 1025, 1040, 128, 129], 5, 1, 66, "fixed"),
+          ([0, 0, 0], 8, 8, 100, "fixed"),
+          ([4224], 40, 8, 264, "fixed"),
+          ([2048] * 15 + [1950], 10, 2, 128, "fixed"),
+          ([2700 - 17 * i for i in range(15)] + [637 - 17 * i for i in range(27)], 8, 8, 200, "share"),
+          ([1855] * 22 + [522] * 11, 8, 8, 200, "half"),
+          ([2498 - 3 * i for i in range(18)] + [305 - 3 * i for i in range(14)], 8, 8, 200, "most"),
+          ([8192] + [16 * (1 + i % 5) for i in range(39)], 8, 8, 512, "share"),
+          ([1077] * 18 + [1358] * 18, 8, 4, 200, "share"),
+          ([3462] * 3 + [1251] * 19, 8, 8, 300, "half"),
+          ([1551] + [732 - 3 * i for i in range(32)], 8, 4, 300, "most")]
 
 
 @pytest.mark.parametrize("bits", [8, 4])
-@pytest.mark.parametrize("lens,Hq,Hkv,max_pages", RAGGED, ids=[f"B{len(c[0])}-q{c[1]}-kv{c[2]}" for c in RAGGED])
-def test_kv_decode_split_by_lengths(lens, Hq, Hkv, max_pages, bits):
+@pytest.mark.parametrize("lens,Hq,Hkv,max_pages,way", RAGGED, ids=[f"B{len(c[0])}-q{c[1]}-kv{c[2]}-{i}"
+                                                                  for i, c in enumerate(RAGGED)])
+def test_kv_decode_split_by_lengths(lens, Hq, Hkv, max_pages, way, bits):
     """Ragged batches against the float64 closed form (the bar of this file: 2e-3), with empty sequences zero and
-    repeated calls bit-identical."""
+    repeated calls bit-identical.  The call writes exactly the partial states of the plan that the case is for, inside
+    its workspace."""
+    from trellis_serve_amd import _lib
     q, kc, vc, ks, vs, table = _case(len(lens) + Hq + bits, lens, Hq, Hkv, bits, max_pages=max_pages)
     sm = D ** -0.5
     first = _run(q, kc, vc, ks, vs, table, lens, bits, sm)
@@ -252,3 +267,23 @@ def test_kv_decode_split_by_lengths(lens, Hq, Hkv, max_pages, bits):
         nrel, mrel = _errs(y[live], ref)
         assert nrel <= 2e-3 and mrel <= 2e-3, (nrel, mrel)
     assert torch.equal(_run(q, kc, vc, ks, vs, table, lens, bits, sm), first)
+
+    plans = [kv_plan.split(lens, Hkv, Hq // Hkv, max_pages, ulps) for ulps in (-1, 0, 1)]
+    assert way in {p.way for p in plans}
+    lib = _lib.load()
+    need = lib.exl3_kv_decode_workspace_bytes(len(lens), Hq, Hkv, max_pages)
+    mark, guard = -7.5e30, 4096
+    ws = torch.full(((need + guard) // 4,), mark, dtype=torch.float32, device="cuda")
+    t = [torch.from_numpy(np.ascontiguousarray(a)).cuda() for a in (q, kc, vc, ks, vs, table, np.asarray(lens, np.int32))]
+    out = torch.empty_like(first)
+    p = [a.data_ptr() for a in t]
+    _lib.check(lib.exl3_kv_decode_attention(p[0], p[1], p[2], p[3], p[4], kc.shape[0], p[5], max_pages, p[6], len(lens), Hq,
+                                            Hkv, D, PAGE, bits, sm, out.data_ptr(), ws.data_ptr(), need,
+                                            torch.cuda.current_stream().cuda_stream), "kv")
+    assert torch.equal(out, first)
+    assert (ws[need // 4:] == mark).all()
+    states = len(lens) * kv_plan.fixed_plan(len(lens), Hkv, Hq // Hkv, max_pages).chunks
+    ml = ws[states * Hq * D:need // 4].view(states, Hq, 2)
+    written = (ml[:, :, 1] != mark)
+    assert (written.all(1) == written.any(1)).all()
+    assert int(written[:, 0].sum()) in {p.states for p in plans}, ([(p.way, p.states) for p in plans])

@@ -8,7 +8,7 @@
 //   page_table int32 [B][max_pages]; seq_lens int32 [B]; q fp16 [B][Hq][D]; out fp16 [B][Hq][D]; D = 128.
 //   Query head h reads KV head h / (Hq / Hkv).
 //
-// kv_decode_kernel: grid (Hkv, chunks of pages over the batch), W = 8 (or 4) waves.  Wave w takes pages w, w+W, ...
+// kv_decode_kernel: grid (chunks of pages, Hkv, sequences), W = 8 (or 4) waves.  Wave w takes pages w, w+W, ...
 // of its workgroup's chunk, with the next page's codes in flight while it works on the current one, and keeps an
 // online softmax for the G = Hq/Hkv query heads (G <= 16; MFMA columns G..15 are idle).  Per 16-token page --
 // exactly one 16-wide MFMA block, so the page's two scales are wave-uniform:
@@ -217,13 +217,17 @@ struct KvState {
 // `cp` pages, cp the batch's pages over the number of workgroups aimed at, so that a long sequence takes many chunks
 // and a short one a single chunk, which writes its output directly.  Measured against the fixed plan (a step of two
 // calls, 40 / 8 heads): 16 sequences of 256 .. 4096 tokens in an 8k table, 8 bits 71.4 -> 49.1 us; 7 sequences of
-// 4681 .. 32768 tokens, 4 bits 117-129 -> 76.6 us.  Deriving the plan costs 0.7-1.3 us per call (decode and merge), seen
-// where every sequence fills the table: 16 x 4k 8 bits 26.0 -> 27.3 us, one sequence of 32k 17.9 -> 18.9.
+// 4681 .. 32768 tokens, 4 bits 117-129 -> 76.6 us.
+// Where the fixed plan's longest chunk is no longer than that (sequences that fill their table, or lie close together),
+// the fixed plan stands: 26 sequences of 8 heads, 53-100 % of 7072 tokens, 8 bits 57.9 us by it, 63.7 split by lengths; 16
+// full sequences of 4k 26.6 -> 26.0, one of 4224 tokens 10.2 -> 8.7.  Having read the lengths costs 0.3-0.7 us per call
+// then (decode and merge; a kernel that does not read them takes 25.4 and 8.3).
 struct KvSplit {
-  int by_length;            // 1: the split by the lengths, aiming at `target` chunks per kv head and with room for
-  int batch, max_tokens;    // `slots` partial states per (kv head, query head)
-  int target, slots;
-  float inv_target, inv_slots;
+  int batch, max_tokens;
+  int target, slots;        // by lengths: aiming at `target` chunks per kv head, room for `slots` partial states per
+                            // (kv head, query head)
+  float inv_target, inv_slots, inv_heads;
+  float worth;              // by lengths where worth * the longest chunk of the fixed plan exceeds the chunks by length
   int chunk_pages, chunks;  // the fixed plan: `chunks` chunks of chunk_pages pages per sequence
 };
 
@@ -251,11 +255,11 @@ __device__ __forceinline__ int kv_per(int pages, int chunks, int waves) {
   return (int)(((unsigned)(pages + chunks - 1) / (unsigned)chunks + waves - 1) & -(unsigned)waves);
 }
 
-__device__ __forceinline__ KvBatch kv_batch(const KvSplit& s, const int* __restrict__ seq_lens, int waves) {
+// The plan by lengths; false: the fixed plan (only len and pages are set)
+__device__ __forceinline__ bool kv_batch(const KvSplit& s, const int* __restrict__ seq_lens, int waves, KvBatch& k) {
   const int lane = threadIdx.x & 63;
-  asm volatile("" ::"s"(s.by_length), "s"(s.batch), "s"(s.max_tokens), "s"(s.target), "s"(s.slots), "s"(s.inv_target),
-               "s"(s.inv_slots), "s"(seq_lens));
-  KvBatch k;
+  asm volatile("" ::"s"(s.batch), "s"(s.max_tokens), "s"(s.target), "s"(s.slots), "s"(s.inv_target), "s"(s.inv_slots),
+               "s"(s.worth), "s"(s.chunks), "s"(s.chunk_pages), "s"(s.inv_heads), "s"(seq_lens));
   k.len = max(min(seq_lens[min(lane, s.batch - 1)], s.max_tokens), 0);
   k.len = lane < s.batch ? k.len : 0;
   k.pages = (k.len + kPage - 1) / kPage;
@@ -267,6 +271,10 @@ __device__ __forceinline__ KvBatch kv_batch(const KvSplit& s, const int* __restr
   auto scan = [&](int v) { return s.batch == 1 ? __builtin_amdgcn_readfirstlane(v) : wave_scan(v); };
   auto total_of = [&](int sums) { return __builtin_amdgcn_readlane(sums, 63); };
   const float total = (float)total_of(scan(k.pages));
+  // the fixed plan's longest chunk, as it weighs, against an equal share of the batch
+  const float longest = (float)min(k.pages, s.chunk_pages) * s.worth;
+  auto any = [](bool b) { return __builtin_amdgcn_ballot_w64(b) != 0; };
+  if (!any(longest > total * fmaxf(s.inv_target, s.inv_slots))) return false;
   const int live = __builtin_popcountll(__builtin_amdgcn_ballot_w64(k.pages > 0));
   // Chunks of an equal share of the batch, if that gives no more chunks than workgroups aimed at (one per CU: a CU
   // with two takes twice as long) and the partial states fit.  Each sequence's last chunk is short, so a ragged batch
@@ -275,54 +283,54 @@ __device__ __forceinline__ KvBatch kv_batch(const KvSplit& s, const int* __restr
   // three times the mean over the slots always fit (fewer than 2 n / cp + 1 chunks in a split sequence of n pages).
   const bool crowded = 2 * live > s.target;
   auto fits = [&](int sums) { return (sums >> 16) <= s.slots && (crowded || (sums & 0xFFFF) <= s.target); };
-  const int share = up(total * s.inv_target - 0.5f);
-  k.chunks = chunks_of(share);
+  const int share = up(__builtin_fmaf(total, s.inv_target, -0.5f));
+  int cp = share;
+  k.chunks = chunks_of(cp);
   k.sums = scan(both(k.chunks));
   if (!fits(total_of(k.sums))) {
     const float room = (float)max(min(s.target, s.slots) - live, 1);  // chunks left when each sequence wastes one
-    auto leaving = [&](float part) { return up(total * __builtin_amdgcn_rcpf(room + part * live)); };
+    auto leaving = [&](float part) { return up(total * __builtin_amdgcn_rcpf(__builtin_fmaf(part, (float)live, room))); };
     const int half = crowded ? share + share / 2 : leaving(0.5f), most = crowded ? 2 * share : leaving(0.25f);
     const int last = crowded ? up(fmaxf(3.f * total * s.inv_slots, 2.f * share)) : leaving(0.f);
     const int b = wave_total(both(chunks_of(half))), c = wave_total(both(chunks_of(most)));
-    k.chunks = chunks_of(fits(b) ? half : fits(c) ? most : last);
+    cp = fits(b) ? half : fits(c) ? most : last;
+    k.chunks = chunks_of(cp);
     k.sums = wave_scan(both(k.chunks));
   }
-  return k;
+  // with a CU for every workgroup of the fixed plan, chunks by lengths may still come out as long (unless every sequence
+  // ends in its first chunk there, whose state would take the merge's detour)
+  return s.slots > s.target || any(longest > (float)cp) || !any(k.pages > s.chunk_pages);
 }
 
 // A workgroup's chunk: pages [p0, p1) of sequence b of length len; slot: its partial state, -1 when it is the whole
 // sequence; b = -1 past the last chunk.
 struct KvChunk {
-  int b, len, p0, p1, slot;
+  int hk, b, len, p0, p1, slot;
 };
 
-__device__ __forceinline__ KvChunk kv_chunk_at(const KvSplit& s, const int* __restrict__ seq_lens, int index,
-                                               int waves) {
-  if (!s.by_length) {
-    const int b = s.chunks == 1 ? index : index / s.chunks, i = index - b * s.chunks;
-    return KvChunk{b, min(seq_lens[b], s.max_tokens), i * s.chunk_pages, (i + 1) * s.chunk_pages,
-                   s.chunks > 1 ? index : -1};
-  }
-  const KvBatch k = kv_batch(s, seq_lens, waves);
-  if (index >= (__builtin_amdgcn_readlane(k.sums, 63) & 0xFFFF)) return KvChunk{-1, 0, 0, 0, -1};
+// The fixed plan's workgroups are (chunk, kv head, sequence).
+__device__ __forceinline__ KvChunk kv_fixed_chunk(const KvSplit& s, int len) {
+  const int i = blockIdx.x, b = blockIdx.z;
+  return KvChunk{(int)blockIdx.y, b, len, i * s.chunk_pages, (i + 1) * s.chunk_pages,
+                 s.chunks > 1 ? b * s.chunks + i : -1};
+}
+
+// By lengths the kv head is the fast index of a workgroup's linear id and the chunk's number the slow one: workgroups
+// past the last chunk then come last and take no CU from a chunk (with the chunk fast, 16 x 4k 26 -> 37 us).
+__device__ __forceinline__ KvChunk kv_chunk_by_length(const KvSplit& s, int Hkv, int waves, const KvBatch& k) {
+  const int id = blockIdx.x + s.chunks * (blockIdx.y + Hkv * blockIdx.z);
+  const int index = __builtin_amdgcn_readfirstlane((int)(((float)id + 0.5f) * s.inv_heads));  // id / Hkv
+  if (index >= (__builtin_amdgcn_readlane(k.sums, 63) & 0xFFFF)) return KvChunk{0, -1, 0, 0, 0, -1};
   const int at = __builtin_popcountll(__builtin_amdgcn_ballot_w64((k.sums & 0xFFFF) <= index));
   const int pages = __builtin_amdgcn_readlane(k.pages, at), chunks = __builtin_amdgcn_readlane(k.chunks, at);
   const int sums = __builtin_amdgcn_readlane(k.sums, at);
-  const int i = index - ((sums & 0xFFFF) - chunks);
+  const int c = index - ((sums & 0xFFFF) - chunks);
   const int per = chunks == 1 ? pages : kv_per(pages, chunks, waves);
-  return KvChunk{at, __builtin_amdgcn_readlane(k.len, at), i * per, (i + 1) * per,
-                 chunks > 1 ? (sums >> 16) - chunks + i : -1};
+  return KvChunk{id - index * Hkv, at, __builtin_amdgcn_readlane(k.len, at), c * per, (c + 1) * per,
+                 chunks > 1 ? (sums >> 16) - chunks + c : -1};
 }
 
-// The chunks of sequence b for the merge: their count, and the first one's partial state
-__device__ __forceinline__ int2 kv_chunks_at(const KvSplit& s, const int* __restrict__ seq_lens, int b, int waves) {
-  if (!s.by_length) return int2{s.chunks, b * s.chunks};
-  const KvBatch k = kv_batch(s, seq_lens, waves);
-  const int chunks = __builtin_amdgcn_readlane(k.chunks, b);
-  return int2{chunks, (__builtin_amdgcn_readlane(k.sums, b) >> 16) - chunks};
-}
-
-template <int BITS, int DEPTH, int WAVES>
+template <int BITS, int DEPTH, int WAVES, bool BY_LENGTH>
 __global__ __launch_bounds__(WAVES * 64) void kv_decode_kernel(
     const _Float16* __restrict__ q, const uint8_t* kc, const uint8_t* vc, const uint16_t* ksc, const uint16_t* vsc,
     int num_pages,
@@ -331,12 +339,22 @@ __global__ __launch_bounds__(WAVES * 64) void kv_decode_kernel(
     _Float16* __restrict__ out) {
   constexpr int ROW = KvRegs<BITS>::ROW;
   extern __shared__ float red[];  // [WAVES][G][D + 1] then [WAVES][G][2]
-  const int hk = blockIdx.x;
-  const KvChunk ch = kv_chunk_at(split, seq_lens, blockIdx.y, WAVES);
-  if (ch.b < 0) return;
-  const int b = ch.b, L = ch.len;
-  const int G = Hq / Hkv;
   const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  KvChunk ch;
+  if constexpr (BY_LENGTH) {
+    KvBatch k;
+    if (kv_batch(split, seq_lens, WAVES, k)) {
+      ch = kv_chunk_by_length(split, Hkv, WAVES, k);
+      if (ch.b < 0) return;
+    } else {
+      if ((int)blockIdx.z >= split.batch) return;
+      ch = kv_fixed_chunk(split, __builtin_amdgcn_readlane(k.len, blockIdx.z));
+    }
+  } else {
+    ch = kv_fixed_chunk(split, min(seq_lens[blockIdx.z], split.max_tokens));
+  }
+  const int hk = ch.hk, b = ch.b, L = ch.len;
+  const int G = Hq / Hkv;
   const int l = threadIdx.x & 63;
   const int n = l & 15, g = l >> 4;
 
@@ -444,6 +462,7 @@ __global__ __launch_bounds__(WAVES * 64) void kv_decode_kernel(
 // out[b][h] = sum_c 2^(m_c - M) O_c / sum_c 2^(m_c - M) l_c.  One workgroup per query head; wave w folds chunks
 // w, w+4, ... into a running (M, L, O) (lane: dims 2l, 2l+1), then the 4 waves combine in LDS.  Fixed order.
 // A sequence of one chunk has its output already; an empty sequence gets zeros.
+template <bool BY_LENGTH>
 __global__ __launch_bounds__(kMergeWaves * 64) void kv_merge_kernel(const float* __restrict__ part_o,
                                                        const float* __restrict__ part_ml, int Hq, int Hkv,
                                                        const int* __restrict__ seq_lens, KvSplit split, int waves,
@@ -453,13 +472,19 @@ __global__ __launch_bounds__(kMergeWaves * 64) void kv_merge_kernel(const float*
   const int h = blockIdx.x, b = blockIdx.y;
   const int G = Hq / Hkv, hk = h / G, q = h - hk * G;
   const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), l = threadIdx.x & 63;
-  const int2 cs = kv_chunks_at(split, seq_lens, b, waves);
-  const int chunks = cs.x;
-  if (chunks == 1) return;
+  int chunks = split.chunks, state0 = b * split.chunks;  // the sequence's chunks, and its first partial state
+  if constexpr (BY_LENGTH) {
+    KvBatch k;
+    if (kv_batch(split, seq_lens, waves, k)) {
+      chunks = __builtin_amdgcn_readlane(k.chunks, b);
+      state0 = (__builtin_amdgcn_readlane(k.sums, b) >> 16) - chunks;
+    }
+    if (chunks == 1) return;
+  }
   float M = -INFINITY, L = 0.f, a0 = 0.f, a1 = 0.f;
 #pragma unroll 4
   for (int c = w; c < chunks; c += kMergeWaves) {
-    const size_t slot = ((size_t)(cs.y + c) * Hkv + hk) * G + q;
+    const size_t slot = ((size_t)(state0 + c) * Hkv + hk) * G + q;
     const float mc = part_ml[slot * 2], lc = part_ml[slot * 2 + 1];
     const float2 oc = *reinterpret_cast<const float2*>(part_o + slot * kHeadDim + 2 * l);
     const float mn = fmaxf(M, mc);
@@ -565,18 +590,21 @@ extern "C" int exl3_kv_decode_attention(const void* q, const void* k_cache, cons
   const float qk_scale = sm_scale * 1.4426950408889634f;  // logits in base 2
   const size_t lds = (size_t)plan.waves * G * (kHeadDim + 1 + 2) * sizeof(float);
   hipStream_t st = as_stream(stream);
-  // The split by lengths, with the merge launch, unless one chunk per sequence needs no merge and either the table is
-  // short (8 pages per wave) or the pairs fill the GPU twice; batches past 64 sequences keep the fixed plan, and so do
-  // tables whose fixed chunks are one page per wave already (a 1.1 us longer start for nothing).
-  const bool by_length = batch <= 64 && plan.chunk_pages > plan.waves &&
-                         !(chunks == 1 && (max_pages <= 8 * plan.waves || (long)batch * num_kv_heads >= 512));
+  // The split by lengths, with the merge launch, for up to 64 sequences, unless the fixed plan's chunks are one page per
+  // wave, or one chunk per sequence needs no merge and either the table is short (16 pages per wave) or the pairs fill
+  // the GPU twice.
   const int target = (kv_target(plan.waves) + num_kv_heads - 1) / num_kv_heads, slots = batch * chunks;
-  const KvSplit split{by_length, batch, max_pages * kPage, target, slots, 1.0f / target, 1.0f / slots, plan.chunk_pages,
-                      chunks};
-  // by lengths: at most `slots` chunks of split sequences, and one for every other sequence.  The kv head is the fast
-  // index: workgroups past the last chunk then come last and take no CU from a chunk (with the chunk fast, 16 x 4k
-  // 26 -> 37 us), and the heads of a page, adjacent in memory, are read together.
-  const dim3 grid(num_kv_heads, by_length ? slots + batch : slots);
+  const bool by_length = batch <= 64 && plan.chunk_pages > plan.waves &&
+                         !(chunks == 1 && (max_pages <= 16 * plan.waves || (long)batch * num_kv_heads >= 512));
+  // How the fixed plan's longest chunk weighs, fitted at 330 random batches: with a CU for every workgroup of it, chunks by
+  // lengths have to be shorter by a seventh (8 sequences, 8 heads, 88 pages for 96: 17.3 us by the fixed plan, 20.2 by
+  // lengths); where some CUs work on two they win also when longer (14 sequences, 8 heads, 336 workgroups of up to 248
+  // pages, share 276: 66 and 53 us); with more than half as many sequences as aimed at both plans have such CUs.
+  const float worth = slots <= target ? 0.87f : 2 * batch <= target ? 1.6f : 1.1f;
+  const KvSplit split{batch,           max_pages * kPage,   target, slots,            1.0f / target,
+                      1.0f / slots,    1.0f / num_kv_heads, worth,  plan.chunk_pages, chunks};
+  // by lengths: at most `slots` chunks of split sequences, and one for every other sequence
+  const dim3 grid(chunks, num_kv_heads, by_length ? batch + (batch + chunks - 1) / chunks : batch);
   auto qp = static_cast<const _Float16*>(q);
   auto kp = static_cast<const uint8_t*>(k_cache);
   auto vp = static_cast<const uint8_t*>(v_cache);
@@ -588,20 +616,22 @@ extern "C" int exl3_kv_decode_attention(const void* q, const void* k_cache, cons
     const char* e = getenv("EXL3_KV_DEPTH");
     return e ? std::min(5, std::max(2, atoi(e))) : 2;
   }();
-  using Kern = decltype(&kv_decode_kernel<8, 2, 4>);
-  static const Kern table[2][2][4] = {
-      {{kv_decode_kernel<4, 2, 4>, kv_decode_kernel<4, 3, 4>, kv_decode_kernel<4, 4, 4>, kv_decode_kernel<4, 5, 4>},
-       {kv_decode_kernel<8, 2, 4>, kv_decode_kernel<8, 3, 4>, kv_decode_kernel<8, 4, 4>, kv_decode_kernel<8, 5, 4>}},
-      {{kv_decode_kernel<4, 2, 8>, kv_decode_kernel<4, 3, 8>, kv_decode_kernel<4, 4, 8>, kv_decode_kernel<4, 5, 8>},
-       {kv_decode_kernel<8, 2, 8>, kv_decode_kernel<8, 3, 8>, kv_decode_kernel<8, 4, 8>, kv_decode_kernel<8, 5, 8>}}};
-  table[plan.waves == 8][bits == 8][depth - 2]<<<grid, plan.waves * 64, lds, st>>>(
+  using Kern = decltype(&kv_decode_kernel<8, 2, 4, false>);
+#define EXL3_KV_DEPTHS(B, W, S) \
+  {kv_decode_kernel<B, 2, W, S>, kv_decode_kernel<B, 3, W, S>, kv_decode_kernel<B, 4, W, S>, kv_decode_kernel<B, 5, W, S>}
+#define EXL3_KV_SPLITS(B, W) {EXL3_KV_DEPTHS(B, W, false), EXL3_KV_DEPTHS(B, W, true)}
+  static const Kern table[2][2][2][4] = {{EXL3_KV_SPLITS(4, 4), EXL3_KV_SPLITS(8, 4)},
+                                         {EXL3_KV_SPLITS(4, 8), EXL3_KV_SPLITS(8, 8)}};
+#undef EXL3_KV_SPLITS
+#undef EXL3_KV_DEPTHS
+  table[plan.waves == 8][bits == 8][by_length][depth - 2]<<<grid, plan.waves * 64, lds, st>>>(
       qp, kp, vp, ksp, vsp, num_pages, pt, max_pages, sl, num_q_heads, num_kv_heads, qk_scale, split,
       part_o, part_ml, static_cast<_Float16*>(out));
   EXL3_CHECK_LAUNCH();
   if (by_length || chunks > 1) {
-    kv_merge_kernel<<<dim3(num_q_heads, batch), kMergeWaves * 64, 0, st>>>(part_o, part_ml, num_q_heads,
-                                                                           num_kv_heads, sl, split, plan.waves,
-                                                                           static_cast<_Float16*>(out));
+    auto merge = by_length ? kv_merge_kernel<true> : kv_merge_kernel<false>;
+    merge<<<dim3(num_q_heads, batch), kMergeWaves * 64, 0, st>>>(part_o, part_ml, num_q_heads, num_kv_heads, sl, split, plan.waves,
+                                              static_cast<_Float16*>(out));
     EXL3_CHECK_LAUNCH();
   }
   return EXL3_OK;
