@@ -610,26 +610,40 @@ static size_t align256(size_t v) { return (v + 255) & ~(size_t)255; }
 
 // Whether a call takes the expert decode-GEMMs (exl3_moe_gemm.hip), and their tile height in slots; 0: the expert GEMVs.
 // The lower of two estimates (us), fitted at 8-128 experts, hidden 1024-4096, inter 512-1536 and 2-128 slots per expert:
-//   GEMVs: the experts' weights once per 16-64 slots (per 4.72 M weights, 128 experts at 2048 / 768 measured 111 us at 4
-//   slots per expert, 165 at 10, 230 at 16, 458 at 32, 1247 at 128), at least 2.4 us per slot of an expert (few experts);
-//   GEMMs: a tile per expert and column block, so at least one tile's k-steps per phase (the same layer 135-140 us up to
-//   10 slots per expert, 141-145 at 16, 189 at 32, 395-404 at 128; 8 experts at 4096 / 1536 about 103 us up to 64).
+//   GEMVs: the experts' weights once per 16-64 slots, at least 2.4 us per slot of an expert (few experts);
+//   GEMMs: a tile per expert and column block, so at least one tile's k-steps per phase (128 experts at 2048 / 768 and
+//   K = 3, GEMVs against GEMMs: 149 and 125 us at 9.5 slots per expert, 199 and 133 at 16, 421 and 181 at 32, 795 and 256
+//   at 64; 8 experts at 4096 / 1536 about 103 us up to 64 slots).
+// Where the GEMVs read the weights once (up to about 20 slots per expert, in passes of 32), wide experts cost them less
+// than that (8 experts, 4096 / 14336, 16 slots: 272 us against 379), so past 2048 columns the GEMMs have to win a second
+// comparison of both forms, by bitrate, width and slots, fitted at 7 such layer shapes of 8-128 experts, K = 2, 3 and 8.
+// It leaves none of their calls measured more than 4 % behind the GEMVs (27 of 260 were, by up to 43 %, without it).
+// Narrower experts stay with the first: their GEMVs' time follows the experts that take one pass more, up to 56 % either
+// side of any estimate by the mean (60 experts, 1408 / 512, 11 slots, K = 2: 88 us, the GEMMs 56).
 // Tiles of 128 slots from 128 per expert (16 experts at 250: 70.8 us against 79.5 with tiles of 64; at 62: 58 against 50).
-static int moe_tile_rows(int slots, int E, int H, int I) {
+static int moe_tile_rows(int slots, int E, int H, int I, int K_gu, int K_dn) {
   const int active = std::min(E, slots);
   const double mean = (double)slots / active, units = active * (3.0 * H * I / 4718592);
-  const double gemv = 22 + std::max(units * (0.5 + 0.06 * mean), 2.4 * mean);
   const int rows = mean >= 128 ? 128 : 64;
   const double tiles = active * std::ceil(mean / rows);
-  auto phase = [&](int ksteps, int ncb) { return ksteps * 0.48 * std::max(1.0, tiles * ncb / 256); };
-  const double gemm = 19 + phase(H / 32, I / 128) + phase(I / 32, (H + 255) / 256);
-  return gemm < gemv ? rows : 0;
+  // us per k-step of the GEMMs, at one round or less of the CUs and per round
+  auto gemms = [&](double least, double per_round) {
+    auto phase = [&](int ksteps, int ncb) { return ksteps * std::max(least, per_round * tiles * ncb / 256); };
+    return phase(H / 32, I / 128) + phase(I / 32, (H + 255) / 256);
+  };
+  if (19 + gemms(0.48, 0.48) >= 22 + std::max(units * (0.5 + 0.06 * mean), 2.4 * mean)) return 0;
+  if (I > 2048 && mean + 2.5 * std::sqrt(mean) <= 32) {
+    const double K = (2.0 * K_gu + K_dn) / 3;
+    const double gemvs = 14 + std::max(units * (0.25 + 0.05 * K + mean * (0.021 + 0.031 * 1024 / I)), 2.55 * mean);
+    if (24 + gemms(0.445, 0.2 + 0.0045 * mean + 0.015 * K) >= gemvs) return 0;
+  }
+  return rows;
 }
 
 static MoePlan moe_plan(int tokens, int top_k, int E, int H, int I, int K_gu, int K_dn) {
   MoePlan p{};
   const int slots = tokens * top_k;
-  p.tile_rows = moe_tile_rows(slots, E, H, I);
+  p.tile_rows = moe_tile_rows(slots, E, H, I, K_gu, K_dn);
   if (p.tile_rows > 0) {
     size_t o = kCounterBytes;  // unused here, but every workspace starts with it
     p.off_sorted = o; o = align256(o + (size_t)slots * sizeof(int2));
