@@ -179,10 +179,11 @@ typedef struct exl3_moe_weights {
   const void* down_svh;     /* fp16 [E][H] */
 } exl3_moe_weights;
 
-/* Workspace bytes of exl3_moe_forward (split counters, routing lists, fp16 rotated inputs, g|u and down rows, fp32
- * partials).  The
- * counter region (EXL3_WORKSPACE_COUNTER_BYTES, holding num_experts * (2 inter + hidden) / 128 counters) must be
- * zero before the first use; every call leaves it zero. */
+/* Workspace bytes that serve exl3_moe_forward with up to `tokens` tokens (split counters, routing lists, fp16 rotated
+ * inputs, g|u and down rows, fp32 partials): never less for more tokens, so a buffer sized for a caller's most tokens
+ * serves every smaller call.  A call itself is refused only below what its own token count needs.  The counter region
+ * (EXL3_WORKSPACE_COUNTER_BYTES, holding num_experts * (2 inter + hidden) / 128 counters) must be zero before the first
+ * use; every call leaves it zero. */
 size_t exl3_moe_workspace_bytes(int tokens, int top_k, int num_experts, int hidden, int inter, int K_gate_up,
                                 int K_down);
 /* y[t] = sum_j w[t, j] * down_e(fp16(silu(gate_e(x[t])) * up_e(x[t]))), e = topk_ids[t, j]; every linear is an EXL3
@@ -208,8 +209,7 @@ typedef struct exl3_moe_class {
   int K_gate_up, K_down;
 } exl3_moe_class;
 
-/* Workspace bytes of exl3_moe_forward_classes (the same layout as exl3_moe_forward's, with one k-split plan shared
- * by the classes).  classes_host holds nclasses entries (only their bitrates are read). */
+/* Workspace bytes of exl3_moe_forward_classes (as exl3_moe_workspace_bytes; one k-split plan is shared by the classes).  classes_host holds nclasses entries (only their bitrates are read). */
 size_t exl3_moe_classes_workspace_bytes(int tokens, int top_k, int num_experts, int hidden, int inter, int nclasses,
                                         const exl3_moe_class* classes_host);
 /* exl3_moe_forward for a layer whose experts come in up to EXL3_MOE_MAX_CLASSES K classes; every expert id in

@@ -16,10 +16,9 @@ def _up(v: int) -> int:
 
 
 def gemm_bytes(tokens: int, top_k: int, E: int, H: int, I: int) -> int:
-    """The workspace of the sorted expert GEMMs."""
+    """The workspace of the sorted expert GEMMs (tiles counted at 64 slots)."""
     slots = tokens * top_k
-    rows = 128 if slots >= 128 * min(E, slots) else 64
-    return (COUNTERS + _up(8 * slots) + _up(8) + _up(16 * (slots // rows + min(E, slots))) + _up(2 * slots * H)
+    return (COUNTERS + _up(8 * slots) + _up(8) + _up(16 * (slots // 64 + min(E, slots))) + _up(2 * slots * H)
             + _up(4 * slots * H) + _up(2 * slots * I))
 
 

@@ -579,16 +579,20 @@ struct MoePhase {
   int splits, chunks;
 };
 
+static int moe_target_wgs() {  // EXL3_MOE_TARGET_WGS: another workgroup target (A/B measurements)
+  static const int target = [] {
+    const char* e = getenv("EXL3_MOE_TARGET_WGS");
+    return e ? std::max(1, atoi(e)) : 2048;
+  }();
+  return target;
+}
+
 static MoePhase moe_phase_plan(int slots, int rows, int nblk, int k, int K, int nt) {
   const int NB = nt / 8;
   const int C = (k / 128 + NB - 1) / NB;
   const double per_split = (double)slots * 8.0 / ((double)rows * k * std::max(K, 1) / 8.0);
   const int cap = std::max(1, (int)(0.25 / per_split));
-  static const int target = [] {  // EXL3_MOE_TARGET_WGS: another workgroup target (A/B measurements)
-    const char* e = getenv("EXL3_MOE_TARGET_WGS");
-    return e ? std::max(1, atoi(e)) : 2048;
-  }();
-  const int want = std::max(1, (target + rows * nblk - 1) / (rows * nblk));
+  const int want = std::max(1, (moe_target_wgs() + rows * nblk - 1) / (rows * nblk));
   const int s = std::min(C, std::min(cap, want));
   MoePhase ph{};
   ph.chunks = (C + s - 1) / s;
@@ -648,7 +652,8 @@ static MoePlan moe_plan(int tokens, int top_k, int E, int H, int I, int K_gu, in
     size_t o = kCounterBytes;  // unused here, but every workspace starts with it
     p.off_sorted = o; o = align256(o + (size_t)slots * sizeof(int2));
     p.off_totals = o; o = align256(o + 8);
-    p.off_tiles = o; o = align256(o + (size_t)moe_gemm_max_tiles(slots, E, p.tile_rows) * sizeof(MoeTile));
+    // counted at 64 slots whatever the height, so that more tokens never need less
+    p.off_tiles = o; o = align256(o + (size_t)moe_gemm_max_tiles(slots, E, 64) * sizeof(MoeTile));
     p.off_dn = o; o = align256(o + (size_t)slots * H * 2);
     p.off_pre_in = o; o = align256(o + (size_t)2 * slots * H * 2);
     p.off_pre_dn = o; o = align256(o + (size_t)slots * I * 2);
@@ -728,13 +733,58 @@ struct MoeClass {
 };
 
 // The classes share one plan: its k-splits come from the smallest bitrates (the partial-size cap is tightest there).
-static MoePlan moe_plan_of(int tokens, int top_k, int E, int H, int I, const MoeClass* cls, int ncls) {
-  int K_gu = cls[0].K_gu, K_dn = cls[0].K_dn;
-  for (int c = 1; c < ncls; c++) {
-    K_gu = std::min(K_gu, cls[c].K_gu);
-    K_dn = std::min(K_dn, cls[c].K_dn);
+struct MoeBits {
+  int K_gu, K_dn;
+};
+static MoeBits moe_least_bits(const MoeClass* cls, int ncls) {
+  MoeBits b{cls[0].K_gu, cls[0].K_dn};
+  for (int c = 1; c < ncls; c++) b = MoeBits{std::min(b.K_gu, cls[c].K_gu), std::min(b.K_dn, cls[c].K_dn)};
+  return b;
+}
+
+// ---- one workspace for every call of up to `tokens` tokens -----------------------------------------------------------
+// A plan's own need (moe_plan) goes down where the k-splits drop and where the GEMMs take over, so the reported size is
+// a bound over all smaller calls; moe_forward_impl holds a call to its own plan's need only.
+
+// Slots from which no call stays with the GEMVs: where moe_tile_rows' estimate of the GEMMs, its maxima taken as sums and
+// its tiles as E (mean / 64 + 1), falls below that of the GEMVs (whose slope in `mean` is the larger one for all shapes)
+static double moe_gemv_most_slots(int E, int H, int I) {
+  const double units = E * (3.0 * H * I / 4718592), steps = 0.48 * (H / 32 + I / 32);
+  const double rounds = 0.48 * E / 256 * ((double)(H / 32) * (I / 128) + (double)(I / 32) * ((H + 255) / 256));
+  const double mean = (steps + rounds - 3 - 0.5 * units) / (0.06 * units - rounds / 64);
+  return std::ceil(E * std::max(21.0, mean));  // and up to 20.9 per expert where it compares once more
+}
+
+// splits * slots of one GEMV phase at most, over all calls of up to `slots` slots.  splits is at most the number of chunks
+// of k, what fills the workgroup target, and the cap on the partials (never below one): with fewer slots than experts
+// (rows = slots) K k / 256 and target / (slots nblk) + 1, else E K k / 256 / slots and the target's share of E experts.
+static size_t moe_phase_most(size_t slots, size_t E, size_t nblk, size_t k, size_t K, size_t nt) {
+  const size_t NB = nt / 8, C = (k / 128 + NB - 1) / NB, target = moe_target_wgs();
+  const size_t few = std::min(slots, E);
+  size_t most = std::min(few * std::min(C, std::max<size_t>(1, k * K / 256)), target / nblk + 1 + few);
+  if (slots >= E)
+    most = std::max(most, std::min(slots * std::min(C, (target + E * nblk - 1) / (E * nblk)),
+                                   std::max(slots, E * k * K / 256 + 1)));
+  return most;
+}
+
+static size_t moe_workspace_bytes(int tokens, int top_k, int E, int H, int I, int K_gu, int K_dn) {
+  const size_t one = moe_plan(1, top_k, E, H, I, K_gu, K_dn).total;
+  if (tokens == 1) return one;
+  const size_t slots = (size_t)tokens * top_k, few = std::min((double)slots, moe_gemv_most_slots(E, H, I));
+  const size_t partial = std::max(moe_phase_most(few, E, 2 * I / 128, H, std::max(K_gu, 1), 16) * 2 * I,
+                                  moe_phase_most(few, E, H / 128, I, std::max(K_dn, 1), 16) * H) * 4;
+  // the GEMVs' regions (moe_plan), which the GEMMs' stay below with the same slots
+  const size_t gemvs = kCounterBytes + 2 * align256((size_t)E * 4) + 256 + align256((size_t)E * few * 4) +
+                       align256(few * H * 2) + align256(2 * few * H * 2) + align256(few * I * 2) + align256(partial);
+  size_t most = std::max(one, gemvs);
+  if (slots > few) {
+    const size_t gemms = kCounterBytes + align256(slots * sizeof(int2)) + 256 +
+                         align256((slots / 64 + std::min<size_t>(E, slots)) * sizeof(MoeTile)) + align256(slots * H * 2) +
+                         align256(2 * slots * H * 2) + align256(slots * I * 2);
+    most = std::max(most, gemms);
   }
-  return moe_plan(tokens, top_k, E, H, I, K_gu, K_dn);
+  return most;
 }
 
 static bool moe_shape_ok(int tokens, int top_k, int E, int H, int I) {
@@ -779,7 +829,8 @@ static int moe_forward_impl(const char* what, const void* x, int x_bf16, int tok
   if (tokens == 0) return EXL3_OK;
   const int slots = tokens * top_k;
   EXL3_CHECK_ARG((int64_t)slots * std::max(2 * inter, hidden) <= INT32_MAX / 4, "%s: too many slots", what);
-  const MoePlan p = moe_plan_of(tokens, top_k, num_experts, hidden, inter, cls, ncls);
+  const MoeBits bits = moe_least_bits(cls, ncls);
+  const MoePlan p = moe_plan(tokens, top_k, num_experts, hidden, inter, bits.K_gu, bits.K_dn);
   EXL3_CHECK_ARG(workspace && workspace_bytes >= p.total, "%s: workspace %zu bytes, need %zu", what, workspace_bytes,
                  p.total);
   uint8_t* ws = static_cast<uint8_t*>(workspace);
@@ -905,7 +956,7 @@ using namespace exl3;
 extern "C" size_t exl3_moe_workspace_bytes(int tokens, int top_k, int num_experts, int hidden, int inter,
                                            int K_gate_up, int K_down) {
   if (!moe_shape_ok(tokens, top_k, num_experts, hidden, inter)) return 0;
-  return moe_plan(tokens, top_k, num_experts, hidden, inter, K_gate_up, K_down).total;
+  return moe_workspace_bytes(tokens, top_k, num_experts, hidden, inter, K_gate_up, K_down);
 }
 
 extern "C" size_t exl3_moe_classes_workspace_bytes(int tokens, int top_k, int num_experts, int hidden, int inter,
@@ -916,7 +967,8 @@ extern "C" size_t exl3_moe_classes_workspace_bytes(int tokens, int top_k, int nu
   MoeClass cls[EXL3_MOE_MAX_CLASSES];
   for (int c = 0; c < nclasses; c++)
     cls[c] = MoeClass{nullptr, nullptr, 0, classes_host[c].K_gate_up, classes_host[c].K_down};
-  return moe_plan_of(tokens, top_k, num_experts, hidden, inter, cls, nclasses).total;
+  const MoeBits b = moe_least_bits(cls, nclasses);
+  return moe_workspace_bytes(tokens, top_k, num_experts, hidden, inter, b.K_gu, b.K_dn);
 }
 
 extern "C" int exl3_moe_forward(const void* x, int x_bf16, int tokens, int hidden, const void* topk_ids,

@@ -164,9 +164,8 @@ def reserve_moe(device: torch.device, max_tokens: int, top_k: int, num_experts: 
     """Reserves the MoE workspace for every call of up to `max_tokens` tokens."""
     lib = _lib.load()
     dev = torch.device("cuda", _dev_index(device))
-    need = _max_need(lambda t: lib.exl3_moe_workspace_bytes(t, top_k, num_experts, hidden, inter, K_gate_up,
-                                                            K_down), max_tokens)
-    _ws("moe", dev).reserve(dev, need)
+    _ws("moe", dev).reserve(dev, lib.exl3_moe_workspace_bytes(max(1, int(max_tokens)), top_k, num_experts, hidden, inter,
+                                                              K_gate_up, K_down))
 
 
 def moe_align_capacity(slots: int, num_experts: int, block: int) -> tuple[int, int]:
