@@ -120,8 +120,8 @@ size_t exl3_linear_workspace_bytes(int rows, int k, int n_total, int K);
 int exl3_linear(const void* x, int x_bf16, int rows, int k, const exl3_shard* shards_host, int nshards, int K,
                 int codebook, void* y, int y_bf16, void* workspace, size_t workspace_bytes, void* stream);
 
-/* Workspace bytes of exl3_gemm_rotated for `rows` rows (below 65 rows those of its decode-GEMV launches, from 65 rows
- * those of the prefill decode-GEMM); 0 for bad shapes.  Same counter-region contract as exl3_linear_workspace_bytes. */
+/* Workspace bytes of exl3_gemm_rotated for up to `rows` rows (its decode-GEMV launches, and from 65 rows the prefill
+ * decode-GEMM); 0 for bad shapes.  Same counter-region contract as exl3_linear_workspace_bytes. */
 size_t exl3_gemm_rotated_workspace_bytes(int rows, int k, int n, int K);
 /* out fp16 [rows, n] = xh @ W_inner in the rotated basis (no Hadamards, no sign vectors); fp32 accumulation, one
  * rounding to fp16; xh fp16 [rows, k].  Identity rows of xh read W_inner out exactly.  The rows run through the
@@ -149,8 +149,8 @@ int exl3_linear_noalloc(const void* x, int x_bf16, int rows, int k, const exl3_s
                         int codebook, void* y, int y_bf16, void* stream);
 
 /* ---- prefill decode-GEMM (subsystem 3) ------------------------------------------------------------------------ */
-/* Workspace bytes of exl3_linear_prefill for `rows` rows of a group with input width k, n_total output columns and
- * nshards shards: EXL3_WORKSPACE_COUNTER_BYTES of split counters (zero before the first use; every call leaves them
+/* Workspace bytes that serve exl3_linear_prefill with up to `rows` rows of a group with input width k, n_total output
+ * columns and nshards shards (never less for more rows; a call itself is refused only below its own need): EXL3_WORKSPACE_COUNTER_BYTES of split counters (zero before the first use; every call leaves them
  * zero), the per-shard rotated activations (fp16 [nshards][rows][k]), then fp32 partials of the shared tiles.
  * Depends on the current device's CU count. */
 size_t exl3_prefill_workspace_bytes(int rows, int k, int n_total, int nshards);

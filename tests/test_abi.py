@@ -1,6 +1,7 @@
 """The C-ABI library without a GPU: it loads, exports every symbol include/exl3_mi355x.h declares, and rejects bad
 arguments before any device work (the reference's TORCH_CHECK paths, cuda/csrc/exl3_marlin.cu:132,189,195)."""
 import ctypes
+import re
 
 import pytest
 import torch
@@ -276,3 +277,26 @@ def test_mixed_moe_entry_points_reject_bad_class_counts(lib):
         _lib.EXL3_ERR_INVALID
     assert "no expert map" in lib.exl3_last_error().decode()
     assert lib.exl3_moe_classes_workspace_bytes(4, 8, 16, 256, 256, 2, cls) > 0
+
+
+@pytest.mark.parametrize("k,ns", [(6144, (5120,)), (5120, (17408, 17408)), (5120, (6144, 1024, 1024)), (17408, (5120,)),
+                                  (128, (128,)), (4096, (1408, 128, 640, 128)), (1664, (32896,)), (1024, (16384,))])
+def test_prefill_workspace_of_the_most_rows_serves_fewer(lib, k, ns):
+    """A workspace sized for a caller's most rows serves every smaller call: the need of each call's own layout, as the
+    refusal of a call without a workspace states it, and gemm_rotated's from its decode-GEMV rows on."""
+    P = 0x1000
+    shards = (_lib.Exl3Shard * len(ns))(*[_lib.Exl3Shard(P, P, P, n) for n in ns])
+    reported = worst = rotated = 0
+    for rows in sorted({*range(17, 2600, 21), 64, 65, 128, 256, 1024, 1025, 4096, 8192}):
+        assert lib.exl3_linear_prefill(P, 0, rows, k, shards, len(ns), 3, 1, P, 0, P, 0, None) == _lib.EXL3_ERR_INVALID
+        worst = max(worst, int(re.search(r"workspace 0 bytes, need (\d+)", lib.exl3_last_error().decode())[1]))
+        size, size_r = (lib.exl3_prefill_workspace_bytes(rows, k, sum(ns), len(ns)),
+                        lib.exl3_gemm_rotated_workspace_bytes(rows, k, ns[0], 3))
+        assert size >= max(worst, reported) and size_r >= rotated, rows
+        reported, rotated = size, size_r
+
+
+@pytest.mark.parametrize("k,n", [(768, 18304), (1664, 26880), (4096, 4096)])
+def test_gemm_rotated_workspace_past_the_switch_serves_fewer(lib, k, n):
+    need = [lib.exl3_gemm_rotated_workspace_bytes(r, k, n, 3) for r in range(1, 80)]
+    assert max(need[:64]) <= need[64] and need == sorted(need)

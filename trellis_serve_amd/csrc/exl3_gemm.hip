@@ -447,6 +447,28 @@ static GemmLayout gemm_layout(int slots, int rows, int k, int nct, int nshards) 
   return L;
 }
 
+// One workspace for every call of up to `rows` rows: a layout's own need goes down where whole rounds or lower tiles need
+// fewer partials.  Tiles are multiples of 64 rows, so up to 1024 rows every layout is looked at (2 us); past that the
+// bound is each height's most stream-K workgroups (gemm_share), which grows with the rows: at most 134 MB of partials.
+static size_t gemm_most_bytes(int slots, int rows, int k, int nct, int nshards) {
+  constexpr int kLooked = 1024;
+  size_t most = 0;
+  for (int r = std::min(rows, 64);; r = std::min(rows, r + 64)) {
+    most = std::max(most, gemm_layout(slots, r, k, nct, nshards).total);
+    if (r == rows || r >= kLooked) break;
+  }
+  if (rows > kLooked) {
+    size_t partials = 0;
+    for (const GemmShape& shape : kGemmShapes) {
+      const int64_t tiles = (rows + 16 * (int64_t)shape.mi - 1) / (16 * shape.mi) * nct;
+      const int64_t groups = std::min<int64_t>(slots, std::min<int64_t>(tiles, 2 * slots) * (k / kBK) / 8);
+      partials = std::max(partials, (size_t)std::max<int64_t>(1, groups) * 2 * gemm_partial_bytes(shape.mi));
+    }
+    most = std::max(most, gemm_layout(slots, rows, k, nct, nshards).partial_off + partials);
+  }
+  return most;
+}
+
 }  // namespace exl3
 
 using namespace exl3;
@@ -459,7 +481,7 @@ extern "C" size_t exl3_prefill_workspace_bytes(int rows, int k, int n_total, int
   const int slots = gemm_slots();
   size_t need = 0;
   for (int nct = (n_total / 128 + 1) / 2; nct <= (n_total / 128 + nshards) / 2; nct++)
-    need = std::max(need, gemm_layout(slots, rows, k, nct, nshards).total);
+    need = std::max(need, gemm_most_bytes(slots, rows, k, nct, nshards));
   return need;
 }
 
@@ -559,7 +581,7 @@ size_t linear_gemm_workspace_bytes(int rows, int k, int n_total) {
 
 size_t prefill_plain_workspace_bytes(int rows, int k, int n) {
   const int nct = (n / 128 + 1) / 2;
-  return gemm_layout(gemm_slots(), rows, k, nct, 1).total;
+  return gemm_most_bytes(gemm_slots(), rows, k, nct, 1);
 }
 
 // exl3_gemm_rotated from kPrefillRows rows: the rows as given (fp16, already in the rotated basis), no output

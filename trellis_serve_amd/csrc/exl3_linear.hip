@@ -1000,12 +1000,12 @@ extern "C" int exl3_linear(const void* x, int x_bf16, int rows, int k, const exl
 
 extern "C" size_t exl3_gemm_rotated_workspace_bytes(int rows, int k, int n, int K) {
   if (rows <= 0 || k <= 0 || n <= 0 || k % 128 || n % 128 || n / 128 > kMaxCounters || !valid_bits(K)) return 0;
-  if (rows >= kPrefillRows) return prefill_plain_workspace_bytes(rows, k, n);
-  return gemv_workspace_bytes(rows, k, n, K, kGemvRows, false);
+  const size_t gemv = gemv_workspace_bytes(std::min(rows, kPrefillRows - 1), k, n, K, kGemvRows, false);
+  return rows < kPrefillRows ? gemv : std::max(gemv, prefill_plain_workspace_bytes(rows, k, n));
 }
 
-// Rows are served by the kernel that serves the same row count in a linear: below kPrefillRows the decode-GEMV (one
-// 16-row group per launch, two decoded tiles per MFMA), from there the prefill decode-GEMM, both without rotations.
+// Below kPrefillRows the decode-GEMV (one 16-row group per launch, two decoded tiles per MFMA), from there the prefill
+// decode-GEMM, both without rotations.
 extern "C" int exl3_gemm_rotated(const void* xh, int rows, int k, const void* trellis, int n, int K, int codebook,
                                  void* out, void* workspace, size_t workspace_bytes, void* stream) {
   EXL3_CHECK_ARG((rows == 0 || (xh && out)) && trellis, "exl3_gemm_rotated: null pointer");
@@ -1015,9 +1015,13 @@ extern "C" int exl3_gemm_rotated(const void* xh, int rows, int k, const void* tr
   EXL3_CHECK_ARG((int64_t)k * n * K / 8 <= INT32_MAX, "exl3_gemm_rotated: trellis exceeds the 2 GiB buffer range");
   EXL3_CHECK_ARG(n / 128 <= kMaxCounters, "exl3_gemm_rotated: n = %d exceeds %d columns", n, kMaxCounters * 128);
   if (rows == 0) return EXL3_OK;
-  if (rows >= kPrefillRows)
+  if (rows >= kPrefillRows) {  // the reported size also covers fewer rows: held to it
+    const size_t need = exl3_gemm_rotated_workspace_bytes(rows, k, n, K);
+    EXL3_CHECK_ARG(workspace && workspace_bytes >= need, "exl3_gemm_rotated: workspace %zu bytes, need %zu",
+                   workspace_bytes, need);
     return prefill_plain_gemm(xh, rows, k, trellis, n, K, codebook, out, workspace, workspace_bytes,
                               as_stream(stream));
+  }
   ShardArgs sa{};
   sa.trellis[0] = static_cast<const uint32_t*>(trellis);
   sa.tn[0] = n / 16;

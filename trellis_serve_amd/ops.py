@@ -155,7 +155,7 @@ def reserve_prefill(device: torch.device, max_rows: int, k: int, n_total: int, n
     lib = _lib.load()
     dev = torch.device("cuda", _dev_index(device))
     with torch.cuda.device(dev):   # the plan depends on the device's CU count
-        need = _max_need(lambda r: lib.exl3_prefill_workspace_bytes(r, k, n_total, nshards), max_rows)
+        need = lib.exl3_prefill_workspace_bytes(max(1, int(max_rows)), k, n_total, nshards)
     _ws("prefill", dev).reserve(dev, need)
 
 
