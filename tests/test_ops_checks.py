@@ -88,3 +88,66 @@ def test_linear_takes_every_form_of_its_rows():
     with pytest.raises(ValueError):
         ops.had_in_group(torch.ones((1, 256), dtype=torch.float16), torch.ones(256, dtype=torch.float16, device="cuda"),
                          torch.empty((1, 256), dtype=torch.float16, device="cuda"))
+
+
+class _Calls:
+    """A library whose size functions and launches record whether the tensors' device was current."""
+
+    def __init__(self, seen, here):
+        self.seen, self.here = seen, here
+
+    def __getattr__(self, name):
+        def call(*args):
+            self.seen.append((name, self.here[-1]))
+            return 4096 if name.endswith("_bytes") else 0
+        return call
+
+
+def test_sizes_and_launches_that_follow_the_cu_count_run_on_the_tensors_device(monkeypatch):
+    """Past 32 rows a linear's workspace and plan follow the current device's CU count: with the tensors on device 1 and
+    device 0 current, both the size and the call are taken with device 1 current (calls switch only when it is not)."""
+    here, switched = [0], []
+
+    class On:
+        def __init__(self, device):
+            self.index = ops._dev_index(device)
+
+        def __enter__(self):
+            switched.append(self.index)
+            here.append(self.index)
+
+        def __exit__(self, *a):
+            here.pop()
+
+    seen = []
+    lib = _Calls(seen, here)
+    monkeypatch.setattr(torch.cuda, "current_device", lambda: here[-1])
+    monkeypatch.setattr(torch.cuda, "device", On)
+    monkeypatch.setattr(ops._lib, "load", lambda *a: lib)
+    monkeypatch.setattr(ops, "_ws", lambda kind, dev: type("W", (), {"reserve": lambda self, dev, n: None})())
+    monkeypatch.setattr(ops, "workspace", lambda dev, n, kind="linear": torch.empty(n, dtype=torch.uint8))
+    monkeypatch.setattr(ops, "_stream", lambda dev: 0)
+    monkeypatch.setattr(ops, "_dev_index", lambda dev: 1)
+    arr = (ops._lib.Exl3Shard * 1)(ops._lib.Exl3Shard(1, 1, 1, 128))
+    monkeypatch.setattr(ops, "_shards", lambda *a: (arr, 256, 3))
+    monkeypatch.setattr(ops, "_check_trellis", lambda t: (256, 128, 3))
+    monkeypatch.setattr(ops, "_half", lambda t, name: t)
+    x = torch.zeros((65, 256), dtype=torch.float16)
+    dev = torch.device("cuda", 1)
+
+    def everything():
+        ops.linear(x, [], [], [], 1)
+        ops.linear_prefill(x, [], [], [], 1)
+        ops.gemm_rotated(x, x, 1)
+        ops.reserve_linear(dev, 40, 256, 128, 3)
+        ops.reserve_prefill(dev, 40, 256, 128, 1)
+
+    everything()
+    assert {n for n, _ in seen} >= {"exl3_linear", "exl3_linear_prefill", "exl3_gemm_rotated",
+                                    "exl3_linear_workspace_bytes", "exl3_prefill_workspace_bytes",
+                                    "exl3_gemm_rotated_workspace_bytes"}
+    assert all(current == 1 for _, current in seen), seen
+    assert here == [0] and switched == [1] * 5
+    here[:] = [1]
+    everything()
+    assert switched == [1] * 7   # the two reservations, at load

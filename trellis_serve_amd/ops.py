@@ -107,6 +107,12 @@ def _dev_index(device: torch.device) -> int:
     return index if index is not None else torch.cuda.current_device()
 
 
+def _elsewhere(device: torch.device) -> bool:
+    """Whether another device is current: plans that follow the current device's CU count (the decode-GEMM's, past 32
+    rows of a linear) are then sized and launched with `device` current."""
+    return _dev_index(device) != torch.cuda.current_device()
+
+
 _initialised: set[int] = set()
 
 
@@ -147,7 +153,9 @@ def reserve_linear(device: torch.device, max_rows: int, k: int, n_total: int, K:
     n_total output columns at bitrate K (the reference reserves its scratch at load, kernels/marlin.py:24-33)."""
     lib = _lib.load()
     dev = torch.device("cuda", _dev_index(device))
-    _ws("linear", dev).reserve(dev, _max_need(lambda r: lib.exl3_linear_workspace_bytes(r, k, n_total, K), max_rows))
+    with torch.cuda.device(dev):   # the plan depends on the device's CU count
+        need = _max_need(lambda r: lib.exl3_linear_workspace_bytes(r, k, n_total, K), max_rows)
+    _ws("linear", dev).reserve(dev, need)
 
 
 def reserve_prefill(device: torch.device, max_rows: int, k: int, n_total: int, nshards: int) -> None:
@@ -296,6 +304,9 @@ def gemm_rotated(xh: torch.Tensor, trellis: torch.Tensor, codebook: int,
     if xh.dim() != 2 or xh.shape[1] != k:
         raise ValueError(f"xh must be [rows, {k}]")
     rows = xh.shape[0]
+    if rows > 64 and _elsewhere(xh.device):
+        with torch.cuda.device(xh.device):
+            return gemm_rotated(xh, trellis, codebook, out)
     if out is None:
         out = torch.empty((rows, n), dtype=torch.float16, device=xh.device)
     _check_out(out, (rows, n), xh, (torch.float16,))
@@ -357,6 +368,9 @@ def linear(x: torch.Tensor, trellis: list[torch.Tensor], suh: list[torch.Tensor]
     arr, k, K = _shards(trellis, suh, svh, device, layout)
     rows2d = _rows2d(x, k)
     rows = rows2d.shape[0]
+    if rows > 32 and _elsewhere(device):
+        with torch.cuda.device(device):
+            return linear(x, trellis, suh, svh, codebook, out, layout)
     n_total = sum([a.n for a in arr])
     out = _out2d(x, rows, n_total, out)
     lib = _lib.load()
@@ -378,12 +392,13 @@ def linear_prefill(x: torch.Tensor, trellis: list[torch.Tensor], suh: list[torch
     arr, k, K = _shards(trellis, suh, svh, device, layout)
     rows2d = _rows2d(x, k)
     rows = rows2d.shape[0]
+    if _elsewhere(device):
+        with torch.cuda.device(device):
+            return linear_prefill(x, trellis, suh, svh, codebook, out, layout)
     n_total = sum([a.n for a in arr])
     out = _out2d(x, rows, n_total, out)
     lib = _lib.load()
-    with torch.cuda.device(device):   # the plan depends on the device's CU count
-        need = lib.exl3_prefill_workspace_bytes(rows, k, n_total, len(arr))
-    ws = workspace(device, need, "prefill")
+    ws = workspace(device, lib.exl3_prefill_workspace_bytes(rows, k, n_total, len(arr)), "prefill")
     _lib.check(lib.exl3_linear_prefill(rows2d.data_ptr(), int(bf16), rows, k, arr, len(arr), K, int(codebook),
                                        out.data_ptr(), int(out.dtype == torch.bfloat16), ws.data_ptr(), ws.numel(),
                                        _stream(device)), "linear_prefill")
