@@ -465,12 +465,8 @@ def test_two_row_groups_match_oracle_with_prepared_rows(coracle, rows):
     assert torch.equal(_ops().linear(_dev(x), *args), y)
 
 
-@pytest.mark.parametrize("rows", [40, 64])
-def test_wide_layer_rows_past_32_take_two_group_launches(coracle, rows):
-    """A wide layer (256 column blocks) at 33-64 rows runs as launches of 32 rows with two row groups (four groups
-    would need more LDS than a launch gets by default); the first and last 1024 columns against the oracle."""
+def _wide_layer(coracle, rows, k, n, K=3, cb=1):
     rng = np.random.default_rng(90 + rows)
-    k, n, K, cb = 2048, 32768, 3, 1
     tr, suh, svh = _trellis(rng, k, n, K), _signs(rng, k), _signs(rng, n)
     x = (rng.standard_normal((rows, k)) * 0.5).astype(np.float16)
     y = _ops().linear(_dev(x), [_dev(tr)], [_dev(suh)], [_dev(svh)], cb).cpu().numpy()
@@ -480,3 +476,18 @@ def test_wide_layer_rows_past_32_take_two_group_launches(coracle, rows):
                                  dtype=np.float64)
         nrel, mrel = _errs(y[:, c0:c0 + 1024], ref)
         assert nrel <= TOL and mrel <= TOL, (c0, nrel, mrel)
+
+
+@pytest.mark.parametrize("rows,k,n", [(40, 640, 49152), (64, 640, 49152), (100, 2048, 32768)])
+def test_wide_layers_of_two_group_launches(coracle, rows, k, n):
+    """Layers with 768 workgroups of 4 blocks of rows or more, below the decode-GEMM's 4096 units (or past its 64 rows),
+    run as launches of 32 rows with two row groups; the first and last 1024 columns against the oracle."""
+    assert n // 128 * -(-k // 512) >= 768 and (n // 128 * (k // 128) < 4096 or rows > 64)
+    _wide_layer(coracle, rows, k, n)
+
+
+@pytest.mark.parametrize("rows", [40, 64])
+def test_wide_layer_rows_past_32(coracle, rows):
+    """A wide layer (256 column blocks, 4096 units) at 33-64 rows runs as one decode-GEMM; the first and last 1024 columns
+    against the oracle."""
+    _wide_layer(coracle, rows, 2048, 32768)

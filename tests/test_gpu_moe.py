@@ -6,6 +6,7 @@ import numpy as np
 import pytest
 import torch
 
+import moe_plan
 from oracle import exl3_oracle as orc
 
 pytestmark = pytest.mark.gpu
@@ -171,9 +172,10 @@ def test_moe_single_token_top_k_range_bf16_and_repeat(top_k):
 
 
 def test_moe_many_slots_use_the_routing_launch():
-    """2080 slots over 8 experts (260 per expert: passes of 64 slots, the last one partial); both ends of the token
-    range against the exact layer, and a repeat is bit-identical."""
+    """2080 slots over 8 experts (260 per expert: the sorted expert GEMMs, three tiles each, the last one shorter); both
+    ends of the token range against the exact layer, and a repeat is bit-identical."""
     from trellis_serve_amd import ops
+    assert moe_plan.way(260, 8, 8, 128, 128) == "gemm128"
     rng = np.random.default_rng(47)
     E, H, I, K, top_k, T = 8, 128, 128, 3, 8, 260  # 2080 slots
     ex = _experts(rng, E, H, I, K)
@@ -253,11 +255,11 @@ def test_moe_full_shape_batched_tokens_match_single_token(coracle):
 
 @pytest.mark.parametrize("T", [3, 20, 40, 300])
 def test_moe_slot_groups_and_passes_match_exact_layer(T):
-    """Several tokens: routing + input rotation launch, up to 16 P slots sharing each decoded tile, the GLU folded into
-    the gate/up reducer.  3 / 20 / 40 / 300 tokens over 8 experts run P = 1 / 2 / 4 / 4 groups (40 tokens: one pass of 40 slots per
-    expert in 3 groups; 300 tokens: 300 slots per expert, several passes).  Every token against the exact layer, and
-    two tokens against their single-token calls (slot mode: other k-split plan) within 1e-3."""
+    """3 / 20 / 40 / 300 slots per expert of a small layer: the sorted expert GEMMs with tiles of 64 slots and, at 300, of
+    128.  Every token against the exact layer, and two tokens against their single-token calls (slot mode) within 1e-3.
+    (The expert GEMVs' groups and passes: test_moe_expert_gemvs_by_groups_and_passes.)"""
     from trellis_serve_amd import ops
+    assert moe_plan.way(T, 8, 8, 256, 256) == ("gemm128" if T == 300 else "gemm64")
     rng = np.random.default_rng(60 + T)
     E, H, I, K, top_k = 8, 256, 256, 3, 8
     ex = _experts(rng, E, H, I, K)
@@ -316,9 +318,10 @@ def test_moe_random_shapes_match_exact_layer(case):
 def test_moe_down_bitrate_differs_from_gate_up(K, K_down, T):
     """A checkpoint may store down_proj at another bitrate than gate_proj / up_proj (the reference requires only gate
     K == up K, cuda/src/sglang_exl3/sglang_glue/moe.py:148-152, and runs bits_gate_up and bits_down separately,
-    kernels/reference.py:123-149).  Single token (slot mode), a few tokens (P = 1) and 40 tokens (P = 2, the GLU
-    folded into the gate/up reducer) against the float64 exact layer, every codebook."""
+    kernels/reference.py:123-149).  Single token (slot mode), a few tokens (expert GEMVs of one group) and 40 tokens
+    (the sorted expert GEMMs) against the float64 exact layer, every codebook."""
     from trellis_serve_amd import ops
+    assert moe_plan.way(T, 4, 8, 256, 384, K, K_down) == {1: "slot", 5: "P1", 40: "gemm64"}[T]
     rng = np.random.default_rng(7000 + 10 * K + K_down + T)
     E, H, I, top_k = 8, 256, 384, 4
     ex = _experts(rng, E, H, I, K, K_down)
@@ -371,7 +374,6 @@ MOE_GEMM_CASES = [(384, 128, 3, 3, 1, (1, 15, 16, 17, 63, 64, 0, 65, 70, 33), Fa
                   (128, 128, 8, 8, 1, (400,), False),
                   (512, 640, 4, 3, 2, (65, 66, 128, 130, 48, 100), True),
                   (384, 256, 3, 4, 1, (32, 31, 33, 1, 16, 17, 64, 2, 0, 30), False),
-                  # more workgroups than CUs, 0 to 34 slots per expert: the 32-row code beside the 64-row one
                   (256, 128, 3, 4, 1, tuple(7 * e % 35 for e in range(300)), False)]
 
 
@@ -405,3 +407,69 @@ def test_moe_expert_gemms_at_tile_edges(case):
     assert nrel <= tol and mrel <= tol, (case, nrel, mrel)
     for _ in range(3):
         assert torch.equal(ops.moe_forward(xt, *args), y)
+
+
+# More workgroups than CUs in both phases: tiles of at most 32 slots run 32-row code, beside tiles of more, in the kernel
+# of 64 slots (1 to 34 slots per expert, every count) and in that of 128 (60 experts of 250 slots, the others 1 to 34).
+# (H, I, K gate/up, K down, codebook, slots per expert, tile height)
+MOE_LOW_TILES = [(256, 128, 3, 4, 1, tuple(e % 34 + 1 for e in range(306)), 64),
+                 (512, 256, 2, 3, 0, (250,) * 60 + tuple(e % 34 + 1 for e in range(40)), 128),
+                 (512, 256, 4, 6, 2, (250,) * 60 + tuple(31 + e % 3 for e in range(40)), 128)]
+
+
+@pytest.mark.parametrize("case", MOE_LOW_TILES, ids=[f"tile{c[6]}-K{c[2]}-{c[3]}-cb{c[4]}" for c in MOE_LOW_TILES])
+def test_moe_expert_gemms_of_low_tiles(case, coracle):
+    """Every token against the float64 exact layer (the bar of this file), repeated calls bit-identical."""
+    from conftest import c_reconstruct
+    from trellis_serve_amd import ops
+    H, I, K, K_down, cb, counts, rows = case
+    E, T = len(counts), -(-sum(counts) // 2)
+    assert moe_plan.way(T, 2, E, H, I, K, K_down) == f"gemm{rows}"
+    tiles = sum(-(-n // rows) for n in counts)
+    assert tiles * (I // 128) > 256 and tiles * -(-H // 256) > 256
+    assert min(counts) <= 32 < max(n for n in counts if n <= 34) and {31, 32, 33} <= set(counts)
+    rng = np.random.default_rng(H + E + K)
+    ex = _experts(rng, E, H, I, K, K_down)
+    cache = {(e, p): c_reconstruct(coracle, ex[e][p][0], K_down if p == "down" else K, cb)
+             for e in range(E) for p in ("gate", "up", "down")}
+    flat = np.concatenate([np.full(n, e) for e, n in enumerate(counts)])
+    ids = rng.permutation(np.append(flat, [-1] * (2 * T - flat.size))).reshape(T, 2).astype(np.int32)
+    x = (rng.standard_normal((T, H)) * 0.1).astype(np.float16)
+    w = rng.random((T, 2)).astype(np.float32)
+    args = (torch.from_numpy(x).cuda(), torch.from_numpy(ids).cuda(), torch.from_numpy(w).cuda(), _stack(ex), cb)
+    y = ops.moe_forward(*args)
+    nrel, mrel = _errs(y.cpu().numpy(), orc.moe_forward(x, ids, w, ex, None, cb, w_cache=cache))
+    assert nrel <= 2e-3 and mrel <= 2e-3, (nrel, mrel)
+    assert torch.equal(ops.moe_forward(*args), y)
+
+
+# The expert GEMVs of several tokens by groups of 16 slots (P) and passes over an expert's weights: one expert has more
+# slots than a pass takes, others fewer, one none; wide inputs and few columns keep these calls on the GEMVs.
+# (H, I, K gate/up, K down, codebook, slots per expert, P)
+MOE_GEMV_CASES = [(4096, 128, 3, 4, 1, (20, 3, 0, 5), 1), (4096, 128, 2, 2, 0, (40, 12, 9, 15), 2),
+                  (4096, 256, 4, 3, 2, (32, 33, 0, 10), 2), (4096, 128, 5, 6, 1, (70, 5, 10, 11), 4),
+                  (16384, 128, 8, 3, 0, (90,), 4), (8192, 128, 6, 8, 2, (64, 17), 4), (4096, 128, 3, 3, 1, (16, 1, 2, 7), 1)]
+
+
+@pytest.mark.parametrize("case", MOE_GEMV_CASES, ids=[f"P{c[6]}-H{c[0]}-{'+'.join(map(str, c[5]))}" for c in MOE_GEMV_CASES])
+def test_moe_expert_gemvs_by_groups_and_passes(case, coracle):
+    """Every token against the float64 exact layer (the bar of this file), repeated calls bit-identical."""
+    from conftest import c_reconstruct
+    from trellis_serve_amd import ops
+    H, I, K, K_down, cb, counts, P = case
+    E, flat = len(counts), np.concatenate([np.full(n, e) for e, n in enumerate(counts)] + [np.array([-1, len(counts)])])
+    top_k = 2 if E > 1 and flat.size % 2 == 0 else 1
+    T = flat.size // top_k
+    assert moe_plan.way(T, top_k, E, H, I, K, K_down) == f"P{P}"
+    rng = np.random.default_rng(sum(counts) + H)
+    ex = _experts(rng, E, H, I, K, K_down)
+    cache = {(e, p): c_reconstruct(coracle, ex[e][p][0], K_down if p == "down" else K, cb)
+             for e in range(E) for p in ("gate", "up", "down")}
+    ids = rng.permutation(flat).reshape(T, top_k).astype(np.int32)
+    x = (rng.standard_normal((T, H)) * 0.05).astype(np.float16)
+    w = rng.random((T, top_k)).astype(np.float32)
+    args = (torch.from_numpy(x).cuda(), torch.from_numpy(ids).cuda(), torch.from_numpy(w).cuda(), _stack(ex), cb)
+    y = ops.moe_forward(*args)
+    nrel, mrel = _errs(y.cpu().numpy(), orc.moe_forward(x, ids, w, ex, None, cb, w_cache=cache))
+    assert nrel <= 2e-3 and mrel <= 2e-3, (nrel, mrel)
+    assert torch.equal(ops.moe_forward(*args), y)

@@ -5,6 +5,7 @@ import pytest
 import torch
 
 from conftest import c_reconstruct
+import gemm_plan
 from oracle import exl3_oracle as orc
 
 pytestmark = pytest.mark.gpu
@@ -86,10 +87,10 @@ def test_prefill_is_deterministic():
 
 
 def test_prefill_split_tail_tiles_match_oracle(coracle):
-    """More tiles than one round of the machine holds: the tiles past the last whole round run as k-split items whose
-    fp32 partials are summed in split order.  The tail (last row block, last column blocks) and a data-parallel tile
-    are checked against the float64 oracle, and repeated calls are bit-identical."""
-    slots = torch.cuda.get_device_properties(0).multi_processor_count  # one 256 x 256 tile per CU at a time
+    """More columns than one round of the machine holds, as whole tiles of 192 rows: the last row block and column blocks
+    and the first are checked against the float64 oracle, and repeated calls are bit-identical.  (The layout that
+    shares the tiles past the whole rounds: test_prefill_shared_tiles_after_whole_rounds_match_oracle.)"""
+    slots = torch.cuda.get_device_properties(0).multi_processor_count
     M, k, K, cb = 768, 1024, 3, 1
     cbk = (slots + 28 + 2) // 3  # 3 row blocks x cbk 256-column tiles = slots + ~28 tail tiles
     n = 256 * cbk
@@ -108,6 +109,31 @@ def test_prefill_split_tail_tiles_match_oracle(coracle):
         assert nrel <= TOL and mrel <= TOL, (rows, cols, nrel, mrel)
     for _ in range(3):
         assert torch.equal(_ops().linear_prefill(_dev(x), *args), y)
+
+
+def test_prefill_shared_tiles_after_whole_rounds_match_oracle(coracle):
+    """Two rounds of tiles: the first 259 are shared out as runs of k-steps whose fp32 partials are summed in run order,
+    the other 256 are whole.  A shared, a whole and the last row block's columns against the float64 oracle, and
+    repeated calls bit-identical."""
+    M, k, ns, K, cb = 640, 2048, (9344, 16768), 3, 1
+    L = gemm_plan.layout(M, k, ns)
+    assert L.height == 128 and L.shared == 259 and L.tiles == 515
+    rng = np.random.default_rng(15)
+    parts = [_case(rng, k, n, K) for n in ns]
+    x = (rng.standard_normal((M, k)) * 0.5).astype(np.float16)
+    args = [[_dev(p[i]) for p in parts] for i in range(3)]
+    y = _ops().linear_prefill(_dev(x), *args, cb)
+    for rows, s, cols in ((slice(0, 128), 0, slice(0, 512)), (slice(256, 384), 0, slice(9088, 9344)),
+                          (slice(512, 640), 1, slice(16256, 16768))):
+        tr, suh, svh = parts[s]
+        t = tr[:, cols.start // 16:cols.stop // 16]
+        ref = orc.linear_forward(x[rows], t, suh, svh[cols], K, cb, w_inner=c_reconstruct(coracle, t, K, cb),
+                                 dtype=np.float64)
+        c0 = s * ns[0]
+        nrel, mrel = _errs(y[rows, c0 + cols.start:c0 + cols.stop].cpu().numpy(), ref)
+        assert nrel <= TOL and mrel <= TOL, (rows, cols, nrel, mrel)
+    for _ in range(3):
+        assert torch.equal(_ops().linear_prefill(_dev(x), *args, cb), y)
 
 
 @pytest.mark.parametrize("M", [1, 16, 40, 255])
@@ -133,11 +159,10 @@ def test_prefill_few_rows_many_contributors(coracle, M, n):
 @pytest.mark.parametrize("rows,k,ns", [(1, 128, (128,)), (5, 384, (256, 128)), (37, 512, (256,)), (333, 1280, (128, 128, 384, 256)),
                                         (2200, 640, (512, 128, 256)), (8200, 2048, (128,))])
 def test_prefill_rotation_layouts_bit_identical(bf16, rows, k, ns):
-    """The input rotation has two kernels: 16 lanes per 128-value unit with 16-byte loads (x and every suh 16-byte
-    aligned) and 32 lanes with 8-byte loads (otherwise).  Both run the butterfly's stages in the same order on the
-    same pairs, so the whole prefill output must be bit-identical.  An input viewed 8 bytes into a buffer takes the
-    second kernel.  The shapes reach 1, 2 and 4 units per lane group of the first (below 2^15, from 2^15, from 2^17
-    units)."""
+    """An input viewed 8 bytes into a buffer (the input rotation loads 8 bytes at a time) gives the bits of an aligned
+    one, and both the result of the rotation-free pieces: fp16(Had(x * suh)) by the wavefront butterfly, the decoded
+    weights in an fp32 product, the output rotation (2e-3; bf16 outputs 6e-3: half an ulp of bf16 is 2^-9).  Rows on
+    both sides of 1024, where one wave takes every shard."""
     rng = np.random.default_rng(9100 + rows + int(bf16))
     K, cb = 3, 1
     cases = [_case(rng, k, n, K) for n in ns]
@@ -152,4 +177,11 @@ def test_prefill_rotation_layouts_bit_identical(bf16, rows, k, ns):
     y8 = _ops().linear_prefill(x_off, *args)
     torch.cuda.synchronize()
     assert torch.equal(y16.view(torch.int16), y8.view(torch.int16))
-    assert torch.isfinite(y16.float()).all()
+    ref = torch.empty((rows, sum(ns)), dtype=torch.float16, device="cuda")
+    col = 0
+    for tr, suh, svh in zip(*args[:3]):
+        xh = _ops().had_in_group(x, suh)
+        _ops().had_out_into((xh.float() @ _ops().reconstruct(tr, cb).float()).half(), svh, ref, col)
+        col += svh.numel()
+    d, tol = (y16.float() - ref.float()), 6e-3 if bf16 else TOL
+    assert (d.norm() / ref.float().norm()).item() <= tol and (d.abs().max() / ref.float().abs().max()).item() <= tol
