@@ -2,7 +2,7 @@
 
     python bench.py [--gpus 1] [--steps K] [--warmup W] [--no-cpu-baseline]
 
-Workload (BASELINE.json configs[1]): the dense 27B-class decoder layer set at K = 3 bpw, MCG codebook, seeded random
+Workload: the dense 27B-class decoder layer set at K = 3 bpw, MCG codebook, seeded random
 packed codes and +-1 sign vectors: q/k/v 5120 -> 6144+1024+1024 (one fused 3-shard group), o_proj 6144 -> 5120,
 gate/up 5120 -> 17408+17408 (one fused 2-shard group), down 17408 -> 5120, fp16 activations N(0,1) at M = 1.
 One step = the four fused linears (decode-GEMV + rotations) over one batch of M rows.  Inputs are resident in HBM
@@ -11,11 +11,11 @@ before timing starts; R rotating copies of the layer set (>= 512 MB, twice the 2
 Prints one JSON line: metric/value = algorithmic HBM GB/s of the layer set at M = 1 (trellis + sign vectors +
 activations in/out: 128,174,080 B per step), plus the roofline of the dominant kernel (the fused
 decode-GEMV), the CPU baseline (the oracle's decode + matmul on up to 16 host cores, on a bounded sample), the
-M = 4 / 16 rates, and the other configs as reported fields: the single 4096 x 4096 linear of configs[0] (K = 4,
-3INST, M = 1), the prefill decode-GEMM TFLOPS (configs[2], `decode_gemm_tflops_m2048` is the second half of the
-metric), the MoE layer (configs[3]) and the quantized-KV decode attention (configs[4]).  For scale: the warm (single copy) layer-set rate, the trellis-only
+M = 4 / 16 rates, and further workloads as reported fields: a single 4096 x 4096 linear (K = 4,
+3INST, M = 1), the prefill decode-GEMM TFLOPS (5120 -> 17408, `decode_gemm_tflops_m2048` is the second half of the
+metric), the MoE layer and the quantized-KV decode attention.  For scale: the warm (single copy) layer-set rate, the trellis-only
 weight-stream rate, hipBLASLt's fp16 8192^3 GEMM, and the reference's prefill design (W decoded to HBM, then the vendor
-GEMM) rebuilt on this box at configs[2] M = 2048.
+GEMM) rebuilt on this box at that shape, M = 2048.
 """
 from __future__ import annotations
 
@@ -159,8 +159,8 @@ def _median_s(fn, runs: int) -> float:
     return float(np.median(times))
 
 
-MOE_SHAPE = (128, 2048, 768, 3, 8)  # E, H, I, K, top_k (BASELINE configs[3])
-KV_SHAPE = (16, 40, 8, 128)         # B, Hq, Hkv, head_dim (BASELINE configs[4])
+MOE_SHAPE = (128, 2048, 768, 3, 8)  # E, H, I, K, top_k
+KV_SHAPE = (16, 40, 8, 128)         # B, Hq, Hkv, head_dim
 
 
 def cpu_table(runs: int = 3, sample_tiles: int = 8192) -> dict:
@@ -364,7 +364,7 @@ def _graph_us(torch, fn, calls: int, reps: int = 3, warm_s: float = 0.05) -> flo
 
 
 def bench_c1(torch, ops, dev) -> dict:
-    """one 4096 -> 4096 linear, K = 4, 3INST, M = 1 (x fp16 N(0,1)): decode-GEMV with both
+    """One 4096 -> 4096 linear, K = 4, 3INST, M = 1 (x fp16 N(0,1)): decode-GEMV with both
     rotations.  64 rotating copies (537 MB > 2 x the 256 MB MALL) keep the weights cold; the graph replays one call per
     copy.  Bytes = 8,421,376 per call (trellis + suh + svh + x + y)."""
     k = n = 4096
@@ -389,7 +389,7 @@ def bench_c1(torch, ops, dev) -> dict:
 
 
 def bench_prefill(torch, ops, dev) -> dict:
-    """one 5120 -> 17408 linear, fp16 x ~ N(0,1) * 0.5, the fused decode-GEMM
+    """One 5120 -> 17408 linear, fp16 x ~ N(0,1) * 0.5, the fused decode-GEMM
     (exl3_linear_prefill).  M in {512, 2048, 8192} at K = 3 MCG, and M = 2048 over K in {2,4,5,6,8} cycling the three
     codebooks.  TFLOPS = 2 M k n / device time."""
     k, n = 5120, 17408
@@ -432,7 +432,7 @@ def bench_vendor(torch, ops, dev) -> dict:
     """The vendor fp16 GEMM on the same box, for scale: (1) torch.mm (hipBLASLt) on 8192^3 fp16, the practical MFMA
     ceiling of a plain GEMM; (2) the reference's own prefill design (decode W_inner to HBM, vendor GEMM, output
     rotation: kernels/reference.py:71-104, runtime/ops.py:36-59) rebuilt from this library's had_in / reconstruct /
-    had_out kernels around torch.mm, at BASELINE configs[2] M = 2048, K = 3 MCG, against the fused decode-GEMM on the
+    had_out kernels around torch.mm, at 5120 -> 17408, M = 2048, K = 3 MCG, against the fused decode-GEMM on the
     same inputs.  Eager launches (each >= tens of us), HIP events."""
     out = {}
     g = torch.Generator(device="cpu").manual_seed(21)
@@ -482,7 +482,7 @@ def bench_vendor(torch, ops, dev) -> dict:
 
 
 def bench_moe(torch, ops, dev) -> dict:
-    """BASELINE configs[3]: 128 experts, top-8, hidden 2048, intermediate 768, K = 3 MCG; router logits fp32 N(0,1),
+    """128 experts, top-8, hidden 2048, intermediate 768, K = 3 MCG; router logits fp32 N(0,1),
     top-8 ids and softmax weights over the selected logits.  Three rotating copies of the experts, a new routing per
     call.  Bytes = touched experts x 1,786,368 (trellis + sign vectors) + T x (8192 + 64)."""
     from trellis_serve_amd.ops import MOE_TENSORS
@@ -523,7 +523,7 @@ def bench_moe(torch, ops, dev) -> dict:
 
 
 def bench_kv(torch, ops, dev) -> dict:
-    """quantized-KV decode attention, 40 query / 8 KV heads, head_dim 128, batch 16, context 4k
+    """Quantized-KV decode attention, 40 query / 8 KV heads, head_dim 128, batch 16, context 4k
     and 32k, 16-token pages in a random page order, 8- and 4-bit codes with per-(page, head) fp16 scales.  Rotating
     cache copies keep >= 512 MB in play at 4k.  Bytes = codes + scales + page table + q/out."""
     B, Hq, Hkv, D = 16, 40, 8, 128
@@ -565,9 +565,10 @@ def _under_profiler() -> bool:
 
 def probe(kind: str, launches: int) -> int:
     """Short GPU programs for counter passes: `gate_up` launches the dominant GEMV kernel `launches` times over five
-    rotating copies of the layer; `prefill` the configs[2] decode-GEMM (5120 -> 17408, K = 3 MCG, M = 2048); `kv8` /
-    `kv4` the configs[4] KV decode attention at 4k context (B = 16, 40 / 8 heads, 8- / 4-bit codes, four rotating
-    caches in a random page order); `copy` runs a plain 512 MiB device copy (the calibration of FETCH_SIZE /
+    rotating copies of the layer (`gate_up16`: 16 rows); `prefill` the decode-GEMM (5120 -> 17408, K = 3 MCG, M = 2048); `kv8` /
+    `kv4` the KV decode attention at 4k context (B = 16, 40 / 8 heads, 8- / 4-bit codes, four rotating
+    caches in a random page order); `moe256` / `moe2048` the expert layer of `bench_moe` at that many tokens, routed over
+    experts of uneven popularity; `copy` runs a plain 512 MiB device copy (the calibration of FETCH_SIZE /
     WRITE_SIZE)."""
     import torch
 
@@ -596,6 +597,20 @@ def probe(kind: str, launches: int) -> int:
         o = torch.empty((B, Hq, D), dtype=torch.float16, device=dev)
         for i in range(launches):
             ops.kv_decode_attention(q, *sets[i % 4][:4], sets[i % 4][4], lens, bits, out=o)
+    elif kind.startswith("moe"):
+        E, top_k, H, I, T = 128, 8, 2048, 768, int(kind[3:])
+        g = torch.Generator(device="cuda").manual_seed(17)
+        st = {}
+        for proj, (kk, nn) in (("gate", (H, I)), ("up", (H, I)), ("down", (I, H))):
+            st[f"{proj}_trellis"] = torch.randint(-32768, 32768, (E, kk // 16, nn // 16, 16 * K_BITS), dtype=torch.int16,
+                                                  generator=g, device=dev)
+            st[f"{proj}_suh"] = (torch.randint(0, 2, (E, kk), generator=g, device=dev) * 2 - 1).half()
+            st[f"{proj}_svh"] = ((torch.randint(0, 2, (E, nn), generator=g, device=dev) * 2 - 1) * kk ** -0.5).half()
+        x = torch.randn((T, H), generator=g, device=dev).half()
+        logits = torch.randn((T, E), generator=g, device=dev) + 0.5 * torch.randn((1, E), generator=g, device=dev)
+        w, ids = torch.topk(logits, top_k, dim=1)
+        for _ in range(launches):
+            ops.moe_forward(x, ids, torch.softmax(w, dim=1), st, CODEBOOK)
     elif kind == "copy":
         src = torch.empty(128 << 20, dtype=torch.float32, device=dev).uniform_()
         dst = torch.empty_like(src)
@@ -604,9 +619,10 @@ def probe(kind: str, launches: int) -> int:
     else:
         # five copies of the layer (5 x 67 MB > the 256 MB MALL), rotated as the timed step rotates its copies, so the
         # counters see weights coming from HBM rather than from the MALL
-        k, ns = LAYERS[kind]
-        copies = [make_layer_set(torch, 99 + r, dev, names=(kind,))[kind] for r in range(5)]
-        x = torch.randn((1, k), dtype=torch.float16, device=dev)
+        name = kind.rstrip("16")
+        k, ns = LAYERS[name]
+        copies = [make_layer_set(torch, 99 + r, dev, names=(name,))[name] for r in range(5)]
+        x = torch.randn((1 if kind == name else 16, k), dtype=torch.float16, device=dev)
         out = ops.linear(x, *copies[0], CODEBOOK)
         for i in range(launches):
             ops.linear(x, *copies[i % len(copies)], CODEBOOK, out=out)
@@ -668,7 +684,7 @@ def main() -> int:
                     help="also report these M (comma list, '' for none; past 16 rows the GEMV takes 2 or 4 row groups)")
     ap.add_argument("--no-traffic", action="store_true", help="skip the rocprofv3 counter passes")
     ap.add_argument("--no-secondary", action="store_true", help="skip the prefill / MoE / KV-attention lines")
-    ap.add_argument("--probe", choices=["gate_up", "prefill", "kv8", "kv4", "copy"], help=argparse.SUPPRESS)
+    ap.add_argument("--probe", choices=["gate_up", "gate_up16", "prefill", "kv8", "kv4", "moe256", "moe2048", "copy"], help=argparse.SUPPRESS)
     ap.add_argument("--probe-launches", type=int, default=20, help=argparse.SUPPRESS)
     args = ap.parse_args()
     if args.probe:

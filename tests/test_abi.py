@@ -195,7 +195,7 @@ def test_zero_rows_launch_nothing_and_accept_null_data_pointers(lib):
 
 
 def test_one_group_split_plan_fills_its_last_round(lib):
-    """The decode-GEMV split plan at the configs[1] shapes, read back through the reported workspace size (counter
+    """The decode-GEMV split plan at the dense layer set's shapes, read back through the reported workspace size (counter
     region + splits x rows x n x 4 bytes of partials, 256-byte aligned): the longest equal split of 40 / 32 / 24 tile
     rows (5 / 4 / 3 blocks of 128 rows) with >= 448 workgroups, unless that needs more than one round of 1024
     workgroups -- then the split whose last round is fullest.  A plan derived here independently of the library."""

@@ -2,7 +2,7 @@
 
 Decoded weights are compared bit for bit (reconstruct and the one-hot readout through the GEMV kernel, the method of
 cuda/src/sglang_exl3/parity/marlin_parity.py:149-159 and xpu/tests/test_bitexact_xpu.py:46-102); layer outputs
-against the float64 evaluation of had(had(x*suh) @ W) * svh (parity/l1_linear.py:28-36) with the north-star gate:
+against the float64 evaluation of had(had(x*suh) @ W) * svh (parity/l1_linear.py:28-36) with the gate:
 norm-relative and max-relative error <= 2e-3.
 """
 import numpy as np
@@ -283,7 +283,7 @@ def test_linear_matches_float64_oracle(coracle, M, K, cb):
 
 
 def test_linear_c1_shape_4096(coracle):
-    """4096 -> 4096, K = 4, 3INST, M = 1."""
+    """One layer: 4096 -> 4096, K = 4, 3INST, M = 1."""
     rng = np.random.default_rng(4096)
     k = n = 4096
     K, cb = 4, 0

@@ -1,7 +1,7 @@
-"""The fused kernels at the benchmark's own shapes (BASELINE configs[1] and [2]), where the split plans, tail tiles
+"""The fused kernels at the benchmark's own shapes, where the split plans, tail tiles
 and shard maps take the forms the small parity shapes never reach.  The reference output is built on the GPU from
 pieces pinned elsewhere: the bit-exact reconstruct (W_inner), the input rotation (1-ulp fp16 agreement with the
-oracle) and an fp32 matmul, then the output rotation; the fused result must agree within the north-star tolerance
+oracle) and an fp32 matmul, then the output rotation; the fused result must agree within the tolerance
 (norm-relative and max-relative 2e-3)."""
 import pytest
 import torch
@@ -52,7 +52,7 @@ C2_LAYERS = {"qkv": (5120, [6144, 1024, 1024]), "o": (6144, [5120]), "gate_up": 
 @pytest.mark.parametrize("M", [1, 4, 16])
 @pytest.mark.parametrize("name", list(C2_LAYERS))
 def test_gemv_c2_layer_set_shapes(name, M):
-    """the four fused K = 3 MCG linears of the 27B-class layer set at M = 1, 4 and 16."""
+    """The four fused K = 3 MCG linears of the 27B-class layer set at M = 1, 4 and 16."""
     g = torch.Generator(device="cpu").manual_seed(100 + M)
     k, ns = C2_LAYERS[name]
     trs, suhs, svhs = _layer(g, k, ns, 3)
@@ -62,7 +62,7 @@ def test_gemv_c2_layer_set_shapes(name, M):
 
 @pytest.mark.parametrize("name", list(C2_LAYERS))
 def test_c2_layer_set_shapes_read_the_repacked_layout_bit_identically(name):
-    """configs[1] at M = 1 with the trellis repacked to the BLOCKS layout: the decode-GEMV gives the same bits as on
+    """The layer set at M = 1 with the trellis repacked to the BLOCKS layout: the decode-GEMV gives the same bits as on
     the stored layout (the split-K chain runs in one XCD's L2 here: every layer has a multiple of 8 column blocks)."""
     g = torch.Generator(device="cpu").manual_seed(7)
     k, ns = C2_LAYERS[name]
@@ -76,7 +76,7 @@ def test_c2_layer_set_shapes_read_the_repacked_layout_bit_identically(name):
 @pytest.mark.parametrize("K,cb,M", [(3, 1, 2048), (2, 0, 512), (8, 2, 512), (3, 1, 8192), (4, 2, 2048), (5, 1, 2048),
                                     (6, 0, 2048), (2, 0, 2048), (8, 2, 2048)])
 def test_prefill_c3_shape(K, cb, M):
-    """the 5120 -> 17408 prefill decode-GEMM (68 column tiles, split-K tail items) at the benchmark's K,
+    """The 5120 -> 17408 prefill decode-GEMM (68 column tiles, split-K tail items) at the benchmark's K,
     codebook and row counts."""
     g = torch.Generator(device="cpu").manual_seed(200 + K)
     trs, suhs, svhs = _layer(g, 5120, [17408], K)

@@ -192,7 +192,7 @@ def test_moe_many_slots_use_the_routing_launch():
 
 
 def test_moe_full_shape_batched_tokens_match_single_token(coracle):
-    """BASELINE configs[3] shape (128 experts, top-8, hidden 2048, inter 768, K = 3 MCG): every k-split plan covers
+    """The benchmark's layer (128 experts, top-8, hidden 2048, inter 768, K = 3 MCG): every k-split plan covers
     all input rows.  One token against the exact layer (C reconstruct); batches of 16 and 256 tokens (other k-split
     plans, other modes: only fp32 summation order differs) within 1e-3 of per-token calls, and sampled tokens of both
     batches against the exact layer."""
@@ -338,7 +338,7 @@ def test_moe_down_bitrate_differs_from_gate_up(K, K_down, T):
 
 
 def test_moe_full_shape_single_token_mixed_bitrates(coracle):
-    """BASELINE configs[3] shape (128 experts, top-8, hidden 2048, inter 768, MCG) with gate/up at K = 3 and down at
+    """The benchmark's layer (128 experts, top-8, hidden 2048, inter 768, MCG) with gate/up at K = 3 and down at
     K = 4: one token against the exact layer (C reconstruct of every touched expert)."""
     from conftest import c_reconstruct
     from trellis_serve_amd import ops

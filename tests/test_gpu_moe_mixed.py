@@ -15,7 +15,7 @@ from test_gpu_moe_stages import _runs
 
 pytestmark = pytest.mark.gpu
 
-E, H, I, TOP_K, CB = 128, 2048, 768, 8, 1
+E, H, I, TOP_K, CB = 128, 2048, 768, 8, 1   # the benchmark's layer
 
 
 def _ops():

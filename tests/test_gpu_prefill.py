@@ -1,5 +1,5 @@
 """GPU parity of the fused prefill decode-GEMM (exl3_linear_prefill) against the float64 oracle, and against the
-decode-GEMV path on the same inputs.  Gate: norm-relative and max-relative error <= 2e-3 (BASELINE north_star)."""
+decode-GEMV path on the same inputs.  Gate: norm-relative and max-relative error <= 2e-3."""
 import numpy as np
 import pytest
 import torch

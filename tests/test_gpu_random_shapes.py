@@ -2,7 +2,7 @@
 per-shard n of 128..5120 and 1..4 shards, every bit width and codebook, fp16 or bf16 input.  The split plans, shard
 maps, tail tiles and half tiles take forms here that the fixed shapes of the other tests do not.  The reference is
 built on the GPU from pieces pinned elsewhere -- the bit-exact reconstruct (W_inner), the input rotation of every
-shard and an fp32 matmul, then the output rotation -- and the fused result must agree within the north-star
+shard and an fp32 matmul, then the output rotation -- and the fused result must agree within the
 tolerance (norm-relative and max-relative 2e-3).  Outputs are fp16 (a bf16 input still gives an fp16 output)."""
 import numpy as np
 import pytest

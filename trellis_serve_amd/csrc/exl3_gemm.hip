@@ -22,9 +22,10 @@
 // 6 us; 729-745 -> 641-676 us in all (636 with the k-steps in pairs).
 //
 // What bounds it: issue.  Per k-step and wave of a 256-row tile 32 MFMAs (512 cycles) and 71 VALU of decode (284),
-// two waves per SIMD.  With 88 VALU (one k-step at a time) the counters at 4096 rows read: matrix core 54 % busy, VALU
-// 37 %, 18 % both, at 2.0 GHz.  The two waves of a SIMD take decode and multiply in opposite order (2-3 %); forced
-// bursts, a deeper fragment window (8) and an explicit MFMA / VALU interleave were slower.
+// two waves per SIMD.  Counters at 2048 rows of 5120 -> 17408: matrix core 50 % busy, VALU 42 % (MFMA issue included),
+// 31 % of the matrix core's cycles beside a VALU instruction, at 1.9 GHz.  The two waves of a SIMD take decode and
+// multiply in opposite order (2-3 %); forced bursts, a deeper fragment window (8) and an explicit MFMA / VALU interleave
+// were slower.
 //
 // Work decomposition (1-D grid of work items, dispatched in order): tiles are numbered column block fastest, so
 // consecutive workgroups share their A rows in L2.  When the tile count is not a multiple of the machine's
@@ -73,7 +74,7 @@ struct GemmPlan {
   int sk_tiles;    // tiles 0 .. sk_tiles-1 are shared out by runs of k-steps among the stream-K workgroups
   int groups;      // stream-K workgroups: grid items 0 .. groups-1; items groups.. are whole tiles sk_tiles..
   int ksteps;      // k / 32
-  float* partial;  // [groups][2 segments][8 waves][8][4][64 lanes] float4: a workgroup's first / last segment
+  float* partial;  // [groups][2 segments][8 waves][MI][2][64 lanes] float4: a workgroup's first / last segment
   int* counters;   // [sk_tiles], zero between calls
 };
 

@@ -10,7 +10,8 @@
 // expert GEMVs decode the weights once per 64 slots too, but each wave reads every activation fragment from LDS for 16
 // columns, and a workgroup waits for each 256 rows of k of its activations (one workgroup per CU at 64 slots per pass):
 // 128 experts, top-8, 2048 / 768 at 2048 tokens, gate|up and down 875 + 456 us (kernel trace)
-// against 245 + 137 here.
+// against 245 + 137 here.  Counters: at 256 tokens (about 16 slots per expert) gate/up VALU 63 %, matrix core 15 %; at
+// 2048 45 % and 25 % with 6 waves per CU.
 #include <algorithm>
 
 #include "exl3_moe_gemm.hpp"
