@@ -90,7 +90,7 @@ def split(lens, hkv: int, group: int, max_pages: int, ulps: int = 0) -> Split:
         half, most, last = ((share + share // 2, 2 * share, up(max(F(3) * total * inv_slots, F(2) * share)))
                             if crowded else (leaving(0.5), leaving(0.25), leaving(0.0)))
         way, cp = ("half", half) if fits(chunks_of(half)) else ("most", most) if fits(chunks_of(most)) else ("last", last)
-    if slots <= target and not any(x > cp for x in longest) and any(p > f.chunk_pages for p in pages):
+    if w == 8 and slots <= target and not any(x > cp for x in longest) and any(p > f.chunk_pages for p in pages):
         return fixed
     c = chunks_of(cp)
     per = [p if n <= 1 else -(-(-(-p // n)) // w) * w for p, n in zip(pages, c)]

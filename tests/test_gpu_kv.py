@@ -237,6 +237,7 @@ RAGGED = [([5000] + [0, 3, 40, 17] * 3, 10, 2, 512, "share"),
           ([3000, 1, 0, 2047, 2048, 2049], 32, 2, 400, "share"),
           ([1024, 1025, 1040, 128, 129], 5, 1, 66, "fixed"),
           ([0, 0, 0], 8, 8, 100, "fixed"),
+          ([305 * (i + 1) for i in range(20)], 16, 1, 382, "half"),
           ([4224], 40, 8, 264, "fixed"),
           ([2048] * 15 + [1950], 10, 2, 128, "fixed"),
           ([2700 - 17 * i for i in range(15)] + [637 - 17 * i for i in range(27)], 8, 8, 200, "share"),

@@ -297,9 +297,11 @@ __device__ __forceinline__ bool kv_batch(const KvSplit& s, const int* __restrict
     k.chunks = chunks_of(cp);
     k.sums = wave_scan(both(k.chunks));
   }
-  // with a CU for every workgroup of the fixed plan, chunks by lengths may still come out as long (unless every sequence
-  // ends in its first chunk there, whose state would take the merge's detour)
-  return s.slots > s.target || any(longest > (float)cp) || !any(k.pages > s.chunk_pages);
+  // With a CU for every workgroup of the fixed plan, chunks by lengths may still come out as long (unless every sequence
+  // ends in its first chunk there, whose state would take the merge's detour).  Four workgroups of 4 waves share a CU:
+  // there it also counts that chunks by lengths lie side by side in the grid, with no empty workgroups between them (20
+  // sequences of 305-6094 tokens, 1 kv head, 8 bits: 510 chunks of 8 pages in both plans, 19.4 us fixed, 16.5 by lengths).
+  return waves == 4 || s.slots > s.target || any(longest > (float)cp) || !any(k.pages > s.chunk_pages);
 }
 
 // A workgroup's chunk: pages [p0, p1) of sequence b of length len; slot: its partial state, -1 when it is the whole
